@@ -40,6 +40,11 @@ struct mnc_ctx {
     float *d_mpv = nullptr;          // Gaunt map in compile-time pattern order (mixed logic)
     unsigned short *d_mh = nullptr;
     int *d_mgptr = nullptr, *d_mgk = nullptr;
+    // FP64 solve with a row of lanes per cell (moment orders up to 4)
+    mnc::OrbitTables orb;
+    double *d_ot = nullptr, *d_ogv = nullptr;
+    unsigned char *d_opos = nullptr;
+    int *d_ogoff = nullptr, *d_ogk = nullptr;
     // FP64 matrix-core operand tables of the high orders (M8)
     mnc::G64Tables g64;
     bool has_g64 = false;
@@ -48,10 +53,9 @@ struct mnc_ctx {
     int state_nm = 0;
     void *d_noalloc = nullptr;       // the library's fixed scratch array on this device (not owned)
     // tuning
-    int rounds = 6;
+    int rounds = -1;                 // -1 (not set): run_newton's choice, 6 or 0
     int tail_blocks = 0;             // 0: 2 per CU
-    int tail_mode = 0;               // 0: wave per cell, 1: lane per cell, 2: wave sweep + serial logic,
-                                     // 3: wave per cell at two waves per SIMD
+    int tail_mode = 0;               // 0, 3: row of lanes per cell, 1: lane per cell, 2: wave sweep + serial logic
     int mix_cond_log10 = 9;          // mixed steps need cond(H) <= 10^this, else FP64
     int mix_defer = 0;               // 0: redone steps wait for the FP64 tail; 1: FP64 lockstep rounds
     int mix_split = 3;               // bf16 parts of e and of the table in the mixed Hessian products
@@ -363,6 +367,13 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     a.gate = std::pow(10.0, ctx->learned_gate_log10);
     a.fallback_iters = ctx->learned_fallback_iters;
     a.mlp_w = ctx->d_mlp;
+    a.ot = ctx->d_ot;
+    a.opos = ctx->d_opos;
+    a.ogoff = ctx->d_ogoff;
+    a.ogk = ctx->d_ogk;
+    a.ogv = ctx->d_ogv;
+    a.no = ctx->orb.no;
+    a.nop = ctx->orb.nop;
     a.gz = ctx->d_gz;
     a.gg = ctx->d_gg;
     a.gh = ctx->d_gh;
@@ -370,7 +381,18 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     a.gnmm = ctx->g64.nmm;
     mnc::LaunchPlan lp;
     lp.r0 = 0;
-    lp.r1 = ctx->rounds;
+    // FP64 cells go straight to the tail kernel unless rounds are asked for.
+    // Not with the reference's line search below TOL 1e-6: there its Armijo
+    // test compares values of f that differ by f's rounding, so the path
+    // depends on the order of the sums, and the lockstep kernels sum in the
+    // reference's; twelve rounds end all but the slow cells there.
+    const bool by_rounding = o->line_search == MNC_LS_REFERENCE && o->tol_rel < 1e-6;
+    const bool network = learned && ctx->learned_gate_log10 < kGateOff;
+    const int rounds = ctx->rounds >= 0 ? ctx->rounds : (mixed || network ? 6 : (by_rounding ? 12 : 0));
+    lp.r1 = rounds;
+    lp.num_cu = ctx->num_cu;
+    lp.fresh = rounds == 0 && !mixed && !network && (ctx->tail_mode == 0 || ctx->tail_mode == 3 || ctx->ppn);
+    if (lp.fresh) lp.init = false;
     lp.tail_blocks = ctx->tail_blocks > 0 ? ctx->tail_blocks : 2 * ctx->num_cu;
     lp.tail_mode = ctx->tail_mode;
     lp.mix_blocks = ctx->mix_blocks > 0 ? ctx->mix_blocks : ctx->num_cu;
@@ -399,7 +421,7 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
             if (reset) mnc::launch_ctl_reset(ctl, ctx->stream);
             if ((s2 = launch(aa, body))) return s2;
         }
-        if (p.tail && ctx->defer_tail) {   // the step launches it (flux_overlap)
+        if (p.tail && ctx->defer_tail && !p.fresh) {   // the step launches it (flux_overlap)
             ctx->tail_saved = true;
             ctx->tail_mixed = mixed;
             ctx->tail_a = aa;
@@ -427,7 +449,7 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
         first.r1 = 1;
         first.tail = false;
         rest.r0 = 1;
-        rest.r1 = std::max(ctx->rounds, 1);
+        rest.r1 = std::max(rounds, 1);
         rest.init = false;
         mnc::NewtonArgs ad = a;
         ad.divert = 1;
@@ -672,6 +694,14 @@ int mnc_create(const mnc_setup *setup, mnc_ctx **out) {
         mnc_destroy(ctx);
         return MNC_ERR_HIP;
     }
+    if (t.nm <= 15) {
+        if (mnc::build_orbit_tables(t, ctx->ppn, ctx->orb) != MNC_OK || up(&ctx->d_ot, ctx->orb.t) ||
+            up(&ctx->d_opos, ctx->orb.pos) || up(&ctx->d_ogoff, ctx->orb.goff) || up(&ctx->d_ogk, ctx->orb.gk) ||
+            up(&ctx->d_ogv, ctx->orb.gv)) {
+            mnc_destroy(ctx);
+            return MNC_ERR_HIP;
+        }
+    }
     // above n = 15 the fused flux's halo of alpha (20 x 20 cells does not fit,
     // 12 x 12 leaves two waves per CU) is slower than the ansatz through HBM
     // (M8 512^2: 18.3 against 8.3 ms per stage, the same results)
@@ -708,6 +738,7 @@ void mnc_destroy(mnc_ctx *ctx) {
     for (auto &ev : ctx->events) { (void)hipEventDestroy(ev.a); (void)hipEventDestroy(ev.b); }
     void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_pT, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
                     ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gg, ctx->d_gh,
+                    ctx->d_ot, ctx->d_opos, ctx->d_ogoff, ctx->d_ogk, ctx->d_ogv,
                     ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
                     ctx->d_ctl, ctx->d_stats, ctx->d_std, ctx->d_sti, ctx->d_lists, ctx->d_mom, ctx->d_alpha, ctx->d_old,
                     ctx->d_st, ctx->d_ss, ctx->d_flux, ctx->d_ansatz, ctx->d_fpart, ctx->d_bu, ctx->d_ba, ctx->d_bo,
@@ -1332,7 +1363,7 @@ int mnc_tune(mnc_ctx *ctx, const char *key, int value) {
 
 int mnc_get_tune(const mnc_ctx *ctx, const char *key, int *value) {
     if (!ctx || !key || !value) return MNC_ERR_ARG;
-    if (std::strcmp(key, "rounds") == 0) { *value = ctx->rounds; return MNC_OK; }
+    if (std::strcmp(key, "rounds") == 0) { *value = ctx->rounds >= 0 ? ctx->rounds : 6; return MNC_OK; }
     if (std::strcmp(key, "tail_mode") == 0) { *value = ctx->tail_mode; return MNC_OK; }
     if (std::strcmp(key, "mix_cond_log10") == 0) { *value = ctx->mix_cond_log10; return MNC_OK; }
     if (std::strcmp(key, "mix_defer") == 0) { *value = ctx->mix_defer; return MNC_OK; }
@@ -1415,8 +1446,8 @@ int mnc_autotune(mnc_ctx *ctx, double dt, const mnc_options *opt, int steps, cha
     knobs.push_back({"flux_tile", {0, 1, 2, 3}, &ctx->flux_tile});
     knobs.push_back({"flux_groups", {2, 3, 4, 6, 8}, &ctx->flux_groups});
     knobs.push_back({"flux_overlap", {0, 1}, &ctx->flux_overlap});
-    knobs.push_back({"rounds", {2, 4, 6, 8, 12}, &ctx->rounds});
-    knobs.push_back({"tail_mode", {0, 1, 2, 3}, &ctx->tail_mode});
+    knobs.push_back({"rounds", {0, 2, 4, 6, 8, 12}, &ctx->rounds});
+    knobs.push_back({"tail_mode", {0, 1, 2}, &ctx->tail_mode});
     knobs.push_back({"tail_blocks", {cu, 2 * cu, 4 * cu}, &ctx->tail_blocks});
     if (opt->precision == MNC_PREC_MIXED) knobs.push_back({"mix_blocks", {cu / 2, cu, 2 * cu}, &ctx->mix_blocks});
     double best = 0.0;

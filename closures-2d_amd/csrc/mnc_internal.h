@@ -76,6 +76,12 @@ struct NewtonArgs {
     const double *mgv;
     const float *mpv;         // the same map in compile-time pattern order, or nullptr
     double cmix;          // condition bound above which a mixed-precision step is redone in FP64
+    // FP64 solve with a row of lanes per cell (OrbitTables, device copies)
+    const double *ot;
+    const unsigned char *opos;
+    const int *ogoff, *ogk;
+    const double *ogv;
+    int no, nop;
     // FP64 matrix-core sweep of the high orders (G64Tables, device copies)
     const double *gz, *gg, *gh;
     int gnt;              // quadrature tiles of 16 points
@@ -131,21 +137,41 @@ struct G64Tables {
 };
 int build_g64_tables(int moment_order, int quad_order, G64Tables &m);
 
+// Tables of the FP64 solve with a row of lanes per cell (mnc_rows.hip), for
+// moment orders up to 4: the quadrature's orbits of four mirrored nodes
+// (mnc_orbit.h), each with its moments at the node with xi, eta > 0.
+struct OrbitTables {
+    int no = 0, nop = 0;           // orbits, padded to a multiple of 64 (zero weight)
+    std::vector<double> t;         // [nop / 16][np2 + 1][16]: tiles of 16 orbits, the table's columns, then the weights
+    std::vector<unsigned char> pos;   // direct Hessian: [16][16] H_rk's place among the sums
+    // Gaunt form: the terms of H_rk as entries off[k] <= e < off[k + 1], for
+    // all r side by side ([e][16], zero coefficients where row r has fewer)
+    std::vector<int> goff, gk;
+    std::vector<double> gv;
+};
+int build_orbit_tables(const Tables &t, bool ppn, OrbitTables &o);
+
 // Launchers (mnc_newton.hip).  Return false if (nm, np2, gaunt) has no instance.
 // One call enqueues (no host synchronisation) the prologue if `init`, the
 // lockstep sweep/logic rounds r0..r1-1 with compaction (round r reads list
-// r & 1) and, if `tail`, the persistent tail.  tail_mode 0: one wave per
-// remaining cell (cooperative sweeps); 1: one lane per cell; 2: one wave per
-// cell, algebra per lane; 3: mode 0 held to two waves per SIMD (direct Mn
-// Hessian; mode 0 elsewhere).
+// r & 1) and, if `tail`, the persistent tail.  tail_mode 0: a row of lanes per
+// remaining cell (mnc_rows.hip); 1: one lane per cell; 2: one wave per
+// cell, algebra per lane; 3: as 0.  fresh: no prologue and no rounds, the
+// tail (mode 0) takes every cell from its u and alpha.
 struct LaunchPlan {
     int r0 = 0, r1 = 0;
-    bool init = true, tail = true;
+    bool init = true, tail = true, fresh = false;
+    int num_cu = 256;
     int tail_blocks = 0, tail_mode = 0;
     int mix_blocks = 0, defer_rounds = 0;   // mixed precision only
     int mix_split = 3;                       // bf16 parts in the mixed sweep's Hessian products (2 or 3)
 };
 bool launch_newton_fp64(const NewtonArgs &a, int nm, int np2, bool gaunt, const LaunchPlan &lp, hipStream_t s);
+// The FP64 solve with a row of lanes per cell (mnc_rows.hip; moment orders up
+// to 4): every cell from its u and alpha (fresh), or those left on lists lin
+// and lin2.
+bool launch_rows(const NewtonArgs &a, int nm, bool gaunt, int lin, int lin2, bool fresh, int num_cu, int tail_blocks,
+                 hipStream_t s);
 // The control word holding list l's count.
 int newton_list_word(int l);
 // The same with the lockstep rounds in mixed precision (MFMA sweeps); the tail

@@ -8,9 +8,10 @@
 // One sweep yields both a trial's f and the full Hessian at the trial point, so
 // an accepted trial goes straight to its Newton step with no second sweep (the
 // reference re-evaluates at the same alpha, giving the same numbers).  After the
-// rounds, a persistent tail (tail_coop_kernel: one wave per remaining cell)
-// takes the few slow cells near the realizability boundary from a queue and
-// iterates each to completion.
+// rounds, a persistent tail (rows_kernel in mnc_rows.hip) takes the few slow
+// cells near the realizability boundary from a queue and iterates each to
+// completion; in FP64 it takes every cell from the start unless rounds are
+// asked for.
 //
 // The per-cell algorithm restates src/momopt/opt/opt.cpp:82-343 (opt,
 // optScaled), src/momopt/opt/linesearch.cpp:21-99 and fobj.cpp:37-129,255-335,
@@ -25,14 +26,12 @@
 #include "mnc_internal.h"
 #include "mnc_coop_la.h"
 #include "mnc_gaunt_pattern.h"
+#include "mnc_newton_state.h"
 
 namespace mnc {
 namespace {
 
 constexpr int kBlock = 256;
-#define kSqrtPi sqrt(M_PI)
-#define kPi M_PI
-__constant__ double kReg[5] = {0.0, 1e-3, 1e-2, 1e-1, 5e-1};   // opt.h:39-40
 
 template <int N> struct Tri {
     static constexpr int size = N * (N + 1) / 2;
@@ -230,15 +229,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-enum : int { ST_NEWTON = 0, ST_TRIAL = 1 };
-constexpr int kHalvings = 2;   // line-search halvings evaluated per wave sweep in the tail (8 measured
-                               // 2-3% slower: the unused candidates' exponentials and registers)
-constexpr int kTailCap = 4;    // quadrature points per lane whose w e the tail keeps between passes
-constexpr int kTailPts = 2;    // points per lane whose chains interleave (2 of the 4 at a time:
-                               // with 4, the rows and the partial sums outgrow the VGPRs and the
-                               // sums move through AGPRs, 4% slower on the M4 lattice)
-constexpr int kTailWaves = 4;  // waves (cells in flight) per block of the cooperative tail
-constexpr int kFirstHalvings = 2;   // candidates in the first batch of halvings after a failed trial
 enum : int { LOGIC_CONTINUE = 0, LOGIC_DONE = 1, LOGIC_DEFER = 2, LOGIC_MLP = 3 };
 constexpr int kMlpList = kMlpListIndex;   // cells waiting for the learned warm start's network
 static_assert(kMlpListWord == kMlpListIndex + 2, "list word of cw()");
@@ -280,16 +270,6 @@ __device__ __forceinline__ double sweep(const double *Pg, const double *Wg, int 
         }
     }
     return sf;
-}
-
-// The same sweep shared by a whole wave for one cell: lane l takes the
-// quadrature points q = l, l+64, ..., and the partial sums are reduced across
-// the wave (butterfly), so every lane ends with the full sums.
-// The PPn ansatz at t = (alpha.m)/2 (fobj.cpp:166-172): G = t + s with
-// s = sqrt(t^2 + delta), taken as -delta / (t - s) for t < 0.
-__device__ __forceinline__ double ppn_g(double t, double delta, double &s) {
-    s = sqrt(t * t + delta);
-    return t < 0.0 ? -delta / (t - s) : t + s;
 }
 
 // The PPn sweep (fobj.cpp:137-236,355-428): f = sum w (t G - delta/2 + delta log G)
@@ -334,6 +314,9 @@ __device__ __forceinline__ double sweep_ppn(const double *Pg, const double *Wg, 
     return sf;
 }
 
+// The same sweep shared by a whole wave for one cell: lane l takes the
+// quadrature points q = l, l+64, ..., and the partial sums are reduced across
+// the wave (butterfly), so every lane ends with the full sums.
 template <int NM, int NP2, bool GAUNT, int R0, int R1, int NA>
 __device__ __forceinline__ double sweep_wave(const double *P, const double *W, int nq, const double (&al)[NM],
                                              double (&acc)[NA]) {
@@ -369,31 +352,6 @@ __device__ __forceinline__ double sweep_wave(const double *P, const double *W, i
     }
     return sf;
 }
-
-// ---- per-cell solver state in HBM ------------------------------------------
-// Structure of arrays [field][cap]: threads handling neighbouring list entries
-// (mostly ascending cell indices) touch neighbouring words.
-// Moment order N of n = (N+1)(N+2)/2 moments, and the order-2N count padded to
-// the 16 columns of an MFMA tile (the mixed sweep's Hessian moments).
-constexpr int order_of(int nm) { int N = 0; while ((N + 1) * (N + 2) / 2 < nm) ++N; return N; }
-constexpr int mix_cols(int nm) { return ((2 * order_of(nm) + 1) * (2 * order_of(nm) + 2) / 2 + 15) / 16 * 16; }
-constexpr int cmax(int a, int b) { return a > b ? a : b; }
-
-template <int NM, int NP2>
-struct Store {
-    static constexpr int nacc = cmax(cmax(NP2, NM * (NM + 1) / 2), mix_cols(NM));
-    enum : int {
-        F_AL = 0, F_U = NM, F_AOLD = 2 * NM, F_D = 3 * NM, F_T = 4 * NM, F_RTOL, F_U0, F_ASCALE, F_FCUR,
-        F_GD, F_MAXF, F_FSCALE, F_DELTA, F_SF, F_GS, F_ACC = F_GS + NM
-    };
-    static constexpr int dfields = F_ACC + nacc;
-    enum : int { I_ITER = 0, I_TOTAL, I_REG, I_MAXIT, I_MODE, I_WARM, ifields };
-    double *D;
-    int *I;
-    size_t cap;
-    __device__ double &d(int f, int c) const { return D[size_t(f) * cap + c]; }
-    __device__ int &i(int f, int c) const { return I[size_t(f) * cap + c]; }
-};
 
 // Per-lane statistics, reduced per block and flushed with one atomic each.
 // One lane's counts within one launch (32-bit: a lane counts far fewer than
@@ -502,23 +460,6 @@ __device__ double grad_norm2(const NewtonArgs &A, const double (&al)[NM], const 
     return s;
 }
 
-// The supplementary stop test (opt.cpp:52-76,288-293): with tol_gamma > 0 a
-// cell whose gradient passes the tolerance stops only when
-// gamma = exp(2 |d|_1 m_inf) (Mn) or 1 + 2 |d|_1 m_inf (PPn) is <= tol_gamma,
-// d the Newton direction and m_inf = sqrt((2 P + 1) / (2 pi)) with
-// P = floor(sqrt(n)) + 1 (computed on the host).  da1 is |d|_1 summed in
-// index order.
-__device__ __forceinline__ bool gamma_ok(const NewtonArgs &A, double da1, bool ppn) {
-    const double x = 2.0 * da1 * A.gamma_minf;
-    return (ppn ? 1.0 + x : exp(x)) <= A.tol_gamma;
-}
-
-// Control word holding the count of list l: lists 0 and 1 (the lockstep
-// ping-pong pair) use words 0 and 1, lists 2 and 3 (the FP64 pair of a
-// mixed-precision solve) words 4 and 5, list 4 (the learned warm start's
-// network rows) word 6.  Word 2 is the tail's queue head, word 3 the error bits.
-__device__ __forceinline__ int cw(int l) { return l < 2 ? l : l + 2; }
-
 // Appends the calling lanes with `want` set to list `dst`, whose count is
 // control word `cw` (wave-aggregated).
 __device__ __forceinline__ void list_append(const NewtonArgs &A, int dst, int cw, bool want, int c) {
@@ -598,22 +539,6 @@ __device__ int cell_init(const NewtonArgs &A, const Store<NM, NP2> &S, int c, La
     S.i(St::I_WARM, c) = warm;
     if (A.warm == MNC_WARM_LEARNED && !A.divert) count_warm(st, warm);
     return INIT_READY;
-}
-
-// The learned warm start's fallback: a cell started from the network's guess
-// (I_WARM 0) that meets a regularization criterion at level 0 -- the iteration
-// limit, a failed factorisation, an exhausted line search, a condition estimate
-// above cond_h_max -- within A.fallback_iters Newton iterations restarts once
-// from isotropicAlpha at level 0 instead of climbing the ladder: the guess, not
-// the problem, may be what failed, and the start from isotropicAlpha is the
-// reference's own (momopt_update.cpp:236-238 with an isotropic previous alpha).
-// A late failure is the problem's (cells beyond what the quadrature resolves
-// fail at level 0 from any start) and climbs the ladder.  I_WARM becomes
-// kWarmFellBack, so a second failure climbs the ladder as the reference does.
-// Only Mn, where the network exists.
-constexpr int kWarmFellBack = 3;
-__device__ __forceinline__ bool net_fallback(const NewtonArgs &A, int reg, int warm, int iter) {
-    return reg == 0 && warm == 0 && iter <= A.fallback_iters;
 }
 
 // One step of optScaled's loop for cell c after a sweep at its evaluation
@@ -1350,14 +1275,6 @@ __global__ __launch_bounds__(kBlock) void logic_kernel(NewtonArgs A, int lin, in
     flush_stats(A, st);
 }
 
-// Entry s of the tail's work: the cells left on list `lin`, then those left
-// on list `lin2` (the FP64 list of a mixed-precision solve).  -1 past the end.
-__device__ __forceinline__ int tail_cell(const NewtonArgs &A, int lin, int count, int lin2, int count2, int s) {
-    if (s < count) return A.lists[size_t(lin) * A.cap + s];
-    if (s < count + count2) return A.lists[size_t(lin2) * A.cap + (s - count)];
-    return -1;
-}
-
 // Persistent tail: lanes pull the remaining cells of list `lin` from a queue
 // and iterate each to completion, so a few cells needing tens of iterations
 // near the realizability boundary cost one launch, not one per iteration.
@@ -1455,580 +1372,6 @@ __global__ __launch_bounds__(kBlock) void tail_wave_kernel(NewtonArgs A, int lin
     st.titer += st.sum;
     st.ttrials = st.trials;
     flush_stats(A, st);
-}
-
-// ---- cooperative tail: one wave per cell, dense algebra in LDS -------------
-//
-// For the few cells still iterating after the lockstep rounds, a wave owns one
-// cell: lane l sweeps the quadrature points q = l, l+64, ...; the partial sums
-// are reduced through LDS; the Hessian and its factor live in LDS and lane i
-// owns row i of the Cholesky factorisation and of the triangular solves.  The
-// order of every sum is the serial one (the column-oriented back substitution
-// subtracts x_{n-1}, x_{n-2}, ... in the order of the dot-product form), so a
-// cell takes the same path here as in the lockstep kernels up to FMA rounding.
-// Per-wave state of the cooperative tail.  The direct Hessian's TRI sums are
-// accumulated in NPASS passes over the quadrature (a flat split of the packed
-// triangle: KH sums, then the rest), so that a pass's partial sums fit the
-// registers; the first pass also carries the PPn gradient sums.
-template <int NM, int NP2, bool GAUNT, int RS, bool PPN = false>
-struct CoopShared {
-    static constexpr int NPASS = (!GAUNT && RS < NM) ? 2 : 1;
-    static constexpr int TRI = Tri<NM>::size;
-    static constexpr int KH = GAUNT ? NP2 : (NPASS == 2 ? (TRI + 1) / 2 : TRI);
-    static constexpr int NG = PPN ? NM : 0;
-    static constexpr int NV0 = KH + NG, NV1 = NPASS == 2 ? TRI - KH : 0;
-    static constexpr int NV = NV0 > NV1 ? NV0 : NV1;      // partial sums per lane and pass
-    static constexpr int H1 = (NV + 1) / 2, H2 = (H1 + 1) / 2;   // values per lane after the two exchanges
-    static constexpr int NACC = Store<NM, NP2>::nacc;
-    double part[H2][65];      // the lane quads' partials, padded
-    double accs[NACC];        // reduced sweep sums
-    double L[NM][NM];         // H, then its Cholesky factor (lower)
-    double x[NM], gvec[NM];
-    double gsum[NM];          // PPn: sum w G m
-};
-
-// The quadrature table (transposed, pT[k][q]) and weights in LDS, shared by the
-// block's waves, when nq <= 64 kTailCap and the rows are the moments (direct
-// Hessian): LDS reads instead of L2 round trips in every sweep.
-template <int NM, bool ON>
-struct TailTable {
-    double t[ON ? NM : 1][ON ? 64 * kTailCap : 1];
-    double w[ON ? 64 * kTailCap : 1];
-};
-
-// v from lane l ^ 1 and from lane l ^ 2 (DPP quad permutations)
-__device__ __forceinline__ double dpp_xor1(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-__device__ __forceinline__ double dpp_xor2(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x4E, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x4E, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-
-// WPE: waves per SIMD the registers are held to.  At 1 the kernel takes up to
-// 512 registers, for the latency of few cells (the lattice's tail: 2.65
-// against 2.88 ms/step at 2); at 2 it holds 256, with a few spill slots,
-// for throughput when many cells enter the tail (the isolated lobe batch:
-// 10.9 against 9.2 M closures/s).  At 2 the lane index passes through an
-// empty asm each pass and the state's base offsets are formed per cell, so
-// that the compiler does not keep lane masks and field addresses live
-// across the loops.
-template <int NM, int NP2, bool GAUNT, int RS, bool PPN = false, int WPE = 1>
-__global__ __launch_bounds__(64 * kTailWaves) __attribute__((amdgpu_waves_per_eu(WPE)))
-void tail_coop_kernel(NewtonArgs A, int lin, int lin2) {
-    // points per lane interleaved: at two waves per SIMD one at a time (fewer
-    // live registers; 4-5% faster there), otherwise kTailPts
-    constexpr int PTS = WPE > 1 ? 1 : kTailPts;
-    static_assert(NM <= 16, "the max/min reductions over the row lanes take one 16-lane DPP row");
-    using St = Store<NM, NP2>;
-    using CS = CoopShared<NM, NP2, GAUNT, RS, PPN>;
-    constexpr int NG = CS::NG;
-    __shared__ CS shw[kTailWaves];
-    __shared__ TailTable<NM, !GAUNT> tab;
-    CS &sh = shw[threadIdx.x >> 6];
-    int lane = threadIdx.x & 63;
-    const bool tabled = !GAUNT && A.nq <= 64 * kTailCap;
-    if constexpr (!GAUNT) {
-        if (tabled) {
-            for (int i = threadIdx.x; i < NM * A.nq; i += blockDim.x) tab.t[i / A.nq][i % A.nq] = A.pT[i];
-            for (int i = threadIdx.x; i < A.nq; i += blockDim.x) tab.w[i] = A.w[i];
-        }
-    }
-    __syncthreads();      // the only block-wide barrier: from here on the waves are independent
-    const int count = A.ctl[cw(lin)], dcount = A.ctl[cw(lin2)];
-    const double p0 = A.p[0];
-    LaneStats st;
-    for (;;) {
-        int s = 0;
-        if (lane == 0) s = atomicAdd(&A.ctl[2], 1);
-        s = __shfl(s, 0);
-        // wave-uniform: state loads become scalar loads
-        const int c = __builtin_amdgcn_readfirstlane(tail_cell(A, lin, count, lin2, dcount, s));
-        if (c < 0) break;
-        size_t capc = A.cap;
-        if constexpr (WPE > 1) __asm__ volatile("" : "+s"(capc));
-        const Store<NM, NP2> S{A.st_d, A.st_i, capc};
-        // The cell's state comes into registers once: the tail runs it to the
-        // end, so nothing is stored back until the outputs.  Vectors are
-        // lane-distributed (element k on lane k), scalars wave-uniform.
-        double al[NM];
-#pragma unroll
-        for (int k = 0; k < NM; ++k) al[k] = S.d(St::F_AL + k, c);
-        int mode = S.i(St::I_MODE, c), iter = S.i(St::I_ITER, c), total = S.i(St::I_TOTAL, c);
-        int reg = S.i(St::I_REG, c), maxit = S.i(St::I_MAXIT, c), warm = S.i(St::I_WARM, c);
-        double t = S.d(St::F_T, c), rtol = S.d(St::F_RTOL, c);
-        if (lane == 0) {
-            ++st.tcells;
-            st.titer -= total;
-        }
-        const double u0 = S.d(St::F_U0, c), ascale = S.d(St::F_ASCALE, c);
-        double fcur_s = S.d(St::F_FCUR, c), gd_s = S.d(St::F_GD, c), fscale_s = S.d(St::F_FSCALE, c);
-        double maxf_s = S.d(St::F_MAXF, c);
-        double ul = lane < NM ? S.d(St::F_U + lane, c) : 0.0;
-        const double delta = PPN ? S.d(St::F_DELTA, c) : 0.0;
-        double aold_l = lane < NM ? S.d(St::F_AOLD + lane, c) : 0.0;
-        double d_l = lane < NM ? S.d(St::F_D + lane, c) : 0.0;
-        for (;;) {
-            if constexpr (WPE > 1) __asm__ volatile("" : "+v"(lane));
-            // ---- sweep(s): partial sums per lane, reduced through DPP and LDS ----
-            double sf = 0.0;
-            double wes[kTailCap];
-#pragma unroll
-            for (int pass = 0; pass < CS::NPASS; ++pass) {
-                // flat range [K0, K1) of the sums of this pass (GAUNT: the
-                // order-2N moments), then the PPn gradient sums
-                const int K0 = pass == 0 ? 0 : CS::KH, K1 = pass == 0 ? CS::KH : CS::TRI;
-                const int nv = pass == 0 ? CS::NV0 : CS::NV1;
-                double acc[CS::NV];
-#pragma unroll
-                for (int k = 0; k < CS::NV; ++k) acc[k] = 0.0;
-                // Lane l takes the points q = l, l + 64, ...; the moment values
-                // come from the LDS table or from the transposed table in global
-                // memory (for each k the wave reads 64 consecutive doubles).
-                // With at most kTailCap points per lane, w e of the first pass
-                // is kept for the second.  The points run PTS at a time,
-                // a scheduling barrier between the groups so that the next
-                // group's rows are not loaded while this group's are live
-                // (each lane's sums still take its points in ascending order).
-                const bool cached = A.nq <= 64 * kTailCap;
-                for (int q0 = 0; q0 < A.nq; q0 += 64 * kTailCap) {
-#pragma unroll
-                    for (int qi = 0; qi < kTailCap; ++qi) {
-                        if (qi > 0 && qi % PTS == 0) {
-                            if (q0 + 64 * qi >= A.nq) break;
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                        // points past nq read point 0 and add exact zeros, so
-                        // the PTS points' chains can interleave (the
-                        // order-2N rows of the Gaunt form are too many registers
-                        // for that: there the points stay sequential)
-                        const int q = q0 + 64 * qi + lane;
-                        if (GAUNT && q >= A.nq) break;
-                        const bool valid = q < A.nq;
-                        const int qq = valid ? q : 0;
-                        double row[GAUNT ? NP2 : NM];
-                        double wq;
-                        if constexpr (!GAUNT) {
-                            if (tabled) {
-#pragma unroll
-                                for (int k = 0; k < NM; ++k) row[k] = tab.t[k][qq];
-                                wq = tab.w[qq];
-                            } else {
-#pragma unroll
-                                for (int k = 0; k < NM; ++k) row[k] = A.pT[size_t(k) * A.nq + qq];
-                                wq = A.w[qq];
-                            }
-                        } else {
-#pragma unroll
-                            for (int k = 0; k < NP2; ++k) row[k] = A.pT[size_t(k) * A.nq + qq];
-                            wq = A.w[qq];
-                        }
-                        double we;                    // the Hessian's weight
-                        if (pass > 0 && cached) {
-                            we = wes[qi];
-                        } else {
-                            double am = 0.0;
-#pragma unroll
-                            for (int k = 0; k < NM; ++k) am = fma(al[k], row[k], am);
-                            if constexpr (PPN) {
-                                const double tq = 0.5 * am;
-                                double sq;
-                                const double G = ppn_g(tq, delta, sq);
-                                we = valid ? 0.5 * wq * (G / sq) : 0.0;
-                                if (pass == 0) {
-                                    sf = sf + (valid ? wq * (tq * G - 0.5 * delta + delta * log(G)) : 0.0);
-                                    const double wg = valid ? wq * G : 0.0;
-#pragma unroll
-                                    for (int k = 0; k < NG; ++k) acc[CS::KH + k] = fma(row[k], wg, acc[CS::KH + k]);
-                                }
-                            } else {
-                                we = valid ? wq * exp(am) : 0.0;
-                            }
-                            wes[qi] = we;
-                        }
-                        if (!PPN && pass == 0) sf += we;
-                        if constexpr (GAUNT) {
-#pragma unroll
-                            for (int k = 0; k < NP2; ++k) acc[k] = fma(we, row[k], acc[k]);
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < NM; ++i) {
-                                if (Tri<NM>::at(i, i) < K0 || Tri<NM>::at(i, 0) >= K1) continue;
-                                const double v = we * row[i];
-#pragma unroll
-                                for (int jj = 0; jj <= i; ++jj) {
-                                    const int k = Tri<NM>::at(i, jj) - K0;
-                                    if (k >= 0 && k < K1 - K0) acc[k] = fma(v, row[jj], acc[k]);
-                                }
-                            }
-                        }
-                    }
-                }
-                // Two exchanges between lanes (l ^ 1, then l ^ 2): each halves
-                // the values a lane holds and sums them over the pair, so that
-                // lane l ends with H2 values summed over its quad -- value
-                // (l & 1 ? H1 : 0) + (l & 2 ? H2 : 0) + r in slot r -- and the
-                // sixteen quads' partials of each value are then added through
-                // LDS by one lane, four chains in quad order.
-                double a1[CS::H1];
-#pragma unroll
-                for (int r = 0; r < CS::H1; ++r) {
-                    const double lo = acc[r], hi = (CS::H1 + r < CS::NV) ? acc[CS::H1 + r] : 0.0;
-                    const bool b = lane & 1;
-                    a1[r] = (b ? hi : lo) + dpp_xor1(b ? lo : hi);
-                }
-#pragma unroll
-                for (int r = 0; r < CS::H2; ++r) {
-                    const double lo = a1[r], hi = (CS::H2 + r < CS::H1) ? a1[CS::H2 + r] : 0.0;
-                    const bool b = lane & 2;
-                    sh.part[r][lane] = (b ? hi : lo) + dpp_xor2(b ? lo : hi);
-                }
-                __builtin_amdgcn_wave_barrier();
-                for (int k = lane; k < nv; k += 64) {
-                    const int hb = k >= CS::H1 ? 1 : 0, rel = k - hb * CS::H1;
-                    const int qb = rel >= CS::H2 ? 1 : 0, r = rel - qb * CS::H2;
-                    const int cls = hb | (qb << 1);
-                    double t4[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                    for (int m = 0; m < 16; m += 4) {
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) t4[u] += sh.part[r][4 * (m + u) + cls];
-                    }
-                    const double tot = (t4[0] + t4[1]) + (t4[2] + t4[3]);
-                    if (PPN && pass == 0 && k >= CS::KH) sh.gsum[k - CS::KH] = tot;
-                    else sh.accs[K0 + k] = tot;
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) sf += __shfl_xor(sf, o);
-            __builtin_amdgcn_wave_barrier();
-            // ---- per-cell logic (cell_logic's steps, cooperative) ----
-            bool newton = (mode == ST_NEWTON), do_reg = false, converged = false;
-            double err = 0.0;
-            if (mode == ST_TRIAL) {
-                if (lane == 0) ++st.trials;
-                double fnew = sf;
-#pragma unroll
-                for (int k = 0; k < NM; ++k) fnew = fnew - al[k] * readlane_d(ul, k);
-                const double fcur = fcur_s, gd = gd_s;
-                bool accept = fnew <= fcur + 1e-3 * t * gd;
-                if (!accept && A.ls_mode == MNC_LS_ROBUST && t == 1.0 && -gd <= 1e3 * DBL_EPSILON * fscale_s)
-                    accept = true;
-                if (accept) {
-                    newton = true;
-                } else {
-                    // The reference halves t and evaluates f again until
-                    // Armijo holds or t * maxf <= eps/2 (linesearch.cpp:45-98).
-                    // The next candidates (kFirstHalvings in the first batch,
-                    // where most searches end, then kHalvings per batch) are
-                    // evaluated in one wave sweep (f only, the same sums in the
-                    // same order as a trial sweep) and the first accepted one is
-                    // taken: the reference's decisions without one pass per
-                    // halving.
-                    const double maxf = maxf_s;
-                    if (lane < NM) {
-                        sh.x[lane] = aold_l;
-                        sh.gvec[lane] = d_l;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    int state = 0;                 // 0 searching, 1 accepted, 2 exhausted
-                    int cap = kFirstHalvings;      // candidates in this batch
-                    while (state == 0) {
-                        int nval = 0;
-#pragma unroll
-                        for (int jj = 0; jj < kHalvings; ++jj)
-                            if (jj < cap && nval == jj && ldexp(t, -(jj + 1)) * maxf > DBL_EPSILON / 2) nval = jj + 1;
-                        if (nval == 0) { state = 2; break; }
-                        double fj[kHalvings];
-#pragma unroll
-                        for (int jj = 0; jj < kHalvings; ++jj) fj[jj] = 0.0;
-                        // candidates outside, the lane's points inside (their
-                        // chains interleave); each fj sums the lane's points in
-                        // order, as the trial sweep's f does
-                        for (int q0 = 0; q0 < A.nq; q0 += 64 * PTS) {
-#pragma unroll
-                            for (int jj = 0; jj < kHalvings; ++jj) {
-                                if (jj >= nval) break;                  // wave-uniform
-                                const double tj = ldexp(t, -(jj + 1));
-                                double aj[NM];
-#pragma unroll
-                                for (int k = 0; k < NM; ++k) aj[k] = fma(tj, sh.gvec[k], sh.x[k]);
-#pragma unroll
-                                for (int qi = 0; qi < PTS; ++qi) {
-                                    const int q = q0 + 64 * qi + lane;
-                                    if (GAUNT && q >= A.nq) break;      // Gaunt form: sequential points
-                                    const bool valid = q < A.nq;
-                                    const int qq = valid ? q : 0;
-                                    double row[NM], wq;
-                                    if constexpr (!GAUNT) {
-                                        if (tabled) {
-#pragma unroll
-                                            for (int k = 0; k < NM; ++k) row[k] = tab.t[k][qq];
-                                            wq = tab.w[qq];
-                                        } else {
-#pragma unroll
-                                            for (int k = 0; k < NM; ++k) row[k] = A.pT[size_t(k) * A.nq + qq];
-                                            wq = A.w[qq];
-                                        }
-                                    } else {
-#pragma unroll
-                                        for (int k = 0; k < NM; ++k) row[k] = A.pT[size_t(k) * A.nq + qq];
-                                        wq = A.w[qq];
-                                    }
-                                    double am = 0.0;
-#pragma unroll
-                                    for (int k = 0; k < NM; ++k) am = fma(aj[k], row[k], am);
-                                    if constexpr (PPN) {
-                                        const double tq = 0.5 * am;
-                                        double sq;
-                                        const double G = ppn_g(tq, delta, sq);
-                                        fj[jj] += valid ? wq * (tq * G - 0.5 * delta + delta * log(G)) : 0.0;
-                                    } else {
-                                        fj[jj] += valid ? wq * exp(am) : 0.0;
-                                    }
-                                }
-                            }
-                        }
-                        int acc = -1;
-                        for (int jj = 0; jj < kHalvings; ++jj) {
-                            if (jj >= nval) break;
-                            double fv = fj[jj];
-#pragma unroll
-                            for (int o = 32; o > 0; o >>= 1) fv += __shfl_xor(fv, o);
-                            const double tj = ldexp(t, -(jj + 1));
-                            for (int k = 0; k < NM; ++k)
-                                fv = fv - fma(tj, sh.gvec[k], sh.x[k]) * readlane_d(ul, k);
-                            if (acc < 0 && fv <= fcur + 1e-3 * tj * gd) acc = jj;
-                        }
-                        if (lane == 0) st.trials += (acc >= 0) ? acc + 1 : nval;
-                        if (acc >= 0) {
-                            t = ldexp(t, -(acc + 1));
-                            state = 1;
-                        } else {
-                            t = ldexp(t, -nval);
-                            if (nval < cap) state = 2;           // the next halving fails the bound
-                        }
-                        cap = kHalvings;
-                    }
-                    if (state == 1) {                  // a full sweep at the accepted point next
-#pragma unroll
-                        for (int k = 0; k < NM; ++k) al[k] = fma(t, readlane_d(d_l, k), readlane_d(aold_l, k));
-                        mode = ST_NEWTON;
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < NM; ++k) al[k] = readlane_d(aold_l, k);
-                        t = 0.0;
-                        ++iter; ++total;
-                        do_reg = true;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                }
-            }
-            if (newton) {
-                ++iter; ++total;
-                // H: row i in the registers of lane i (full symmetric row)
-                double row[NM];
-#pragma unroll
-                for (int jj = 0; jj < NM; ++jj) {
-                    const int i0 = lane > jj ? lane : jj, j0 = lane > jj ? jj : lane;
-                    double hij = 0.0;
-                    if (lane < NM) {
-                        if constexpr (GAUNT) {
-                            const int pr = j0 * NM + i0;
-                            for (int cc = A.gptr[pr]; cc < A.gptr[pr + 1]; ++cc)
-                                hij = fma(A.gv[cc], sh.accs[A.gk[cc]], hij);
-                        } else {
-                            hij = sh.accs[Tri<NM>::at(i0, j0)];
-                        }
-                    }
-                    row[jj] = hij;
-                }
-                // g_i = H_i0 / m0 - u_i on lane i; f, its scale and ||g|| in the serial order
-                const double gv = lane < NM ? (PPN ? sh.gsum[lane] : row[0] / p0) - ul : 0.0;
-                if (lane < NM) sh.gvec[lane] = gv;
-                double fcur = PPN ? sf : readlane_d(row[0], 0) / (p0 * p0), fscale = fabs(fcur), gg = 0.0;
-#pragma unroll
-                for (int i = 0; i < NM; ++i) {
-                    const double ui = readlane_d(ul, i);
-                    const double gi = readlane_d(gv, i);
-                    gg = fma(gi, gi, gg);
-                    fcur = fcur - al[i] * ui;
-                    fscale += fabs(al[i] * ui);
-                }
-                double rs = 0.0, dg = 0.0;             // row sums (utils.cpp:36-52), diagonal
-#pragma unroll
-                for (int jj = 0; jj < NM; ++jj) {
-                    rs += fabs(row[jj]);
-                    dg = (jj == lane) ? row[jj] : dg;
-                }
-                const double anorm = row16_max(lane < NM ? rs : 0.0);
-                const double gersh = row16_min(lane < NM ? 2.0 * dg - rs : DBL_MAX);
-                err = sqrt(gg);
-                const bool chol_ok = reg_cholesky<NM>(row, lane);
-                // the columns of the factor (lane i: L[k][i], k > i) for the back substitution
-                double col[NM];
-                if (lane < NM) {
-#pragma unroll
-                    for (int k = 0; k < NM; ++k) sh.L[lane][k] = row[k];
-                }
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int k = 0; k < NM; ++k) col[k] = (lane < NM && k > lane) ? sh.L[k][lane] : 0.0;
-                __builtin_amdgcn_wave_barrier();
-                // reciprocals of the factor's diagonal, independent of each
-                // other: the solves below multiply by them (as blocked trsm
-                // kernels do) instead of dividing on their dependent chains
-                double rd[NM];
-#pragma unroll
-                for (int k = 0; k < NM; ++k) rd[k] = 1.0 / readlane_d(row[k], k);
-                double condest = 0.0;
-                // where the bounds cannot decide the test, the exact ||A^-1||_1
-                // bound and the direction come from one pass over the factor
-                double xv = gv;
-                bool solved = false;
-                if (chol_ok && !cond_proven_below(anorm, gersh, NM, A.cond_h_max)) {
-                    const double inv1 = reg_inv_norm1_solve<NM>(row, col, rd, xv, lane);
-                    solved = true;
-                    if (!(2.0 * anorm * inv1 <= A.cond_h_max))
-                        condest = 1.0 / reg_rcond<NM>(row, col, anorm, lane);
-                }
-                if (iter >= maxit || !chol_ok || t == 0.0 || condest > A.cond_h_max) {
-                    do_reg = true;
-                } else {
-                    if (!solved) reg_apply_inv_rcp<NM>(row, col, rd, xv, lane);
-                    bool stop = err <= rtol;
-                    if (stop && A.tol_gamma > 0.0) {
-                        double da1 = 0.0;
-#pragma unroll
-                        for (int i = 0; i < NM; ++i) da1 = da1 + fabs(readlane_d(xv, i));
-                        stop = gamma_ok(A, da1, PPN);
-                    }
-                    if (stop) {
-                        converged = true;
-                    } else {
-                        const double di = -xv;
-                        double al_l = 0.0;
-#pragma unroll
-                        for (int k = 0; k < NM; ++k) al_l = (k == lane) ? al[k] : al_l;
-                        const double maxf = row16_max(lane < NM ? fabs(di) / (fabs(al_l) + 1e-100) : 0.0);
-                        double gd = 0.0;
-#pragma unroll
-                        for (int i = 0; i < NM; ++i) gd = fma(readlane_d(gv, i), readlane_d(di, i), gd);
-                        aold_l = lane < NM ? al_l : 0.0;
-                        d_l = lane < NM ? di : 0.0;
-                        maxf_s = maxf;
-                        gd_s = gd;
-                        fcur_s = fcur;
-                        fscale_s = fscale;
-                        t = 1.0;
-                        if (t * maxf > DBL_EPSILON / 2) {
-#pragma unroll
-                            for (int i = 0; i < NM; ++i) al[i] = al[i] + t * readlane_d(di, i);
-                            mode = ST_TRIAL;
-                        } else {
-                            t = 0.0;
-                            ++iter; ++total;
-                            do_reg = true;
-                        }
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            bool done = false;
-            if (do_reg && !PPN && net_fallback(A, reg, warm, iter)) {   // the network's guess failed
-                warm = kWarmFellBack;
-                if (lane == 0) {
-                    S.i(St::I_WARM, c) = kWarmFellBack;
-                    ++st.fallback;
-                }
-                al[0] = 2.0 * kSqrtPi * log(0.5 / kSqrtPi);
-#pragma unroll
-                for (int k = 1; k < NM; ++k) al[k] = 0.0;
-                iter = 0;
-                t = 1.0;
-                mode = ST_NEWTON;
-            } else if (do_reg) {
-                if (reg < 4) {
-                    ++reg;
-                    const double r = kReg[reg];
-                    const double *uin = A.u + size_t(c) * NM;
-                    ul = lane == 0 ? 1.0 : (lane < NM ? (uin[lane] / u0) * (1.0 - r) : 0.0);
-                    double ss = 1.0;
-                    for (int k = 1; k < NM; ++k) {
-                        const double uk = readlane_d(ul, k);
-                        ss = fma(uk, uk, ss);
-                    }
-                    rtol = sqrt(ss) * A.tol;
-                    al[0] = PPN ? 1.0 - 4.0 * delta * kPi : 2.0 * kSqrtPi * log(0.5 / kSqrtPi);
-#pragma unroll
-                    for (int k = 1; k < NM; ++k) al[k] = 0.0;
-                    iter = 0;
-                    t = 1.0;
-                    if (reg == 4) maxit = 10 * maxit;
-                    mode = ST_NEWTON;
-                } else {
-                    if (lane == 0) {
-                        st.err_bits |= 1 << MNC_ERR_MAXREG;
-                        if (A.outs) { A.outs[c].iter = total; A.outs[c].r = -1.0; A.outs[c].norm_g = err; }
-                    }
-                    done = true;
-                }
-            } else if (converged) {
-                if (PPN) {                                    // no reconstruction; opt.cpp:131-136
-                    if (lane < NM) {
-                        double ak = 0.0;
-#pragma unroll
-                        for (int kk = 0; kk < NM; ++kk) ak = (kk == lane) ? al[kk] : ak;
-                        A.u[size_t(c) * NM + lane] = ul * u0;
-                        A.alpha[size_t(c) * NM + lane] = ak * u0;
-                    }
-                } else {
-                    const double u0p = readlane_d(ul, 0) + sh.gvec[0];
-                    double a0 = al[0];
-                    a0 -= log(u0p) * 2.0 * kSqrtPi;
-                    a0 = a0 + ascale;
-                    if (lane < NM) {
-                        A.u[size_t(c) * NM + lane] = ((ul + sh.gvec[lane]) / u0p) * u0;
-                        double ak = 0.0;
-#pragma unroll
-                        for (int kk = 0; kk < NM; ++kk) ak = (kk == lane) ? al[kk] : ak;
-                        A.alpha[size_t(c) * NM + lane] = lane == 0 ? a0 : ak;
-                    }
-                }
-                if (lane == 0) {
-                    if (A.outs) { A.outs[c].iter = total; A.outs[c].r = kReg[reg]; A.outs[c].norm_g = err; }
-                    st.max_iter = total > st.max_iter ? total : st.max_iter;
-                    st.sum += total;
-                    ++st.n;
-                    count_reg(st, reg);
-                }
-                done = true;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (done) break;
-        }
-    }
-    // statistics: only lane 0 of each wave counted
-    if (lane == 0 && (st.n || st.trials || st.err_bits || st.tcells)) {
-        atomicAdd((unsigned long long *)&A.stats[13], (unsigned long long)st.tcells);
-        atomicAdd((unsigned long long *)&A.stats[14], (unsigned long long)(st.titer + st.sum));
-        atomicAdd((unsigned long long *)&A.stats[15], (unsigned long long)st.trials);
-        atomicMax((unsigned long long *)&A.stats[0], (unsigned long long)st.max_iter);
-        atomicAdd((unsigned long long *)&A.stats[1], (unsigned long long)st.sum);
-        atomicAdd((unsigned long long *)&A.stats[2], (unsigned long long)st.n);
-        for (int r = 0; r < 5; ++r) atomicAdd((unsigned long long *)&A.stats[3 + r], (unsigned long long)st.hist[r]);
-        atomicAdd((unsigned long long *)&A.stats[8], (unsigned long long)st.trials);
-        if (st.fallback) atomicAdd((unsigned long long *)&A.stats[16], (unsigned long long)st.fallback);
-        if (st.err_bits) atomicOr(&A.ctl[3], st.err_bits);
-    }
 }
 
 // ---- mixed-precision sweep on the matrix cores ------------------------------
@@ -2483,22 +1826,15 @@ __global__ __launch_bounds__(64) void logic_g64_kernel(NewtonArgs A, int lin) {
     }
 }
 
+// Modes 0 and 3, and PPn always: a row of lanes per cell (mnc_rows.hip).
 template <int NM, int NP2, bool G, int RS, bool PPN = false>
-void launch_tail(const NewtonArgs &a, int lin, int lin2, int tail_blocks, int tail_mode, hipStream_t s) {
-    if constexpr (!G && !PPN) {   // the cooperative tail at two waves per SIMD (direct Mn Hessian)
-        if (tail_mode == 3) {
-            hipLaunchKernelGGL((tail_coop_kernel<NM, NP2, G, RS, PPN, 2>), dim3(tail_blocks * 4 / kTailWaves),
-                               dim3(64 * kTailWaves), 0, s, a, lin, lin2);
-            return;
-        }
-    }
-    if (tail_mode == 0 || tail_mode == 3 || PPN)   // PPn: the cooperative tail only
-        hipLaunchKernelGGL((tail_coop_kernel<NM, NP2, G, RS, PPN>), dim3(tail_blocks * 4 / kTailWaves),
-                           dim3(64 * kTailWaves), 0, s, a, lin, lin2);
-    else if (tail_mode == 2)
-        hipLaunchKernelGGL((tail_wave_kernel<NM, NP2, G, RS>), dim3(tail_blocks), dim3(kBlock), 0, s, a, lin, lin2);
+void launch_tail(const NewtonArgs &a, int lin, int lin2, const LaunchPlan &lp, hipStream_t s) {
+    if (lp.tail_mode == 0 || lp.tail_mode == 3 || PPN)
+        launch_rows(a, NM, G, lin, lin2, lp.fresh, lp.num_cu, lp.tail_blocks, s);
+    else if (lp.tail_mode == 2)
+        hipLaunchKernelGGL((tail_wave_kernel<NM, NP2, G, RS>), dim3(lp.tail_blocks), dim3(kBlock), 0, s, a, lin, lin2);
     else
-        hipLaunchKernelGGL((tail_kernel<NM, NP2, G, RS>), dim3(tail_blocks), dim3(kBlock), 0, s, a, lin, lin2);
+        hipLaunchKernelGGL((tail_kernel<NM, NP2, G, RS>), dim3(lp.tail_blocks), dim3(kBlock), 0, s, a, lin, lin2);
 }
 
 // Rounds r0..r1-1 of the lockstep solve (round r reads list r & 1), with the
@@ -2513,7 +1849,7 @@ void launch_all(const NewtonArgs &a, const LaunchPlan &lp, hipStream_t s) {
         hipLaunchKernelGGL((logic_kernel<NM, NP2, G, false, PPN>), dim3(nb), dim3(kBlock), 0, s, a, lin, 2);
         lin ^= 1;
     }
-    if (lp.tail) launch_tail<NM, NP2, G, RS, PPN>(a, lin, 2, lp.tail_blocks, lp.tail_mode, s);   // list 2 empty
+    if (lp.tail) launch_tail<NM, NP2, G, RS, PPN>(a, lin, 2, lp, s);   // list 2 empty
 }
 
 template <int NM, int NP2, bool G, int RS>
@@ -2542,7 +1878,7 @@ void launch_mixed_all(const NewtonArgs &a, const LaunchPlan &lp, hipStream_t s) 
         }
         lin ^= 1;
     }
-    if (lp.tail) launch_tail<NM, NP2, G, RS>(a, lin, flin, lp.tail_blocks, lp.tail_mode, s);
+    if (lp.tail) launch_tail<NM, NP2, G, RS>(a, lin, flin, lp, s);
 }
 
 }  // namespace

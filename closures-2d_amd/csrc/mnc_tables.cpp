@@ -2,11 +2,13 @@
 // for the Mn closure (the host setup of MomOptSolver::init,
 // src/momopt/momopt_init.cpp:88-259, and utils_getGaussianWeightsAndNodes,
 // src/utils.cpp:55-60).  Host code; the tables are uploaded once per context.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
 #include "mnc_internal.h"
 #include "mnc_gaunt_pattern.h"
+#include "mnc_orbit.h"
 
 namespace mnc {
 namespace {
@@ -332,6 +334,72 @@ int build_g64_tables(int moment_order, int quad_order, G64Tables &m) {
     m.gptr = t.gptr;
     m.gk = t.gk;
     m.gv = t.gv;
+    return MNC_OK;
+}
+
+namespace {
+
+// Places of the sums (OrbitSums) in the kernel's buffer, for one order and form.
+template <int N, bool GAUNT>
+void orbit_places(const Tables &t, bool ppn, OrbitTables &o) {
+    using S = OrbitSums<N, GAUNT>;
+    constexpr typename S::Lists L = S::lists();
+    if (!GAUNT) {
+        o.pos.assign(256, 0);
+        for (int c = 0; c < 4; ++c)
+            for (int e = L.first[c]; e < L.first[c + 1]; ++e)
+                o.pos[L.a[e] * 16 + L.b[e]] = o.pos[L.b[e] * 16 + L.a[e]] = (unsigned char)orbit_slot(e, c, ppn);
+        return;
+    }
+    std::vector<int> place(S::n2, 0);
+    for (int c = 0; c < 4; ++c)
+        for (int e = L.first[c]; e < L.first[c + 1]; ++e) place[L.a[e]] = orbit_slot(e, c, ppn);
+    const int n = S::n;
+    o.goff.assign(n + 1, 0);
+    o.gk.clear();
+    o.gv.clear();
+    for (int k = 0; k < n; ++k) {
+        int most = 0;
+        for (int r = 0; r < n; ++r) most = std::max(most, t.gptr[r * n + k + 1] - t.gptr[r * n + k]);
+        for (int e = 0; e < most; ++e)
+            for (int r = 0; r < 16; ++r) {
+                const int at = r < n ? t.gptr[r * n + k] + e : 0;
+                const bool has = r < n && at < t.gptr[r * n + k + 1];
+                o.gk.push_back(has ? place[t.gk[at]] : 0);
+                o.gv.push_back(has ? t.gv[at] : 0.0);
+            }
+        o.goff[k + 1] = o.goff[k] + most;
+    }
+}
+
+template <int N>
+void orbit_places_n(const Tables &t, bool ppn, OrbitTables &o) {
+    if (t.use_gaunt) orbit_places<N, true>(t, ppn, o);
+    else orbit_places<N, false>(t, ppn, o);
+}
+
+}  // namespace
+
+int build_orbit_tables(const Tables &t, bool ppn, OrbitTables &o) {
+    if (t.N > 4) return MNC_ERR_ARG;
+    const int half = t.Q / 2;              // polar nodes, and azimuths below pi / 2
+    o.no = half * half;
+    o.nop = (o.no + 63) / 64 * 64;
+    o.t.assign(size_t(t.np2 + 1) * o.nop, 0.0);
+    for (int i = 0; i < half; ++i)
+        for (int j = 0; j < half; ++j) {
+            const int q = 2 * i * t.Q + j, at = i * half + j;
+            double *tile = &o.t[size_t(at / 16) * (t.np2 + 1) * 16 + at % 16];
+            for (int k = 0; k < t.np2; ++k) tile[k * 16] = t.p[size_t(q) * t.np2 + k];
+            tile[t.np2 * 16] = t.w[q];
+        }
+    switch (t.N) {
+    case 0: orbit_places_n<0>(t, ppn, o); break;
+    case 1: orbit_places_n<1>(t, ppn, o); break;
+    case 2: orbit_places_n<2>(t, ppn, o); break;
+    case 3: orbit_places_n<3>(t, ppn, o); break;
+    default: orbit_places_n<4>(t, ppn, o); break;
+    }
     return MNC_OK;
 }
 

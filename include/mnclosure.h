@@ -277,13 +277,16 @@ int mnc_get_stats(mnc_ctx *ctx, mnc_stats *st);
 int mnc_reset_stats(mnc_ctx *ctx);
 
 /* Tuning knobs of the batched solve (set by the autotuner or by hand):
- *   "rounds"       lockstep sweep/logic rounds before the persistent tail (0-512)
+ *   "rounds"       lockstep sweep/logic rounds before the persistent tail (0-512);
+ *                  until it is set: 6 in mixed precision or where the network
+ *                  is consulted, 0 in FP64 (the tail's kernel takes every cell;
+ *                  12 with the reference's line search below TOL 1e-6, whose
+ *                  decisions depend on the order of the sums); reads 6 then
  *   "tail_blocks"  workgroups of the persistent tail kernel (1-65536)
- *   "tail_mode"    0: one wave per remaining cell, dense algebra shared in LDS;
+ *   "tail_mode"    0: a 16-lane row per remaining cell, four cells per wave (one
+ *                  wave per cell when there are few);
  *                  1: one lane per cell; 2: one wave per cell, algebra per lane;
- *                  3: as 0 at two waves per SIMD (more cells in flight, each
- *                  a little slower: for tails of many cells; direct Mn
- *                  Hessian, elsewhere 0)
+ *                  3: as 0
  *   "mix_cond_log10"  MNC_PREC_MIXED: a Newton step uses the mixed-precision
  *                  Hessian only while its condition estimate is <= 10^value
  *                  (0-10, default 9); otherwise the step is redone in FP64
