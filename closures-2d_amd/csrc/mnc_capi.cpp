@@ -232,19 +232,20 @@ int check_opts(mnc_ctx *ctx, const mnc_options *o) {
 }
 
 // ---- learned warm start -------------------------------------------------------
-constexpr int kMlpChunk = 65536;   // rows per forward pass of the Newton prologue / predict
-
 mnc::MlpBuffers mlp_buffers(mnc_ctx *ctx) {
     const size_t np = size_t(mnc::mlp_param_count()) + mnc::kMlpStats;
-    return {ctx->d_mlp, ctx->d_mlp + np, ctx->d_mlp + 2 * np, ctx->d_mlp + 3 * np, ctx->d_mlp_scratch,
-            ctx->d_mlp_loss};
+    return {ctx->d_mlp, ctx->d_mlp + np, ctx->d_mlp + 2 * np, ctx->d_mlp + 3 * np,
+            (unsigned short *)(ctx->d_mlp + 4 * np), ctx->d_mlp_scratch, ctx->d_mlp_loss};
 }
 
-int mlp_alloc(mnc_ctx *ctx, int rows, size_t losses) {
-    int st;
-    if (!ctx->d_mlp &&
-        (st = dalloc(ctx, &ctx->d_mlp, 4 * (size_t(mnc::mlp_param_count()) + mnc::kMlpStats))))
-        return st;
+int mlp_alloc(mnc_ctx *ctx) {
+    if (ctx->d_mlp) return MNC_OK;
+    return dalloc(ctx, &ctx->d_mlp, 4 * (size_t(mnc::mlp_param_count()) + mnc::kMlpStats) + mnc::mlp_operand_floats());
+}
+
+int mlp_train_alloc(mnc_ctx *ctx, int rows, size_t losses) {
+    int st = mlp_alloc(ctx);
+    if (st) return st;
     const size_t need = mnc::mlp_scratch_floats(rows);
     if (need > ctx->mlp_scratch_cap) {
         if ((st = dalloc(ctx, &ctx->d_mlp_scratch, need))) return st;
@@ -270,21 +271,6 @@ int mlp_check(mnc_ctx *ctx, bool need_ready) {
     if (ctx->tab.nm != 15) return ctx_fail(ctx, MNC_ERR_ARG, "the learned warm start exists for moment order 4 only");
     if (need_ready && !ctx->mlp_ready)
         return ctx_fail(ctx, MNC_ERR_STATE, "no MLP parameters (mnc_mlp_init/mnc_mlp_set_params first)");
-    return MNC_OK;
-}
-
-// Scaled multipliers predicted for n rows of scaled moments (device arrays).
-int mlp_predict_dev(mnc_ctx *ctx, int n, const double *us, double *alpha) {
-    int st = mlp_alloc(ctx, std::min(n, kMlpChunk), 1);
-    if (st) return st;
-    const auto b = mlp_buffers(ctx);
-    for (int i0 = 0; i0 < n; i0 += kMlpChunk) {
-        const int rows = std::min(kMlpChunk, n - i0);
-        mnc::mlp_gather(b, us, nullptr, n, rows, 0, i0, ctx->stream);
-        mnc::mlp_forward(b, rows, ctx->stream);
-        mnc::mlp_unscale(b, rows, alpha + size_t(i0) * 15, ctx->stream);
-    }
-    MNC_HIP_CHECK(hipGetLastError());
     return MNC_OK;
 }
 
@@ -324,7 +310,6 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
             if ((st = dalloc(ctx, &ctx->d_guess, size_t(ncells) * 15))) return st;
             ctx->guess_cap = size_t(ncells);
         }
-        if ((st = mlp_alloc(ctx, ncells, 1))) return st;
         alpha_guess = ctx->d_guess;
     }
     mnc::NewtonArgs a{};
@@ -1499,7 +1484,7 @@ int mnc_mlp_init(mnc_ctx *ctx, unsigned long long seed) {
     int st = mlp_check(ctx, false);
     if (st) return st;
     MNC_HIP_CHECK(hipSetDevice(ctx->device));
-    if ((st = mlp_alloc(ctx, 1, 1))) return st;
+    if ((st = mlp_alloc(ctx))) return st;
     const int np = mnc::mlp_param_count();
     std::vector<float> h(size_t(np) + mnc::kMlpStats, 0.0f);
     // SplitMix64 stream -> U(-1, 1); weights U(-b, b), b = sqrt(6 / (fan_in + fan_out)); biases 0
@@ -1522,6 +1507,8 @@ int mnc_mlp_init(mnc_ctx *ctx, unsigned long long seed) {
     const size_t nall = h.size();
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp, h.data(), nall * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     MNC_HIP_CHECK(hipMemsetAsync(ctx->d_mlp + 2 * nall, 0, 2 * nall * sizeof(float), ctx->stream));   // Adam m, v
+    mnc::mlp_pack(mlp_buffers(ctx), ctx->stream);
+    MNC_HIP_CHECK(hipGetLastError());
     MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     ctx->mlp_ready = true;
     ctx->mlp_stats_set = false;
@@ -1537,7 +1524,7 @@ int mnc_mlp_train(mnc_ctx *ctx, long long npairs, const double *u_scaled, const 
     if (npairs < 1 || !u_scaled || !alpha_scaled || steps < 0 || batch < 1 || batch > (1 << 20) || !(lr > 0.0))
         return ctx_fail(ctx, MNC_ERR_ARG, "bad training arguments");
     MNC_HIP_CHECK(hipSetDevice(ctx->device));
-    if ((st = mlp_alloc(ctx, batch, size_t(std::max(steps, 1)))) || (st = mlp_io(ctx, size_t(npairs) * 30))) return st;
+    if ((st = mlp_train_alloc(ctx, batch, size_t(std::max(steps, 1)))) || (st = mlp_io(ctx, size_t(npairs) * 30))) return st;
     const size_t n15 = size_t(npairs) * 15;
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp_io, u_scaled, n15 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp_io + n15, alpha_scaled, n15 * sizeof(double), hipMemcpyHostToDevice,
@@ -1562,7 +1549,6 @@ int mnc_mlp_train(mnc_ctx *ctx, long long npairs, const double *u_scaled, const 
         ctx->mlp_stats_set = true;
     }
     const auto b0 = mlp_buffers(ctx);
-    MNC_HIP_CHECK(hipMemsetAsync(ctx->d_mlp_loss, 0, size_t(std::max(steps, 1)) * sizeof(float), ctx->stream));
     {
         Timed tm(ctx, MNC_KCLASS_MLP);
         for (int k = 0; k < steps; ++k) {
@@ -1570,10 +1556,8 @@ int mnc_mlp_train(mnc_ctx *ctx, long long npairs, const double *u_scaled, const 
             b.loss = ctx->d_mlp_loss + k;
             const int step = ++ctx->mlp_step;
             const unsigned long long sk = (seed * 0x9e3779b97f4a7c15ull) ^ (unsigned long long)(step) ^ 0x5bd1e995ull;
-            mnc::mlp_gather(b, ctx->d_mlp_io, ctx->d_mlp_io + n15, npairs, batch, sk | 1ull, 0, ctx->stream);
-            mnc::mlp_forward(b, batch, ctx->stream);
-            mnc::mlp_backward(b, batch, ctx->stream);
-            mnc::mlp_adam(b, float(lr), step, ctx->stream);
+            mnc::mlp_train_step(b, ctx->d_mlp_io, ctx->d_mlp_io + n15, npairs, batch, sk | 1ull, float(lr), step,
+                                ctx->stream);
         }
     }
     MNC_HIP_CHECK(hipGetLastError());
@@ -1596,8 +1580,9 @@ int mnc_mlp_predict(mnc_ctx *ctx, int n, const double *u_scaled, double *alpha_s
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp_io, u_scaled, n15 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     {
         Timed tm(ctx, MNC_KCLASS_MLP);
-        if ((st = mlp_predict_dev(ctx, n, ctx->d_mlp_io, ctx->d_mlp_io + n15))) return st;
+        mnc::mlp_predict(mlp_buffers(ctx), ctx->d_mlp_io, n, ctx->d_mlp_io + n15, ctx->stream);
     }
+    MNC_HIP_CHECK(hipGetLastError());
     MNC_HIP_CHECK(hipMemcpyAsync(alpha_scaled, ctx->d_mlp_io + n15, n15 * sizeof(double), hipMemcpyDeviceToHost,
                                  ctx->stream));
     MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -1620,10 +1605,12 @@ int mnc_mlp_set_params(mnc_ctx *ctx, const float *params) {
     int st = mlp_check(ctx, false);
     if (st) return st;
     MNC_HIP_CHECK(hipSetDevice(ctx->device));
-    if ((st = mlp_alloc(ctx, 1, 1))) return st;
+    if ((st = mlp_alloc(ctx))) return st;
     const size_t nall = size_t(mnc_mlp_num_params());
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp, params, nall * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     MNC_HIP_CHECK(hipMemsetAsync(ctx->d_mlp + 2 * nall, 0, 2 * nall * sizeof(float), ctx->stream));
+    mnc::mlp_pack(mlp_buffers(ctx), ctx->stream);
+    MNC_HIP_CHECK(hipGetLastError());
     MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     ctx->mlp_ready = true;
     ctx->mlp_stats_set = true;
@@ -1639,16 +1626,13 @@ int mnc_mlp_gradient(mnc_ctx *ctx, int rows, const double *u_scaled, const doubl
     if (rows < 1 || rows > (1 << 20) || !u_scaled || !alpha_scaled || !grad || !loss)
         return ctx_fail(ctx, MNC_ERR_ARG, "bad gradient arguments");
     MNC_HIP_CHECK(hipSetDevice(ctx->device));
-    if ((st = mlp_alloc(ctx, rows, 1)) || (st = mlp_io(ctx, size_t(rows) * 30))) return st;
+    if ((st = mlp_train_alloc(ctx, rows, 1)) || (st = mlp_io(ctx, size_t(rows) * 30))) return st;
     const size_t n15 = size_t(rows) * 15;
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp_io, u_scaled, n15 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
     MNC_HIP_CHECK(hipMemcpyAsync(ctx->d_mlp_io + n15, alpha_scaled, n15 * sizeof(double), hipMemcpyHostToDevice,
                                  ctx->stream));
-    MNC_HIP_CHECK(hipMemsetAsync(ctx->d_mlp_loss, 0, sizeof(float), ctx->stream));
     const auto b = mlp_buffers(ctx);
-    mnc::mlp_gather(b, ctx->d_mlp_io, ctx->d_mlp_io + n15, rows, rows, 0, 0, ctx->stream);
-    mnc::mlp_forward(b, rows, ctx->stream);
-    mnc::mlp_backward(b, rows, ctx->stream);
+    mnc::mlp_gradient(b, ctx->d_mlp_io, ctx->d_mlp_io + n15, rows, ctx->stream);
     MNC_HIP_CHECK(hipGetLastError());
     MNC_HIP_CHECK(hipMemcpyAsync(grad, b.grad, size_t(mnc::mlp_param_count()) * sizeof(float), hipMemcpyDeviceToHost,
                                  ctx->stream));

@@ -220,30 +220,32 @@ void newton_store_fields(int nm, int np2, int *dfields, int *ifields);
 
 // The learned warm start (mnc_mlp.hip).  w: the 37,007 parameters followed by
 // in_mean, in_std, out_mean, out_std (15 each); grad, m, v: like the
-// parameters; scratch: mlp_scratch_floats(rows); loss: one float (accumulated).
+// parameters; pk: the weights' bf16 matrix operands (mlp_operand_floats()
+// floats), which follow w after mlp_pack and every training step; scratch:
+// mlp_scratch_floats(rows), for training and gradients; loss: one float.
 struct MlpBuffers {
-    float *w, *grad, *m, *v, *scratch, *loss;
+    float *w, *grad, *m, *v;
+    unsigned short *pk;
+    float *scratch, *loss;
 };
 constexpr int kMlpStats = 60;
 int mlp_param_count();
+size_t mlp_operand_floats();
 size_t mlp_scratch_floats(int rows);
-// Minibatch (seed != 0: rows drawn with replacement; seed == 0: rows i0.. in
-// order; as == nullptr: inputs only) into the scratch's input/target slots.
-void mlp_gather(const MlpBuffers &b, const double *us, const double *as, long long npairs, int rows,
-                unsigned long long seed, long long i0, hipStream_t s);
-// mdev: if set, the row count is *mdev (at most rows), read on the device.
-void mlp_forward(const MlpBuffers &b, int rows, hipStream_t s, const int *mdev = nullptr);
-void mlp_backward(const MlpBuffers &b, int rows, hipStream_t s);
-void mlp_adam(const MlpBuffers &b, float lr, int step, hipStream_t s);
-// Scaled multipliers of the last forward pass into alpha[rows][15] (FP64).
-void mlp_unscale(const MlpBuffers &b, int rows, double *alpha, hipStream_t s);
-void mlp_scale_moments(const double *u, int ncells, double *us, hipStream_t s);
+void mlp_pack(const MlpBuffers &b, hipStream_t s);
+// One Adam step on `rows` pairs drawn with replacement (seed != 0); *loss <- the
+// minibatch's mean squared error.
+void mlp_train_step(const MlpBuffers &b, const double *us, const double *as, long long npairs, int rows,
+                    unsigned long long seed, float lr, int step, hipStream_t s);
+// grad and *loss of the mean squared error on all rows, in order.
+void mlp_gradient(const MlpBuffers &b, const double *us, const double *as, int rows, hipStream_t s);
+// Scaled multipliers alpha[rows][15] of the scaled moments us.
+void mlp_predict(const MlpBuffers &b, const double *us, int rows, double *alpha, hipStream_t s);
 // The network for the cells listed in list[0 .. *count) (a device count; at
 // most max_rows): scaled moments gathered from u (unscaled), guesses scattered
 // into alpha[cell][15].
 void mlp_predict_listed(const MlpBuffers &b, const double *u, const int *list, const int *count, int max_rows,
                         double *alpha, hipStream_t s);
-float *mlp_output(const MlpBuffers &b, int rows);
 
 // Arguments of the grid kernels (mnc_grid.hip).
 struct GridArgs {

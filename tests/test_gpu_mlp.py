@@ -341,3 +341,38 @@ def test_learned_fallback_restores_the_isotropic_answer():
     assert res["learned"][1] > 0 and res["no-fallback"][1] == 0 and res["iso"][1] == 0
     assert reg["learned"] <= reg["iso"]
     assert reg["no-fallback"] > reg["learned"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 511, 513, 1040])
+def test_mlp_gradient_and_update_over_row_remainders(rows):
+    """Row blocks of 16, matrix steps of 32 and groups of 16 steps with remainders:
+    the gradient against the reference, and predictions that follow a training
+    step's weights.  A bf16 operand that rounds the other way moves one of its
+    128 columns by 2^-8, hence 1e-2 of a layer's norm."""
+    print("case mlp rows %d" % rows, flush=True)
+    mnc, ctx = _ctx()
+    rng = np.random.default_rng(rows)
+    p = _params_with_stats(ctx, rng)
+    us = rng.normal(0, 0.3, (rows, 15))
+    us[:, 0] = 1.0
+    al = rng.normal(0, 2.0, (rows, 15))
+    g, loss = ctx.mlp_gradient(us, al)
+    x, t = mlp_ref.standardise(p, us, al)
+    lref, gref = mlp_ref.loss_and_grad(p, x, t, bf=True)
+    assert abs(loss - lref) <= 1e-4 * lref
+    off = 0
+    for i in range(4):
+        for n in (mlp_ref.DIMS[i] * mlp_ref.DIMS[i + 1], mlp_ref.DIMS[i + 1]):
+            assert np.linalg.norm(g[off:off + n] - gref[off:off + n]) <= 1e-2 * np.linalg.norm(gref[off:off + n])
+            off += n
+    ctx.mlp_train(us, al, steps=1, batch=rows, lr=1e-2, seed=3)
+    q = ctx.mlp_params().astype(np.float64)
+    assert np.abs(q - p)[:mlp_ref.NPARAM].max() > 1e-3
+    x, _ = mlp_ref.standardise(q, us)
+    _, st = mlp_ref.unpack(q)
+    y = mlp_ref.forward(q, x, bf=True)[1][-1] * st[3] + st[2]
+    got = ctx.mlp_predict(us)
+    err = np.abs(got - y) / np.abs(y).max()
+    assert np.median(err) <= 1e-5 and err.max() <= 1e-2
+    ctx.close()
