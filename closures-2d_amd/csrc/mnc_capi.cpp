@@ -94,6 +94,9 @@ struct mnc_ctx {
     float *d_mlp = nullptr;          // parameters + standardisation, grad, m, v (4 blocks)
     float *d_mlp_scratch = nullptr, *d_mlp_loss = nullptr;
     size_t mlp_scratch_cap = 0, mlp_loss_cap = 0;
+    double *d_cb_batch = nullptr;    // the host-array optcb entry's arrays and workspace, its outputs
+    mnc_outs *d_cb_outs = nullptr;
+    size_t cb_batch_cap = 0, cb_outs_cap = 0;
     double *d_mlp_io = nullptr;      // host-call staging (inputs, targets/outputs)
     size_t mlp_io_cap = 0;
     double *d_us = nullptr, *d_guess = nullptr;   // Newton prologue: u/u0 and the MLP guesses
@@ -724,7 +727,7 @@ void mnc_destroy(mnc_ctx *ctx) {
     void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_pT, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
                     ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gg, ctx->d_gh,
                     ctx->d_ot, ctx->d_opos, ctx->d_ogoff, ctx->d_ogk, ctx->d_ogv,
-                    ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
+                    ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
                     ctx->d_ctl, ctx->d_stats, ctx->d_std, ctx->d_sti, ctx->d_lists, ctx->d_mom, ctx->d_alpha, ctx->d_old,
                     ctx->d_st, ctx->d_ss, ctx->d_flux, ctx->d_ansatz, ctx->d_fpart, ctx->d_bu, ctx->d_ba, ctx->d_bo,
                     ctx->d_cbB, ctx->d_cbaP, ctx->d_cbws, ctx->d_tflag};
@@ -833,13 +836,21 @@ int mnc_optcb_batch_host(mnc_ctx *ctx, int ncells, double *u, double *P2M, doubl
     const int nm = ctx->tab.nm, nq = ctx->tab.nq;
     const int blocks = std::min(ncells, 16 * ctx->num_cu);
     const size_t nv = size_t(ncells) * nm, nb = size_t(ncells) * nm * nm, nws = size_t(blocks) * nq * nm;
-    double *d = nullptr;
-    mnc_outs *d_outs = nullptr;
-    MNC_HIP_CHECK(hipMalloc((void **)&d, (3 * nv + nb + nws) * sizeof(double)));
-    if (hipMalloc((void **)&d_outs, size_t(ncells) * sizeof(mnc_outs)) != hipSuccess) {
-        (void)hipFree(d);
-        return ctx_fail(ctx, MNC_ERR_HIP, "hipMalloc failed");
+    // the context keeps the largest batch's buffers: 126 MB of workspace at M4,
+    // whose allocation and release took longer than the solve of 5,000 cells
+    const size_t nd = 3 * nv + nb + nws;
+    if (nd > ctx->cb_batch_cap) {
+        ctx->cb_batch_cap = 0;
+        if ((st = dalloc(ctx, &ctx->d_cb_batch, nd))) return st;
+        ctx->cb_batch_cap = nd;
     }
+    if (size_t(ncells) > ctx->cb_outs_cap) {
+        ctx->cb_outs_cap = 0;
+        if ((st = dalloc(ctx, &ctx->d_cb_outs, size_t(ncells)))) return st;
+        ctx->cb_outs_cap = size_t(ncells);
+    }
+    double *d = ctx->d_cb_batch;
+    mnc_outs *d_outs = ctx->d_cb_outs;
     double *d_u = d, *d_aP = d + nv, *d_aM = d + 2 * nv, *d_B = d + 3 * nv, *d_ws = d_B + nb;
     mnc::CbArgs a{};
     a.ncells = ncells;
@@ -887,10 +898,7 @@ int mnc_optcb_batch_host(mnc_ctx *ctx, int ncells, double *u, double *P2M, doubl
         MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         return s2;
     };
-    st = run();
-    (void)hipFree(d);
-    (void)hipFree(d_outs);
-    return st;
+    return run();
 }
 
 int mnc_batch_set(mnc_ctx *ctx, int ncells, const double *u, const double *alpha) {

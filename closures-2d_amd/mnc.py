@@ -43,6 +43,10 @@ class Outs(C.Structure):
     _fields_ = [("r", C.c_double), ("iter", C.c_int), ("norm_g", C.c_double)]
 
 
+# the same record for numpy: a batch's fields come out as strided copies, not cell by cell
+OUTS_DTYPE = np.dtype([(n, t) for n, t in Outs._fields_], align=True)
+
+
 class GridDesc(C.Structure):
     _fields_ = [("num_cells_x", C.c_int), ("num_cells_y", C.c_int), ("dx", C.c_double),
                 ("dy", C.c_double), ("init_x", C.c_double), ("init_y", C.c_double),
@@ -203,11 +207,9 @@ class Context:
         n = self._batch_n
         u = np.zeros((n, self.nm))
         a = np.zeros((n, self.nm))
-        outs = (Outs * n)()
-        self._check(lib().mnc_batch_get(self.h, _p(u), _p(a), outs), "mnc_batch_get")
-        it = np.array([o.iter for o in outs], dtype=np.int32)
-        r = np.array([o.r for o in outs])
-        return u, a, it, r
+        outs = np.zeros(n, dtype=OUTS_DTYPE)
+        self._check(lib().mnc_batch_get(self.h, _p(u), _p(a), outs.ctypes.data_as(C.POINTER(Outs))), "mnc_batch_get")
+        return u, a, outs["iter"].copy(), outs["r"].copy()
 
     def opt_batch_host(self, u, alpha, opt=None, allow_status=(OK,)):
         """Batched opt() on host arrays; returns (status, u, alpha, iter, r, normG)."""
@@ -215,13 +217,12 @@ class Context:
         u = np.array(u, dtype=np.float64, order="C").reshape(-1, self.nm)
         alpha = np.array(alpha, dtype=np.float64, order="C").reshape(-1, self.nm)
         n = u.shape[0]
-        outs = (Outs * max(n, 1))()
-        st = lib().mnc_opt_batch_host(self.h, n, _p(u), _p(alpha), C.byref(opt), outs)
+        outs = np.zeros(n, dtype=OUTS_DTYPE)
+        st = lib().mnc_opt_batch_host(self.h, n, _p(u), _p(alpha), C.byref(opt),
+                                      outs.ctypes.data_as(C.POINTER(Outs)))
         if st not in allow_status:
             self._check(st, "mnc_opt_batch_host")
-        it = np.array([o.iter for o in outs[:n]], dtype=np.int32)
-        r = np.array([o.r for o in outs[:n]])
-        ng = np.array([o.norm_g for o in outs[:n]])
+        it, r, ng = outs["iter"].copy(), outs["r"].copy(), outs["norm_g"].copy()
         return st, u, alpha, it, r, ng
 
     def optcb_batch_host(self, u, P2M, alphaP, opt=None, allow_status=(OK,)):
@@ -235,13 +236,12 @@ class Context:
         P2M = np.array(P2M, dtype=np.float64, order="C").reshape(n, self.nm * self.nm)
         alphaP = np.array(alphaP, dtype=np.float64, order="C").reshape(n, self.nm)
         alphaM = np.zeros_like(alphaP)
-        outs = (Outs * max(n, 1))()
-        st = lib().mnc_optcb_batch_host(self.h, n, _p(u), _p(P2M), _p(alphaP), _p(alphaM), C.byref(opt), outs)
+        outs = np.zeros(n, dtype=OUTS_DTYPE)
+        st = lib().mnc_optcb_batch_host(self.h, n, _p(u), _p(P2M), _p(alphaP), _p(alphaM), C.byref(opt),
+                                        outs.ctypes.data_as(C.POINTER(Outs)))
         if st not in allow_status:
             self._check(st, "mnc_optcb_batch_host")
-        it = np.array([o.iter for o in outs[:n]], dtype=np.int32)
-        r = np.array([o.r for o in outs[:n]])
-        ng = np.array([o.norm_g for o in outs[:n]])
+        it, r, ng = outs["iter"].copy(), outs["r"].copy(), outs["norm_g"].copy()
         return st, u, P2M, alphaP, alphaM, it, r, ng
 
     # ---- grid ----
