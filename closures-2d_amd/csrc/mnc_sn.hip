@@ -30,21 +30,18 @@ constexpr int kSnThreads = 256;
 struct SnArgs {
     int nx, ny, nq, init_cond;
     double dx, dy, dt, init_x, init_y;
-    const double *w, *xi, *eta;       // [nq]
+    const double *w, *xi, *eta;       // [nq]; the speeds over the cell sizes, xi / dx and eta / dy
     const double *sigma_t, *sigma_s;  // [(nx+4)(ny+4)]
 };
 
-// The reference's selects as v_min / v_max (kinetic_update.cpp:22-25):
-// fabs(x) < y s ? fabs(x) : y s is fmin(fabs(x), y s) and m > 0 ? m : 0 is
-// fmax(m, 0) -- equal values, NaN included; only the sign of an exact zero
-// slope may differ, which a sum with any nonzero term does not see.
-__device__ __forceinline__ double sn_minmod(double x, double y) {
-    const double s = (x >= 0.0) ? 1.0 : -1.0;
-    const double m = fmin(fabs(x), y * s);
-    return s * fmax(m, 0.0);
-}
-__device__ __forceinline__ double sn_slopefit(double l, double c, double r) {   // :31-35, theta = 2
-    return sn_minmod(2.0 * (r - c), sn_minmod(0.5 * (r - l), 2.0 * (c - l)));
+// The reference's slope fit (kinetic_update.cpp:22-35, theta = 2) in twelve
+// instructions: with d1 = r - c and d2 = c - l of opposite signs it is 0, else the
+// smallest of 2|d1|, 2|d2| and |r - l|/2 with their sign -- equal values; only the
+// sign of an exact zero may differ, which a sum with any nonzero term does not see.
+__device__ __forceinline__ double sn_slope(double l, double c, double r) {
+    const double d1 = r - c, d2 = c - l;
+    const double v = fmin(2.0 * fmin(fabs(d1), fabs(d2)), 0.5 * fabs(r - l));
+    return (__double2hiint(d1) ^ __double2hiint(d2)) < 0 ? 0.0 : copysign(v, d1);
 }
 
 // ghosts of f (and of f2 when not null) <- the opposite interior layers of f
@@ -99,7 +96,8 @@ __global__ __launch_bounds__(kSnThreads) void sn_stage_kernel(SnArgs a, const do
         const int rows_per = sn_rows_per_xcd(a.nx);
         const int r0 = (blockIdx.x & 7) * rows_per;
         const int rows = min(a.nx, r0 + rows_per) - r0;
-        const int L = (blockIdx.x >> 3) * kSnWaves + (threadIdx.x >> 6);   // the XCD's cell, strip order
+        // the wave's number and with it its cell in scalar registers
+        const int L = (blockIdx.x >> 3) * kSnWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the XCD's cell, strip order
         if (rows <= 0 || L >= rows * a.ny) return;   // uniform over the wave; no block barrier follows
         const int full = rows * kSnStrip;             // cells of a full strip
         const int sidx = L / full, j0 = sidx * kSnStrip;
@@ -116,26 +114,36 @@ __global__ __launch_bounds__(kSnThreads) void sn_stage_kernel(SnArgs a, const do
         // evaluates the source test |x| < 0.5 (kinetic_update.cpp:173-175)
         const double x_i = edge_coord(a.init_x, i, a.dx), y_j = edge_coord(a.init_y, j, a.dy);
         const bool src = a.init_cond == 1 && fabs(x_i) < 0.5 && fabs(y_j) < 0.5;
-        const size_t sx = size_t(NY) * nq;     // x neighbour stride; y neighbours are nq apart
+        // The neighbours' places: x and y rows apart, the opposite layers past a
+        // periodic side (no ghost fill between the stages).
+        const bool wrap = a.init_cond == 2;
+        auto at = [&](int ii, int jj) -> const double * {
+            if (wrap) {
+                ii = ii < 2 ? ii + a.nx : ii >= a.nx + 2 ? ii - a.nx : ii;
+                jj = jj < 2 ? jj + a.ny : jj >= a.ny + 2 ? jj - a.ny : jj;
+            }
+            return in + (size_t(ii) * NY + jj) * nq;
+        };
+        const double *fc = at(i, j), *fym2 = at(i, j - 2), *fym1 = at(i, j - 1), *fyp1 = at(i, j + 1), *fyp2 = at(i, j + 2);
+        const double *fxm2 = at(i - 2, j), *fxm1 = at(i - 1, j), *fxp1 = at(i + 1, j), *fxp2 = at(i + 2, j);
         for (int q = lane; q < nq; q += 64) {
             // The upwind side differs between the lanes' ordinates, so both
             // sides' stencils are selected, not branched to (a branch would
             // run both slope fits on every wave).  s + h * slope with h = +-0.5
             // is the reference's s +- 0.5 * slope exactly (0.5 * slope is exact).
-            const double *f = in + c * nq + q;
-            const double c0 = f[0];
-            const double ym2 = f[-2 * nq], ym1 = f[-nq], yp1 = f[nq], yp2 = f[2 * nq];
-            const double xm2 = f[-2 * sx], xm1 = f[-sx], xp1 = f[sx], xp2 = f[2 * sx];
+            const double c0 = fc[q];
+            const double ym2 = fym2[q], ym1 = fym1[q], yp1 = fyp1[q], yp2 = fyp2[q];
+            const double xm2 = fxm2[q], xm1 = fxm1[q], xp1 = fxp1[q], xp2 = fxp2[q];
             const double xiq = a.xi[q], etq = a.eta[q];
             const bool ep = etq > 0, xp = xiq > 0;
             const double hy = ep ? 0.5 : -0.5, hx = xp ? 0.5 : -0.5;
             const double y1 = ep ? ym2 : ym1, y2 = ep ? ym1 : c0, y3 = ep ? c0 : yp1, y4 = ep ? yp1 : yp2;
             const double x1 = xp ? xm2 : xm1, x2 = xp ? xm1 : c0, x3 = xp ? c0 : xp1, x4 = xp ? xp1 : xp2;
-            const double nF = y3 + hy * sn_slopefit(y2, y3, y4);
-            const double sF = y2 + hy * sn_slopefit(y1, y2, y3);
-            const double eF = x3 + hx * sn_slopefit(x2, x3, x4);
-            const double wF = x2 + hx * sn_slopefit(x1, x2, x3);
-            const double flux = (eF - wF) * xiq / a.dx + (nF - sF) * etq / a.dy;
+            const double nF = y3 + hy * sn_slope(y2, y3, y4);
+            const double sF = y2 + hy * sn_slope(y1, y2, y3);
+            const double eF = x3 + hx * sn_slope(x2, x3, x4);
+            const double wF = x2 + hx * sn_slope(x1, x2, x3);
+            const double flux = (eF - wF) * xiq + (nF - sF) * etq;
             double v = c0;
             v = v - a.dt * st * v + a.dt * integral;
             if (src) v = v + a.dt;
@@ -159,6 +167,9 @@ extern "C" int mnc_sn_run(int nx, int ny, int quad_order, double dx, double dy, 
     mnc::Tables t;
     if (mnc::build_tables(1, quad_order, 0, t) != MNC_OK) return MNC_ERR_ARG;   // the same ordinates
     const int nq = t.nq;
+    std::vector<double> vx(t.xi.begin(), t.xi.begin() + nq), vy(t.eta.begin(), t.eta.begin() + nq);
+    for (double &v : vx) v /= dx;
+    for (double &v : vy) v /= dy;
     const size_t ncell = size_t(nx + 4) * (ny + 4), n = ncell * nq;
     if (hipSetDevice(device) != hipSuccess) return MNC_ERR_HIP;
     double *d = nullptr;
@@ -174,8 +185,8 @@ extern "C" int mnc_sn_run(int nx, int ny, int quad_order, double dx, double dy, 
         ok(hipMemcpyAsync(st, sigma_t, ncell * sizeof(double), hipMemcpyHostToDevice, s)) &&
         ok(hipMemcpyAsync(ss, sigma_s, ncell * sizeof(double), hipMemcpyHostToDevice, s)) &&
         ok(hipMemcpyAsync(w, t.w.data(), nq * sizeof(double), hipMemcpyHostToDevice, s)) &&
-        ok(hipMemcpyAsync(xi, t.xi.data(), nq * sizeof(double), hipMemcpyHostToDevice, s)) &&
-        ok(hipMemcpyAsync(eta, t.eta.data(), nq * sizeof(double), hipMemcpyHostToDevice, s)) &&
+        ok(hipMemcpyAsync(xi, vx.data(), nq * sizeof(double), hipMemcpyHostToDevice, s)) &&
+        ok(hipMemcpyAsync(eta, vy.data(), nq * sizeof(double), hipMemcpyHostToDevice, s)) &&
         ok(hipEventRecord(e0, s))) {
         SnArgs a{nx, ny, nq, init_cond, dx, dy, dt, init_x, init_y, w, xi, eta, st, ss};
         // four cells each, one row range per XCD
@@ -183,16 +194,14 @@ extern "C" int mnc_sn_run(int nx, int ny, int quad_order, double dx, double dy, 
         const long long gw = 2LL * (nx + ny) * nq;
         const int gblocks = int(std::min<long long>((gw + 255) / 256, 4096));
         for (int k = 0; k < steps && rc == MNC_OK; ++k) {
-            // the reference fills the ghosts of its one array before each stage,
-            // so after the step they hold the first stage's layers: the second
-            // fill writes them into the state too
-            if (init_cond == 2)
-                hipLaunchKernelGGL(sn_ghost_kernel, dim3(gblocks), dim3(256), 0, s, f, (double *)nullptr, nx, ny, nq);
             hipLaunchKernelGGL(sn_stage_kernel, dim3(blocks), dim3(kSnThreads), 0, s, a, f, f1, nullptr);
-            if (init_cond == 2) hipLaunchKernelGGL(sn_ghost_kernel, dim3(gblocks), dim3(256), 0, s, f1, f, nx, ny, nq);
             hipLaunchKernelGGL(sn_stage_kernel, dim3(blocks), dim3(kSnThreads), 0, s, a, f1, f, f);
             ok(hipGetLastError());
         }
+        // the reference fills the ghosts of its one array before each stage, so
+        // at the end they hold the last first stage's layers
+        if (init_cond == 2 && steps > 0)
+            hipLaunchKernelGGL(sn_ghost_kernel, dim3(gblocks), dim3(256), 0, s, f1, f, nx, ny, nq);
         if (ok(hipEventRecord(e1, s)) && ok(hipMemcpyAsync(kinetic, f, n * sizeof(double), hipMemcpyDeviceToHost, s)) &&
             ok(hipStreamSynchronize(s)) && kernel_ms) {
             float ms = 0.0f;

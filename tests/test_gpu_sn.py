@@ -48,6 +48,16 @@ def test_sn_centre_source_fixed_ghosts_matches_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ic", [1, 2])
+@pytest.mark.parametrize("nx,ny,Q", [(2, 2, 2), (3, 70, 4), (65, 18, 12), (4, 3, 32)])
+def test_sn_smallest_and_ragged_grids_match_oracle(nx, ny, Q, ic):
+    """Periodic neighbours read from the opposite side on the smallest grids, rows
+    past a strip, ordinates below and past a wave."""
+    f, g, o, rel = _case(nx, ny, Q, 10 * Q + ic, ic, 3, 2.0 / nx, 2.2 / ny, -1.0, -1.1, 0.3 / (nx + ny))
+    assert rel <= 1e-13
+
+
+@pytest.mark.gpu
 def test_sn_mass_conservation_at_size():
     """128 x 128 cells, Q = 16 (256 ordinates), sigma_t = sigma_s per cell,
     periodic: the total sum_q w_q f_q stays to rounding over 20 steps."""
