@@ -75,6 +75,9 @@ struct mnc_ctx {
     double *d_mom = nullptr, *d_alpha = nullptr, *d_old = nullptr, *d_st = nullptr, *d_ss = nullptr,
            *d_flux = nullptr, *d_ansatz = nullptr, *d_fpart = nullptr;
     int ansatz_chunk = 0;
+    mnc::FluxTables ftab;            // orders 5 to 8
+    double *d_foz = nullptr, *d_fop = nullptr, *d_fodir = nullptr;
+    int *d_foidx = nullptr;
     int *d_tflag = nullptr;          // flux_tile 3 tile flags (flux_overlap)
     hipStream_t stream2 = nullptr;   // the second stream of flux_overlap (default priority)
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -596,8 +599,16 @@ mnc::GridArgs grid_args(mnc_ctx *ctx) {
     g.delta = ctx->grid.delta_ppn;
     g.tile_flag = ctx->d_tflag;
     g.tile_mode = 0;
+    g.oz = ctx->d_foz;
+    g.op = ctx->d_fop;
+    g.odir = ctx->d_fodir;
+    g.oidx = ctx->d_foidx;
+    g.ont = ctx->ftab.nt;
     return g;
 }
+
+// Nodes the unfused flux's ansatz holds: whole tiles of 16 orbits above order 4.
+int ansatz_nodes(const mnc_ctx *ctx) { return ctx->ftab.nt > 0 ? 64 * ctx->ftab.nt : ctx->tab.nq; }
 
 // solveFlux (+ Euler stage when stage > 0) over all quadrature chunks.
 int flux_stage(mnc_ctx *ctx, int stage, double dt) {
@@ -609,7 +620,7 @@ int flux_stage(mnc_ctx *ctx, int stage, double dt) {
         MNC_HIP_CHECK(hipGetLastError());
         return MNC_OK;
     }
-    const int nq = ctx->tab.nq, ch = ctx->ansatz_chunk;
+    const int nq = ansatz_nodes(ctx), ch = ctx->ansatz_chunk;
     for (int q0 = 0; q0 < nq; q0 += ch) {
         const int nqc = std::min(ch, nq - q0);
         {
@@ -691,9 +702,15 @@ int mnc_create(const mnc_setup *setup, mnc_ctx **out) {
         }
     }
     // above n = 15 the fused flux's halo of alpha (20 x 20 cells does not fit,
-    // 12 x 12 leaves two waves per CU) is slower than the ansatz through HBM
-    // (M8 512^2: 18.3 against 8.3 ms per stage, the same results)
+    // 12 x 12 leaves two waves per CU) loses to the ansatz through HBM, whose two
+    // passes go by orbits on the matrix cores (M8 96^2: 0.11 ms a stage)
     if (t.nm > 15) ctx->flux_tile = 0;
+    if (t.N >= 5 && t.N <= 8 &&
+        (mnc::build_flux_tables(t, ctx->ftab) != MNC_OK || up(&ctx->d_foz, ctx->ftab.z) || up(&ctx->d_fop, ctx->ftab.p) ||
+         up(&ctx->d_fodir, ctx->ftab.dir) || up(&ctx->d_foidx, ctx->ftab.idx))) {
+        mnc_destroy(ctx);
+        return MNC_ERR_HIP;
+    }
     if (!ctx->ppn && t.nm == 45 && mnc::build_g64_tables(setup->moment_order, setup->quad_order, ctx->g64) == MNC_OK &&
         ctx->g64.kz == 12 && ctx->g64.ngt == 3 && ctx->g64.nht == 10) {   // the instantiated tile counts
         if (up(&ctx->d_gz, ctx->g64.z) || up(&ctx->d_gg, ctx->g64.g) || up(&ctx->d_gh, ctx->g64.h) ||
@@ -727,7 +744,7 @@ void mnc_destroy(mnc_ctx *ctx) {
     void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_pT, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
                     ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gg, ctx->d_gh,
                     ctx->d_ot, ctx->d_opos, ctx->d_ogoff, ctx->d_ogk, ctx->d_ogv,
-                    ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
+                    ctx->d_foz, ctx->d_fop, ctx->d_fodir, ctx->d_foidx, ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
                     ctx->d_ctl, ctx->d_stats, ctx->d_std, ctx->d_sti, ctx->d_lists, ctx->d_mom, ctx->d_alpha, ctx->d_old,
                     ctx->d_st, ctx->d_ss, ctx->d_flux, ctx->d_ansatz, ctx->d_fpart, ctx->d_bu, ctx->d_ba, ctx->d_bo,
                     ctx->d_cbB, ctx->d_cbaP, ctx->d_cbws, ctx->d_tflag};
@@ -967,8 +984,9 @@ int mnc_grid_create(mnc_ctx *ctx, const mnc_grid_desc *grid, const double *momen
         return st;
     // ansatz buffer: all q at once unless that exceeds 8 GiB
     const size_t max_elems = (size_t(8) << 30) / sizeof(double);
-    int ch = ctx->tab.nq;
+    int ch = ansatz_nodes(ctx);
     while (ch > 1 && size_t(ch) * nc > max_elems) ch = (ch + 1) / 2;
+    if (ctx->ftab.nt > 0) ch = (ch + 63) / 64 * 64;
     ctx->ansatz_chunk = ch;
     if ((st = dalloc(ctx, &ctx->d_ansatz, size_t(ch) * nc))) return st;
     MNC_HIP_CHECK(hipMemcpy(ctx->d_mom, moments, n * sizeof(double), hipMemcpyHostToDevice));

@@ -6,7 +6,11 @@
 // [(i*(ny+4)+j)][k] (x-major, 2 ghost cells per side); the ansatz is stored
 // [q][cell] so that, for one quadrature direction, neighbouring threads (cells)
 // read neighbouring words.
+#include <algorithm>
+#include <type_traits>
+
 #include "mnc_internal.h"
+#include "mnc_orbit.h"
 
 namespace mnc {
 namespace {
@@ -303,13 +307,6 @@ __global__ void ghost_y_kernel(GridArgs g) {
     g.moments[(size_t(i) * NY + y3 + jj) * nm + k] = g.moments[(size_t(i) * NY + y1 + jj) * nm + k];
 }
 
-template <int NM>
-void launch_flux_t(const GridArgs &g, int q0, int nqc, int stage, double dt, bool fc, bool lc, hipStream_t s) {
-    const int n = g.nx * g.ny;
-    hipLaunchKernelGGL(flux_euler_kernel<NM>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, g, q0, nqc,
-                       stage, dt, int(fc), int(lc));
-}
-
 // The fused ansatz + flux with the directions split into gridDim.z groups of
 // consecutive q: block (tile, z) sums the flux of its TX x TY cells over group
 // z's directions into fpart[z] (interior cells, [cell][k]), and
@@ -451,10 +448,225 @@ void launch_fused_t(const GridArgs &g, int tile, int stage, double dt, hipStream
                        stage, dt);
 }
 
+// ---- flux of the orders 5 to 8 through HBM, on the matrix cores ---------------
+//
+// The ansatz at the four images of an orbit (mnc_orbit.h) needs one pass over the
+// moments: z = sum of four class sums with signs; and the moments of the four
+// fluxes one pass back: F_k = sum over orbits of m_k C[class of k], C the signed
+// sums of the images' fluxes.  Both passes are products on the matrix cores,
+// sixteen cells a wave.
+//
+// A lane per cell and one direction at a time these were 965 us (ansatz) and
+// 1,709 us (flux) at 96 x 96 M8 cells and 1,024 directions, on 40 blocks and a
+// serial walk over all directions; the products are a quarter of the FMAs, and
+// the two take 31 and 75 us.
+
+typedef double gf64x4 __attribute__((ext_vector_type(4)));
+
+template <int N>
+struct FluxShape {
+    static constexpr int kz(int c) { return (orbit_class_size(N, c) + 3) / 4; }
+    static constexpr int k0(int c) { return c == 0 ? 0 : k0(c - 1) + kz(c - 1); }
+    static constexpr int KZ = k0(4);
+};
+template <class T>
+__device__ __forceinline__ void each_class(T &&f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+    f(std::integral_constant<int, 3>{});
+}
+
+// E[4 orbit + image][cell] of the orbit tiles T0 .. T0 + ntc - 1.  A wave takes 16
+// cells and every gridDim.y-th tile.  Bound by the exponentials and the store (82 MB at 96^2).
+template <int N>
+__global__ __launch_bounds__(256) void ansatz_orbit_kernel(GridArgs g, int T0, int ntc) {
+    using F = FluxShape<N>;
+    constexpr int NM = orbit_nm(N);
+    const int ncell = g.NX * g.NY;
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const int cell = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + (lane & 15);
+    const int src = min(cell, ncell - 1);
+    double al[F::KZ];
+    each_class([&](auto C) {
+        constexpr int c = decltype(C)::value, n = F::kz(c), at = F::k0(c);
+#pragma unroll
+        for (int kk = 0; kk < n; ++kk) {
+            const int k = g.oidx[c * 16 + 4 * kk + q];
+            al[at + kk] = k >= 0 ? g.alpha[size_t(src) * NM + k] : 0.0;
+        }
+    });
+    for (int T = blockIdx.y; T < ntc; T += gridDim.y) {
+        const double *zt = g.oz + size_t(T0 + T) * F::KZ * 64 + lane;
+        gf64x4 z[4];
+        each_class([&](auto C) {
+            constexpr int c = decltype(C)::value, n = F::kz(c), at = F::k0(c);
+            z[c] = gf64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int kk = 0; kk < n; ++kk)
+                z[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(zt[(at + kk) * 64], al[at + kk], z[c], 0, 0, 0);
+        });
+        if (cell >= ncell) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            double *E = g.ansatz + size_t(64 * T + 4 * mfma_f64_row(r, q)) * ncell + cell;
+            const double ep = z[0][r] + z[1][r], em = z[0][r] - z[1][r], op = z[2][r] + z[3][r], om = z[2][r] - z[3][r];
+            E[0] = ansatz_value(g, ep + op);
+            E[size_t(ncell)] = ansatz_value(g, em + om);             // -xi: classes 1 and 3 change sign
+            E[2 * size_t(ncell)] = ansatz_value(g, ep - op);         // -eta: classes 2 and 3
+            E[3 * size_t(ncell)] = ansatz_value(g, em - om);         // both: classes 1 and 2
+        }
+    }
+}
+
+// minmod(theta (r - c), (r - l) / 2, theta (c - l)): 0 unless all three share
+// their sign, else the smallest magnitude with it (slopefit's values).
+__device__ __forceinline__ double slope3(double l, double c, double r, double theta) {
+    const double a = theta * (r - c), b = theta * (c - l), m = 0.5 * (r - l);
+    const double v = fmin(fmin(fabs(a), fabs(b)), fabs(m));
+    const int s = __double2hiint(m);
+    return ((__double2hiint(a) ^ s) | (__double2hiint(b) ^ s)) < 0 ? 0.0 : copysign(v, m);
+}
+
+// Difference of the face values around c for the upwind side `up` (+1: the wind
+// comes from below).
+template <int UP>
+__device__ __forceinline__ double face_diff(double m2, double m1, double c, double p1, double p2, double theta) {
+    if constexpr (UP > 0) return c + 0.5 * slope3(m1, c, p1, theta) - m1 - 0.5 * slope3(m2, m1, c, theta);
+    else return p1 - 0.5 * slope3(c, p1, p2, theta) - c + 0.5 * slope3(m1, c, p1, theta);
+}
+
+constexpr int kFluxWaves = 8;
+
+// Flux of sixteen interior cells a block, then the Euler stage; the block's waves
+// share the steps of four orbits (lane: cell lane % 16, orbit lane / 16), so that
+// 96^2 cells are 4,608 waves.  Bound by the L1/L2 reads of the stencil (28 words a
+// cell and orbit; XCD b % 8 owns a contiguous range of cells so that the x
+// neighbours' rows stay in its L2).
+template <int N>
+__global__ __launch_bounds__(64 * kFluxWaves) void flux_orbit_kernel(GridArgs g, int T0, int ntc, int stage, double dt,
+                                                                     int first_chunk, int last_chunk) {
+    constexpr int NM = orbit_nm(N);
+    __shared__ double red[4][16][64];
+    const int cells = g.nx * g.ny, tiles = (cells + 15) / 16, per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || tile >= tiles) return;           // uniform over the block
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, q = lane >> 4;
+    const size_t ncell = size_t(g.NX) * g.NY, NY = g.NY;
+    const int idx = min(tile * 16 + (lane & 15), cells - 1);
+    const size_t at = size_t(2 + idx / g.ny) * NY + 2 + idx % g.ny;
+    const double theta = g.theta, rdx = 1.0 / g.dx, rdy = 1.0 / g.dy;
+    gf64x4 acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = gf64x4{0.0, 0.0, 0.0, 0.0};
+    for (int s = wv; s < 4 * ntc; s += kFluxWaves) {
+        const int o = 4 * s + q;
+        const double *d = g.odir + size_t(16 * T0 + o) * 4;
+        const double fx = d[0] * d[2] * rdx, fy = d[1] * d[2] * rdy;
+        const double *E = g.ansatz + size_t(4 * o) * ncell + at;
+        const double *pt = g.op + size_t(4 * T0 + s) * 256 + lane;
+        double comb[4];
+        auto image = [&](auto img) {
+            constexpr int I = decltype(img)::value;
+            constexpr int UX = I & 1 ? -1 : 1, UY = I & 2 ? -1 : 1;
+            const double *e = E + size_t(I) * ncell;
+            const double c = e[0], xm1 = *(e - NY), xp1 = e[NY], ym1 = *(e - 1), yp1 = e[1];
+            const double xo = UX > 0 ? *(e - 2 * NY) : e[2 * NY], yo = UY > 0 ? *(e - 2) : e[2];
+            comb[I] = UX * fx * face_diff<UX>(xo, xm1, c, xp1, xo, theta) + UY * fy * face_diff<UY>(yo, ym1, c, yp1, yo, theta);
+        };
+        each_class(image);
+        const double ep = comb[0] + comb[1], em = comb[0] - comb[1], op = comb[2] + comb[3], om = comb[2] - comb[3];
+        const double C[4] = {ep + op, em + om, ep - op, em - om};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(C[c], pt[c * 64], acc[c], 0, 0, 0);
+    }
+    // the waves' sums: 4 .. 7 onto 0 .. 3, then wave c takes class c of those four
+    auto put = [&](int v) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[v][4 * c + r][lane] = acc[c][r];
+    };
+    if (wv >= 4) put(wv - 4);
+    __syncthreads();
+    if (wv < 4) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[c][r] += red[wv][4 * c + r][lane];
+        put(wv);
+    }
+    __syncthreads();
+    if (wv >= 4) return;
+    // element r of lane l: cell mfma_f64_row(r, l / 16), moment l % 16 of the class
+    const int k = g.oidx[wv * 16 + (lane & 15)];
+    if (k < 0) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int id = tile * 16 + mfma_f64_row(r, q);
+        if (id >= cells) continue;
+        const int i = 2 + id / g.ny, j = 2 + id % g.ny;
+        const size_t cc = size_t(i) * NY + j, o = cc * NM + k;
+        double Fk = (red[0][4 * wv + r][lane] + red[1][4 * wv + r][lane]) + (red[2][4 * wv + r][lane] + red[3][4 * wv + r][lane]);
+        if (!first_chunk) Fk += g.flux[o];
+        if (!last_chunk || stage == 0) {
+            g.flux[o] = Fk;
+            continue;
+        }
+        // the Euler stage of euler_epilogue, one moment a lane
+        const double st = g.sigma_t[cc], u = g.moments[o];
+        double v;
+        if (k == 0) {
+            v = u * (1.0 + dt * g.sigma_s[cc] - dt * st) - dt * Fk;
+            if (g.init_cond == 1 && fabs(edge_coord(g.init_x, i - 2, g.dx)) < 0.5 && fabs(edge_coord(g.init_y, j - 2, g.dy)) < 0.5)
+                v = v + dt * 2.0 * sqrt(M_PI);
+        } else {
+            v = u * (1.0 - dt * st) - dt * Fk;
+        }
+        if (stage == 2) v = 0.5 * (v + g.moments_old[o]);
+        g.moments[o] = v;
+    }
+}
+
+template <int NM> constexpr int order_of_nm() {
+    int N = 0;
+    while (orbit_nm(N) < NM) ++N;
+    return N;
+}
+
+template <int NM>
+void launch_ansatz_orbit(const GridArgs &g, int T0, int ntc, hipStream_t s) {
+    const int bx = (g.NX * g.NY + 63) / 64;
+    const int by = std::min(ntc, std::max(1, 1024 / bx));      // about four waves per SIMD
+    hipLaunchKernelGGL(ansatz_orbit_kernel<order_of_nm<NM>()>, dim3(bx, by), dim3(256), 0, s, g, T0, ntc);
+}
+
+template <int NM>
+void launch_flux_orbit(const GridArgs &g, int T0, int ntc, int stage, double dt, bool fc, bool lc, hipStream_t s) {
+    const int tiles = (g.nx * g.ny + 15) / 16;
+    hipLaunchKernelGGL(flux_orbit_kernel<order_of_nm<NM>()>, dim3(8 * ((tiles + 7) / 8)), dim3(64 * kFluxWaves), 0, s, g,
+                       T0, ntc, stage, dt, int(fc), int(lc));
+}
+
+template <int NM>
+void launch_flux_t(const GridArgs &g, int q0, int nqc, int stage, double dt, bool fc, bool lc, hipStream_t s) {
+    if constexpr (NM > 15) {
+        launch_flux_orbit<NM>(g, q0 / 64, nqc / 64, stage, dt, fc, lc, s);
+    } else {
+        const int n = g.nx * g.ny;
+        hipLaunchKernelGGL(flux_euler_kernel<NM>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, g, q0, nqc,
+                           stage, dt, int(fc), int(lc));
+    }
+}
+
 template <int NM>
 void launch_ansatz_t(const GridArgs &g, int q0, int nqc, hipStream_t s) {
-    const int n = g.NX * g.NY;
-    hipLaunchKernelGGL(ansatz_kernel<NM>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, g, q0, nqc);
+    if constexpr (NM > 15) {
+        launch_ansatz_orbit<NM>(g, q0 / 64, nqc / 64, s);
+    } else {
+        const int n = g.NX * g.NY;
+        hipLaunchKernelGGL(ansatz_kernel<NM>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, g, q0, nqc);
+    }
 }
 
 __global__ void tile_flag_clear_kernel(int *flags, int n) {

@@ -151,6 +151,16 @@ struct OrbitTables {
 };
 int build_orbit_tables(const Tables &t, bool ppn, OrbitTables &o);
 
+// Matrix operands of the flux for moment orders 5 to 8 (mnc_grid.hip), by orbits.
+struct FluxTables {
+    int nt = 0;                    // tiles of 16 orbits (padded with zero weight)
+    std::vector<double> z;         // [nt][sum of ceil(n_c / 4)][64]: moments of 16 orbits, four of a class at a time
+    std::vector<double> p;         // [4 nt][4 classes][64]: moments of four orbits, a class's (at most 16) side by side
+    std::vector<double> dir;       // [16 nt][4]: xi, eta (both > 0), w, 0
+    std::vector<int> idx;          // [4 classes][16]: the moments of a class, -1 past the last
+};
+int build_flux_tables(const Tables &t, FluxTables &f);
+
 // Launchers (mnc_newton.hip).  Return false if (nm, np2, gaunt) has no instance.
 // One call enqueues (no host synchronisation) the prologue if `init`, the
 // lockstep sweep/logic rounds r0..r1-1 with compaction (round r reads list
@@ -260,6 +270,9 @@ struct GridArgs {
     double delta;         // its delta
     // flux_tile 3 on part of the grid: 0 every tile; 1 the tiles whose flag is
     // 0 (no unfinished closure in their stencil region); 2 the flagged ones
+    const double *oz, *op, *odir;   // FluxTables (orders 5 to 8)
+    const int *oidx;
+    int ont;
     const int *tile_flag; // [tiles_x][tiles_y] of kSplitTile x kSplitTile cells
     int tile_mode;
 };
@@ -293,6 +306,7 @@ struct CbArgs {
 int launch_optcb(const CbArgs &a, int max_blocks, int num_cu, hipStream_t s);
 
 void launch_ghost_fill(const GridArgs &g, hipStream_t s);
+// Orders 5 to 8 count nodes in whole tiles of 16 orbits (64 of the ont tiles' 64 ont nodes).
 void launch_ansatz(const GridArgs &g, int q0, int nqc, hipStream_t s);
 // stage: 0 = flux only (writes g.flux), 1 = Euler stage, 2 = Euler + Heun average
 bool launch_flux_euler(const GridArgs &g, int q0, int nqc, int stage, double dt, bool first_chunk,

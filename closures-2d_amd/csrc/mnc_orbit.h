@@ -37,6 +37,17 @@ MNC_HD constexpr int orbit_class(int k) {
         }
 }
 
+// moments of order N in class c
+MNC_HD constexpr int orbit_class_size(int N, int c) {
+    int n = 0;
+    for (int k = 0; k < orbit_nm(N); ++k) n += orbit_class(k) == c;
+    return n;
+}
+
+// The sign of class c at image `img` of an orbit (bit 1: -xi, bit 2: -eta) is
+// negative when they share an odd number of bits.
+MNC_HD constexpr bool orbit_negative(int c, int img) { return ((c & img & 1) ^ ((c & img) >> 1)) != 0; }
+
 // The sums of one solve in the order the kernel forms them, class by class.
 // Direct Hessian: entry e is the product m_a m_b (a >= b within a class; for
 // two classes a runs over the smaller one, so that C m_a is formed least

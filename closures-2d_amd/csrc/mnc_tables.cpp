@@ -337,6 +337,35 @@ int build_g64_tables(int moment_order, int quad_order, G64Tables &m) {
     return MNC_OK;
 }
 
+int build_flux_tables(const Tables &t, FluxTables &f) {
+    if (t.N < 5 || t.N > 8) return MNC_ERR_ARG;
+    const int n = orbit_nm(t.N), half = t.Q / 2, no = half * half;
+    f.nt = (no + 15) / 16;
+    f.idx.assign(64, -1);
+    int size[4] = {0, 0, 0, 0};
+    for (int k = 0; k < n; ++k) {
+        const int c = orbit_class(k);
+        f.idx[c * 16 + size[c]++] = k;
+    }
+    auto node = [&](int o) { return 2 * (o / half) * t.Q + o % half; };     // the orbit's node with xi, eta > 0
+    auto P = [&](int o, int c, int at) {
+        return o < no && at < size[c] ? t.p[size_t(node(o)) * t.np2 + f.idx[c * 16 + at]] : 0.0;
+    };
+    for (int T = 0; T < f.nt; ++T)
+        for (int c = 0; c < 4; ++c)
+            for (int kk = 0; 4 * kk < size[c]; ++kk)
+                for (int l = 0; l < 64; ++l) f.z.push_back(P(16 * T + l % 16, c, 4 * kk + l / 16));
+    for (int s = 0; s < 4 * f.nt; ++s)
+        for (int c = 0; c < 4; ++c)
+            for (int l = 0; l < 64; ++l) f.p.push_back(P(4 * s + l / 16, c, l % 16));
+    for (int o = 0; o < 16 * f.nt; ++o) {
+        const bool in = o < no;
+        const double d[4] = {in ? t.xi[node(o)] : 0.0, in ? t.eta[node(o)] : 0.0, in ? t.w[node(o)] : 0.0, 0.0};
+        f.dir.insert(f.dir.end(), d, d + 4);
+    }
+    return MNC_OK;
+}
+
 namespace {
 
 // Places of the sums (OrbitSums) in the kernel's buffer, for one order and form.

@@ -129,3 +129,30 @@ def test_m8_512_steps_conserve_mass_and_match_oracle_sample():
     print("M8 512^2 sample: same iterations %.3f, max ||du||/||u|| %.2e" % ((itg == ito).mean(), err.max()))
     assert (rg == ro).all() and (itg == ito).mean() >= 0.97
     assert err.max() <= 4e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ic", [1, 2])
+@pytest.mark.parametrize("order,Q,nx,ny", [(5, 6, 5, 7), (6, 10, 17, 3), (7, 12, 33, 16), (8, 32, 4, 41)])
+def test_orbit_flux_matches_fused(order, Q, nx, ny, ic):
+    """The flux of the orders above 4 by orbits on the matrix cores against the
+    fused kernel's direction by direction: cells and orbits that do not fill a
+    tile of 16.  The two differ in the order of at most 4 Q^2 + 45 roundings of
+    terms whose sum may cancel: 1e-12 of the largest flux."""
+    mnc = load_pkg("mnc")
+    print("case orbit flux order=%d Q=%d %dx%d ic=%d" % (order, Q, nx, ny, ic), flush=True)
+    nm = (order + 1) * (order + 2) // 2
+    rng = np.random.default_rng(order * 10 + ic)
+    shape = (nx + 4, ny + 4)
+    a = rng.normal(0.0, 0.3, shape + (nm,)) / (1.0 + np.arange(nm))
+    m = rng.random(shape + (nm,))
+    ctx = mnc.Context(order, Q)
+    ctx.grid_create(nx, ny, 2.0 / nx, 2.0 / ny, -1.0, -1.0, ic, 1.7, m, a, np.ones(shape), np.ones(shape))
+    res = {}
+    for tile in (1, 0):
+        ctx.tune("flux_tile", tile)
+        res[tile] = ctx.flux()
+    ctx.close()
+    err = np.abs(res[0] - res[1]).max() / np.abs(res[1]).max()
+    print("flux rel %.3e" % err)
+    assert np.abs(res[1]).max() > 0.0 and err <= 1e-12
