@@ -48,7 +48,8 @@ struct mnc_ctx {
     // FP64 matrix-core operand tables of the high orders (M8)
     mnc::G64Tables g64;
     bool has_g64 = false;
-    double *d_gz = nullptr, *d_gg = nullptr, *d_gh = nullptr;
+    double *d_gz = nullptr, *d_gh = nullptr, *d_gmap = nullptr;
+    int *d_gidx = nullptr, *d_gpos = nullptr;
     size_t state_cap = 0;
     int state_nm = 0;
     void *d_noalloc = nullptr;       // the library's fixed scratch array on this device (not owned)
@@ -366,10 +367,11 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     a.no = ctx->orb.no;
     a.nop = ctx->orb.nop;
     a.gz = ctx->d_gz;
-    a.gg = ctx->d_gg;
     a.gh = ctx->d_gh;
+    a.gmap = ctx->d_gmap;
+    a.gidx = ctx->d_gidx;
+    a.gpos = ctx->d_gpos;
     a.gnt = ctx->g64.nt;
-    a.gnmm = ctx->g64.nmm;
     mnc::LaunchPlan lp;
     lp.r0 = 0;
     // FP64 cells go straight to the tail kernel unless rounds are asked for.
@@ -475,11 +477,10 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
             // count is read back between batches, so this path is not captured)
             if (!mnc::launch_newton_g64_init(a, t.nm, t.np2, ctx->stream))
                 return ctx_fail(ctx, MNC_ERR_ARG, "no FP64 matrix-core Newton instance for this order");
-            const int blocks = 2 * ctx->num_cu;
             int lin = 0;
             for (int batch = 0;; ++batch) {
                 if (batch > 4000) return ctx_fail(ctx, MNC_ERR_STATE, "closure solve did not finish");
-                mnc::launch_newton_g64_rounds(a, t.nm, t.np2, lin, 4, blocks, ctx->stream);
+                mnc::launch_newton_g64_rounds(a, t.nm, t.np2, lin, 4, ctx->num_cu, ctx->stream);
                 int left = 0;
                 MNC_HIP_CHECK(hipMemcpyAsync(&left, ctl + lin, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
                 MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -711,10 +712,9 @@ int mnc_create(const mnc_setup *setup, mnc_ctx **out) {
         mnc_destroy(ctx);
         return MNC_ERR_HIP;
     }
-    if (!ctx->ppn && t.nm == 45 && mnc::build_g64_tables(setup->moment_order, setup->quad_order, ctx->g64) == MNC_OK &&
-        ctx->g64.kz == 12 && ctx->g64.ngt == 3 && ctx->g64.nht == 10) {   // the instantiated tile counts
-        if (up(&ctx->d_gz, ctx->g64.z) || up(&ctx->d_gg, ctx->g64.g) || up(&ctx->d_gh, ctx->g64.h) ||
-            up(&ctx->d_mgptr, ctx->g64.gptr) || up(&ctx->d_mgk, ctx->g64.gk) || up(&ctx->d_mgv, ctx->g64.gv)) {
+    if (!ctx->ppn && t.nm == 45 && mnc::build_g64_tables(setup->moment_order, setup->quad_order, ctx->g64) == MNC_OK) {
+        if (up(&ctx->d_gz, ctx->g64.z) || up(&ctx->d_gh, ctx->g64.h) || up(&ctx->d_gmap, ctx->g64.map) ||
+            up(&ctx->d_gidx, ctx->g64.idx) || up(&ctx->d_gpos, ctx->g64.pos)) {
             mnc_destroy(ctx);
             return MNC_ERR_HIP;
         }
@@ -742,7 +742,7 @@ void mnc_destroy(mnc_ctx *ctx) {
     for (auto &g : ctx->graphs) drop_graph(g);
     for (auto &ev : ctx->events) { (void)hipEventDestroy(ev.a); (void)hipEventDestroy(ev.b); }
     void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_pT, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
-                    ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gg, ctx->d_gh,
+                    ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gh, ctx->d_gmap, ctx->d_gidx, ctx->d_gpos,
                     ctx->d_ot, ctx->d_opos, ctx->d_ogoff, ctx->d_ogk, ctx->d_ogv,
                     ctx->d_foz, ctx->d_fop, ctx->d_fodir, ctx->d_foidx, ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
                     ctx->d_ctl, ctx->d_stats, ctx->d_std, ctx->d_sti, ctx->d_lists, ctx->d_mom, ctx->d_alpha, ctx->d_old,

@@ -37,51 +37,6 @@ __device__ __forceinline__ void coop_apply_inv(double (*L)[NM], double *x, int l
     }
 }
 
-// coop_apply_inv with x in registers (x_i on lane i): x_j is read with
-// v_readlane instead of a store, a barrier and a load per step; the same
-// operations on each element.
-template <int NM>
-__device__ __forceinline__ void coop_apply_inv_reg(double (*L)[NM], double &x, int lane) {
-    for (int j = 0; j < NM; ++j) {
-        const double xj = readlane_d(x, j) / L[j][j];
-        if (lane == j) x = xj;
-        else if (lane > j && lane < NM) x = fma(-xj, L[lane][j], x);
-    }
-    for (int j = NM - 1; j >= 0; --j) {
-        const double xj = readlane_d(x, j) / L[j][j];
-        if (lane == j) x = xj;
-        else if (lane < j) x = fma(-L[j][lane], xj, x);
-    }
-}
-
-// Cholesky in place on the lower triangle (dpotf2 order); uniform result.
-template <int NM>
-__device__ __forceinline__ bool coop_cholesky(double (*L)[NM], int lane) {
-    bool ok = true;
-    for (int j = 0; j < NM; ++j) {
-        // the inner loops unrolled so that their LDS reads are issued ahead of
-        // the dependent FMA chains (the same FMAs in the same order)
-        double dot = 0.0;
-#pragma unroll 8
-        for (int k = 0; k < j; ++k) dot = fma(L[j][k], L[j][k], dot);
-        double ajj = L[j][j] - dot;
-        ok = ok && (ajj > 0.0);
-        ajj = sqrt(ajj > 0.0 ? ajj : 1.0);
-        double y = 0.0;
-        if (lane > j && lane < NM) {
-            y = L[lane][j];
-#pragma unroll 8
-            for (int k = 0; k < j; ++k) y = fma(-L[j][k], L[lane][k], y);
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane == j) L[j][j] = ajj;
-        const double r = 1.0 / ajj;
-        if (lane > j && lane < NM) L[lane][j] = y * r;
-        __builtin_amdgcn_wave_barrier();
-    }
-    return ok;
-}
-
 // Higham's estimate of ||A^{-1}||_1 (dpocon's role); every lane ends with it.
 template <int NM>
 __device__ __forceinline__ double coop_rcond(double (*L)[NM], double *x, double anorm, int lane) {

@@ -83,9 +83,9 @@ struct NewtonArgs {
     const double *ogv;
     int no, nop;
     // FP64 matrix-core sweep of the high orders (G64Tables, device copies)
-    const double *gz, *gg, *gh;
-    int gnt;              // quadrature tiles of 16 points
-    int gnmm;             // order-2N moments
+    const double *gz, *gh, *gmap;
+    const int *gidx, *gpos;
+    int gnt;              // tiles of 16 orbits
 };
 
 // Control words of a batched solve: [0], [1] counts of lists 0/1 (the
@@ -125,15 +125,16 @@ bool gaunt_pattern_values(int n, const std::vector<int> &gptr, const std::vector
 // Returns MNC_OK, or MNC_ERR_ARG when the order/quadrature has no mixed kernel.
 int build_mix_tables(int moment_order, int quad_order, MixTables &m);
 
-// Operand tables of the FP64 matrix-core sweep (the high orders, where the
-// direct Hessian does not fit a lane): quadrature padded to 16-point tiles
-// (zero weight), moments to kz = ceil(n/4) groups of 4, the sums to g tiles
-// of 16 columns (the last column is w), the order-2N moments to h tiles.
+// Operand tables of the FP64 matrix-core sweep (M8, whose 1035 Hessian sums do
+// not fit a lane), by quadrature orbits and moment classes (mnc_orbit.h).
 struct G64Tables {
-    int nt = 0, kz = 0, ngt = 0, nht = 0, nmm = 0;
-    std::vector<double> z, g, h;
-    std::vector<int> gptr, gk;
-    std::vector<double> gv;
+    int nt = 0;                    // tiles of 16 orbits, padded with zero weight
+    std::vector<double> z;         // [nt][kG64Z][64]: moments of 16 orbits, four of a class at a time
+    std::vector<double> h;         // [nt][4][12][64]: w m of four orbits, the order-2N moments of a class in
+                                   // three columns of 16 (after class 0's, w itself)
+    std::vector<double> map;       // class by class [column of 16 Hessian entries][four moments][64]: the Gaunt map
+    std::vector<int> idx;          // [4][48]: the order-2N moments of a class, -1 past the last
+    std::vector<int> pos;          // [n (n + 1) / 2]: the entries in the map's order, 256 i + j (i >= j)
 };
 int build_g64_tables(int moment_order, int quad_order, G64Tables &m);
 
@@ -202,7 +203,7 @@ bool launch_newton_net_judge(const NewtonArgs &a, int nm, int np2, bool gaunt, i
 // batch; the caller repeats batches until control word `lin` reads zero.
 // Returns false for an order without an instance.
 bool launch_newton_g64_init(const NewtonArgs &a, int nm, int np2, hipStream_t s);
-bool launch_newton_g64_rounds(const NewtonArgs &a, int nm, int np2, int &lin, int rounds, int blocks, hipStream_t s);
+bool launch_newton_g64_rounds(const NewtonArgs &a, int nm, int np2, int &lin, int rounds, int num_cu, hipStream_t s);
 // Scratch of the no-allocation entry point (mnc_opt_batch_noalloc): a
 // file-scope device array in mnc_newton.hip with the Newton state, lists and
 // control words of up to kNoAllocCells cells of moment order <= 4.

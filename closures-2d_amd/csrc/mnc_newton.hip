@@ -25,6 +25,7 @@
 
 #include "mnc_internal.h"
 #include "mnc_coop_la.h"
+#include "mnc_orbit.h"
 #include "mnc_gaunt_pattern.h"
 #include "mnc_newton_state.h"
 
@@ -1552,99 +1553,201 @@ __global__ __launch_bounds__(64 * kMixWaves) void sweep_mix_kernel(NewtonArgs A,
     }
 }
 
-// ---- FP64 matrix-core path for the high orders (M8: n = 45, nq = 1024) -------
+// ---- FP64 matrix-core path for M8 (n = 45) -------------------------------------
 //
-// The direct Hessian of 45 moments (1035 sums) does not fit a lane, so the
-// sweep runs on the matrix cores with the lane scheme of the mixed sweep, all in
-// FP64, sixteen cells per wave:
-//   z = alpha.m        KZ products per 16-point tile
-//   G = sums w e m_i   NGT column tiles; the last column is sum w e (f)
-//   Hm = sums w e p2N  NHT column tiles: the order-2N moments, from which the
-//                      logic forms H through the Gaunt map
-// f, g and H are then the reference's full evaluation (fobj.cpp:266-287) to
-// rounding: f = sum w e - alpha.u, g_i = sum w e m_i - u_i, and H differs from
-// the direct sum only by the Gaunt least-squares fit (~1e-14).  The operand
-// tables (build_g64_tables, 2 MB at M8/Q32) are read from global memory.
-template <int NM, int NP2, int KZ, int NGT, int NHT>
-__global__ __launch_bounds__(256) void sweep_g64_kernel(NewtonArgs A, int lin) {
-    using St = Store<NM, NP2>;
-    static_assert(16 * NGT - 1 >= NM, "the last sum column holds sum w e");
-    static_assert(16 * NHT <= St::nacc, "order-2N moments exceed the store");
+// The direct Hessian of 45 moments (1035 sums) does not fit a lane, so the sweep
+// runs on the matrix cores in FP64, sixteen cells a wave, by the quadrature's
+// orbits (mnc_orbit.h): per class c of moments
+//   z_c = alpha.m over the class; the four exponents of an orbit are signed sums
+//   C_c = signed sum of the four e
+//   M_c = sum over orbits of C_c w p_2N, the order-2N moments of the class (the
+//         first of them are sum w e m; after class 0's comes sum w e)
+//   H   = the Gaunt map of M, H_ij from the class of m_i m_j alone
+// which is 61 products per 64 nodes where a node by node form takes 256.  f, g and H
+// are the reference's full evaluation (fobj.cpp:266-287) to rounding:
+// f = sum w e - alpha.u, g_i = sum w e m_i - u_i, and H differs from the direct
+// sum only by the Gaunt least-squares fit (~1e-14).
+struct G64 {
+    static constexpr int N = 8, n = orbit_nm(N), nh = n * (n + 1) / 2;
+    static constexpr int size(int c) { return orbit_class_size(N, c); }
+    static constexpr int size2(int c) { return orbit_class_size(2 * N, c); }
+    static constexpr int kz(int c) { return (size(c) + 3) / 4; }
+    static constexpr int z0(int c) { return c == 0 ? 0 : z0(c - 1) + kz(c - 1); }
+    static constexpr int kz2(int c) { return (size2(c) + 3) / 4; }
+    static constexpr int entries(int c) {     // pairs i >= j whose product is in class c
+        int e = 0;
+        for (int p = 0; p < 4; ++p) e += c == 0 ? size(p) * (size(p) + 1) / 2 : ((p ^ c) > p ? size(p) * size(p ^ c) : 0);
+        return e;
+    }
+    static constexpr int e0(int c) { return c == 0 ? 0 : e0(c - 1) + entries(c - 1); }
+    static constexpr int cols(int c) { return (entries(c) + 15) / 16; }
+    static constexpr int m0(int c) { return c == 0 ? 0 : m0(c - 1) + cols(c - 1) * kz2(c - 1) * 64; }
+    static_assert(orbit_class_size(16, 0) < 48, "sum w e after class 0's moments");
+};
+template <int I> struct ClassC { static constexpr int value = I; };
+template <class T>
+__device__ __forceinline__ void each_class(T &&f) {
+    f(ClassC<0>{});
+    f(ClassC<1>{});
+    f(ClassC<2>{});
+    f(ClassC<3>{});
+}
+
+// A block takes sixteen cells, its four waves a quarter of the orbit tiles each;
+// then wave c adds up class c's sums and forms the class's Hessian entries.  With
+// a wave alone on sixteen cells and every node (597 us at 10,000 cells and 1,024
+// nodes) the chip held 625 waves, each waiting on its operand loads; by orbits and
+// quarters 110 us, H included.
+__global__ __launch_bounds__(256, 2) void sweep_g64_kernel(NewtonArgs A, int lin) {
+    using St = Store<G64::n, G64::n>;
+    constexpr int nh = G64::nh;
+    static_assert(nh <= St::nacc, "the Hessian entries exceed the store");
+    __shared__ double part[3][12][64];
+    __shared__ double mom[4][16][49];
     if (blockIdx.x == 0 && threadIdx.x == 0) A.ctl[lin ^ 1] = 0;
     const int count = A.ctl[lin];
     const int ntiles = (count + 15) >> 4;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ci = lane & 15, g = lane >> 4;
     const St S{A.st_d, A.st_i, A.cap};
-    const int nt = A.gnt, nmm = A.gnmm;
-    for (int tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
+    double *H = A.st_d + size_t(St::F_ACC) * A.cap;      // [slot][nh] in the accumulators' place
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const int slot = tile * 16 + ci;
-        const int c = slot < count ? A.lists[size_t(lin) * A.cap + slot] : -1;
+        const int c16 = slot < count ? A.lists[size_t(lin) * A.cap + slot] : -1;
+        constexpr int KZ = G64::z0(4);
         double ab[KZ];
+        mf64x4 acc[4][3];
+        each_class([&](auto C) {
+            constexpr int c = decltype(C)::value, kz = G64::kz(c), z0 = G64::z0(c), nc = G64::size(c);
 #pragma unroll
-        for (int kk = 0; kk < KZ; ++kk) {
-            const int k = 4 * kk + g;
-            ab[kk] = (c >= 0 && k < NM) ? S.d(St::F_AL + k, c) : 0.0;
-        }
-        mf64x4 gacc[NGT], hacc[NHT];
+            for (int kk = 0; kk < kz; ++kk) {
+                const int e = 4 * kk + g;
+                ab[z0 + kk] = (c16 >= 0 && e < nc) ? S.d(St::F_AL + A.gidx[c * 48 + e], c16) : 0.0;
+            }
 #pragma unroll
-        for (int n = 0; n < NGT; ++n) gacc[n] = mf64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int n = 0; n < NHT; ++n) hacc[n] = mf64x4{0.0, 0.0, 0.0, 0.0};
-        for (int T = 0; T < nt; ++T) {
+            for (int m = 0; m < 3; ++m) acc[c][m] = mf64x4{0.0, 0.0, 0.0, 0.0};
+        });
+        for (int T = wave; T < A.gnt; T += 4) {
             const double *zt = A.gz + size_t(T) * KZ * 64 + lane;
-            const double *gt = A.gg + size_t(T) * 4 * NGT * 64 + lane;
-            const double *ht = A.gh + size_t(T) * 4 * NHT * 64 + lane;
-            mf64x4 z = {0.0, 0.0, 0.0, 0.0};
+            const double *ht = A.gh + size_t(T) * 48 * 64 + lane;
+            mf64x4 z[4];
+            each_class([&](auto C) {
+                constexpr int c = decltype(C)::value, kz = G64::kz(c), z0 = G64::z0(c);
+                z[c] = mf64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int kk = 0; kk < KZ; ++kk) z = __builtin_amdgcn_mfma_f64_16x16x4f64(zt[kk * 64], ab[kk], z, 0, 0, 0);
+                for (int kk = 0; kk < kz; ++kk)
+                    z[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(zt[(z0 + kk) * 64], ab[z0 + kk], z[c], 0, 0, 0);
+            });
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const double e = exp(z[r]);
+                const double ep = z[0][r] + z[1][r], em = z[0][r] - z[1][r], op = z[2][r] + z[3][r], om = z[2][r] - z[3][r];
+                const double e0 = exp(ep + op), e1 = exp(em + om), e2 = exp(ep - op), e3 = exp(em - om);
+                const double s01 = e0 + e1, d01 = e0 - e1, s23 = e2 + e3, d23 = e2 - e3;
+                const double cc[4] = {s01 + s23, d01 + d23, s01 - s23, d01 - d23};
 #pragma unroll
-                for (int n = 0; n < NGT; ++n)
-                    gacc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(e, gt[(r * NGT + n) * 64], gacc[n], 0, 0, 0);
+                for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int n = 0; n < NHT; ++n)
-                    hacc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(e, ht[(r * NHT + n) * 64], hacc[n], 0, 0, 0);
+                    for (int m = 0; m < 3; ++m)
+                        acc[c][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(cc[c], ht[(r * 12 + 3 * c + m) * 64], acc[c][m], 0, 0, 0);
             }
         }
-        const int j = lane & 15;
+        // element r of lane l: cell mfma_f64_row(r, l / 16), column l % 16
+        each_class([&](auto C) {
+            constexpr int c = decltype(C)::value, nc = G64::size(c), nc2 = G64::size2(c);
+            __syncthreads();
+            if (wave != c) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int cg = __shfl(c, mfma_f64_row(r, g));
-            if (cg < 0) continue;
+                for (int m = 0; m < 3; ++m)
 #pragma unroll
-            for (int n = 0; n < NGT; ++n) {
-                const int col = 16 * n + j;
-                if (col < NM) S.d(St::F_GS + col, cg) = gacc[n][r];
-                if (col == 16 * NGT - 1) S.d(St::F_SF, cg) = gacc[n][r];
+                    for (int r = 0; r < 4; ++r) part[wave > c ? wave - 1 : wave][4 * m + r][lane] = acc[c][m][r];
             }
+            __syncthreads();
+            if (wave == c) {
 #pragma unroll
-            for (int n = 0; n < NHT; ++n) {
-                const int col = 16 * n + j;
-                if (col < nmm) S.d(St::F_ACC + col, cg) = hacc[n][r];
+                for (int m = 0; m < 3; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const double v = ((acc[c][m][r] + part[0][4 * m + r][lane]) + part[1][4 * m + r][lane]) +
+                                         part[2][4 * m + r][lane];
+                        const int row = mfma_f64_row(r, g), col = 16 * m + ci;
+                        mom[c][row][col] = v;
+                        const int cell = __shfl(c16, row);
+                        if (cell >= 0) {
+                            if (col < nc) S.d(St::F_GS + A.gidx[c * 48 + col], cell) = v;
+                            if (c == 0 && col == nc2) S.d(St::F_SF, cell) = v;
+                        }
+                    }
             }
-        }
+        });
+        __builtin_amdgcn_wave_barrier();
+        each_class([&](auto C) {
+            constexpr int c = decltype(C)::value, kz2 = G64::kz2(c), cols = G64::cols(c), ne = G64::entries(c),
+                          nc2 = G64::size2(c), m0 = G64::m0(c), e0 = G64::e0(c);
+            if (wave != c) return;
+            double a[kz2];
+#pragma unroll
+            for (int kk = 0; kk < kz2; ++kk) {
+                const int e = 4 * kk + g;
+                a[kk] = e < nc2 ? mom[c][ci][e] : 0.0;
+            }
+            const double *map = A.gmap + m0 + lane;
+#pragma unroll 2
+            for (int col = 0; col < cols; ++col) {
+                mf64x4 h = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int kk = 0; kk < kz2; ++kk)
+                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kk], map[(col * kz2 + kk) * 64], h, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int to = tile * 16 + mfma_f64_row(r, g);
+                    if (to < count && 16 * col + ci < ne) H[size_t(to) * nh + e0 + 16 * col + ci] = h[r];
+                }
+            }
+        });
     }
 }
 
-template <int NM, int NACC>
+constexpr int kG64Stride = G64::n + 1;
 struct G64Shared {
-    double L[NM][NM];   // H, then its Cholesky factor (lower)
-    double x[NM], gvec[NM], al[NM];
-    double mom[NACC];   // the sweep's order-2N moments of the cell
+    double L[kG64Stride * kG64Stride];     // H, then the factor's columns, then (for the condition estimate) its rows
+    double x[G64::n], gvec[G64::n], al[G64::n];
 };
 
+template <int J, int NM>
+__device__ __forceinline__ void chol_column(double (&a)[NM], double &rd, double *L, bool &ok, int lane) {
+    // the lane as the compiler cannot see through: its 45 comparisons would be
+    // kept in scalar registers, which spill
+    __asm__ volatile("" : "+v"(lane));
+    const double piv = readlane_d(a[J], J);
+    ok = ok && (piv > 0.0);
+    const double s = sqrt(piv > 0.0 ? piv : 1.0), r = 1.0 / s;
+    a[J] = lane == J ? s : a[J] * r;
+    rd = lane == J ? r : rd;
+    double *col = L + J * kG64Stride;
+    // no branch (the lanes past the gradient's hold copies of it): the compiler
+    // would put off the updates into the blocks after it, and keep 990 factors
+    col[min(lane, NM)] = a[J];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = J + 1; k < NM; ++k) a[k] = fma(-a[J], col[k], a[k]);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J + 1 < NM) chol_column<J + 1, NM>(a, rd, L, ok, lane);
+}
+
 // One step of optScaled's logic per cell after sweep_g64_kernel, one wave per
-// cell (lane i owns row i of H and of its factor; the iterate in LDS).  The
+// cell.  Lane i holds row i of H in registers, lane n the gradient, and the factor
+// goes column by column: the pivot by a lane read, the column to LDS, and every
+// lane updates its row from LDS broadcasts, so that the gradient's lane ends with
+// L^-1 g.  Bound by the 45 dependent columns and 990 broadcast FMAs; with the
+// rows in LDS, H formed there term by term from the Gaunt map in HBM and
+// dot products in a chain this took 438 us at 10,000 cells, now 193.  The
 // steps are those of cell_logic (opt.cpp:209-318, linesearch.cpp:38-98);
 // cells needing another sweep go onto list lin^1.
-template <int NM, int NP2>
-__global__ __launch_bounds__(64) void logic_g64_kernel(NewtonArgs A, int lin) {
-    using St = Store<NM, NP2>;
-    constexpr int NK = gp_nm(2 * order_of(NM));    // the order-2N moments (153 at n = 45)
-    __shared__ G64Shared<NM, NK> sh;
+__global__ __launch_bounds__(64, 2) void logic_g64_kernel(NewtonArgs A, int lin) {
+    constexpr int NM = G64::n;
+    using St = Store<NM, NM>;
+    __shared__ __attribute__((aligned(16))) G64Shared sh;
+    const double *H = A.st_d + size_t(St::F_ACC) * A.cap;
     const St S{A.st_d, A.st_i, A.cap};
     const int lane = threadIdx.x;
     const int count = A.ctl[lin];
@@ -1684,26 +1787,40 @@ __global__ __launch_bounds__(64) void logic_g64_kernel(NewtonArgs A, int lin) {
         }
         if (newton) {
             ++iter; ++total;                                        // opt.cpp:212-213
-            // the cell's moments into LDS first: each Gaunt term then reads its
-            // moment from LDS, not through a load that waits on the term's index
-            for (int k = lane; k < NK; k += 64) sh.mom[k] = S.d(St::F_ACC + k, c);
-            __builtin_amdgcn_wave_barrier();
-            double rs = 0.0, gi = 0.0, dg = 0.0;
-            if (lane < NM) {                                        // row `lane` of H (Gaunt map)
-                for (int jj = 0; jj < NM; ++jj) {
-                    const int pr = (lane < jj) ? lane * NM + jj : jj * NM + lane;
-                    double hij = 0.0;
-                    // the same sum in the same order; four terms' loads in flight
-#pragma unroll 4
-                    for (int cc = A.mgptr[pr]; cc < A.mgptr[pr + 1]; ++cc)
-                        hij = fma(A.mgv[cc], sh.mom[A.mgk[cc]], hij);
-                    sh.L[lane][jj] = hij;
-                    rs += fabs(hij);
-                    if (jj == lane) dg = hij;
+            {                                                       // H: both triangles into LDS
+                constexpr int per = (G64::nh + 63) / 64;
+                double h[per];
+                int ij[per];
+#pragma unroll
+                for (int m = 0; m < per; ++m) {
+                    const int e = lane + 64 * m;
+                    h[m] = e < G64::nh ? H[size_t(slot) * G64::nh + e] : 0.0;
+                    ij[m] = e < G64::nh ? A.gpos[e] : 0;
                 }
+#pragma unroll
+                for (int m = 0; m < per; ++m)
+                    if (lane + 64 * m < G64::nh) {
+                        const int i = ij[m] >> 8, jj = ij[m] & 255;
+                        sh.L[i * NM + jj] = h[m];
+                        sh.L[jj * NM + i] = h[m];
+                    }
+            }
+            double gi = 0.0;
+            if (lane < NM) {
                 gi = S.d(St::F_GS + lane, c) - ul;
                 sh.gvec[lane] = gi;
             }
+            __builtin_amdgcn_wave_barrier();
+            double a[NM], rs = 0.0, dg = 0.0;
+            const double *row = lane < NM ? sh.L + lane * NM : sh.gvec;   // lane n: the gradient
+#pragma unroll
+            for (int jj = 0; jj < NM; ++jj) {
+                a[jj] = row[jj];
+                rs += fabs(a[jj]);
+            }
+            if (lane < NM) dg = sh.L[lane * NM + lane];
+            else rs = 0.0;
+            __builtin_amdgcn_wave_barrier();
             const double au = wave_sum(lane < NM ? sh.al[lane] * ul : 0.0);
             const double aus = wave_sum(lane < NM ? fabs(sh.al[lane] * ul) : 0.0);
             const double fcur = S.d(St::F_SF, c) - au;
@@ -1712,15 +1829,41 @@ __global__ __launch_bounds__(64) void logic_g64_kernel(NewtonArgs A, int lin) {
             const double anorm = wave_max(rs);                     // utils.cpp:36-52
             const double gersh = wave_min(lane < NM ? 2.0 * dg - rs : DBL_MAX);
             __builtin_amdgcn_wave_barrier();
-            const bool chol_ok = coop_cholesky<NM>(sh.L, lane);
+            bool chol_ok = true;
+            double rd = 0.0;
+            chol_column<0, NM>(a, rd, sh.L, chol_ok, lane);
+            // L^-T (L^-1 g): lane i takes column i below the diagonal
+            double xr = 0.0;
+            {
+                const int at = lane < NM ? lane * kG64Stride : 0;
+                xr = lane < NM ? sh.L[at + NM] : 0.0;
+                double b[NM];
+#pragma unroll
+                for (int i = 1; i < NM; ++i) b[i] = sh.L[at + i];
+#pragma unroll
+                for (int i = NM - 1; i > 0; --i) {
+                    int ln = lane;
+                    __asm__ volatile("" : "+v"(ln));
+                    const double xi = readlane_d(xr * rd, i);
+                    xr = ln < i ? fma(-xi, b[i], xr) : xr;
+                }
+                xr = xr * rd;
+            }
             double condest = 0.0;
-            if (chol_ok && !cond_proven_below(anorm, gersh, NM, A.cond_h_max))
-                condest = 1.0 / coop_rcond<NM>(sh.L, sh.x, anorm, lane);
+            if (chol_ok && !cond_proven_below(anorm, gersh, NM, A.cond_h_max)) {
+                double (*L)[NM] = (double (*)[NM])sh.L;             // the factor by rows
+#pragma unroll
+                for (int jj = 0; jj < NM; ++jj) a[jj] = lane <= NM ? sh.L[jj * kG64Stride + lane] : 0.0;
+                __builtin_amdgcn_wave_barrier();
+                if (lane < NM)
+#pragma unroll
+                    for (int jj = 0; jj < NM; ++jj) L[lane][jj] = a[jj];
+                __builtin_amdgcn_wave_barrier();
+                condest = 1.0 / coop_rcond<NM>(L, sh.x, anorm, lane);
+            }
             if (iter >= maxit || !chol_ok || t == 0.0 || condest > A.cond_h_max) {
                 do_reg = true;                                      // opt.cpp:244
             } else {
-                double xr = lane < NM ? sh.gvec[lane] : 0.0;
-                coop_apply_inv_reg<NM>(sh.L, xr, lane);             // dpotrs (:278-282)
                 if (lane < NM) sh.x[lane] = xr;
                 __builtin_amdgcn_wave_barrier();
                 bool stop = err <= S.d(St::F_RTOL, c);
@@ -1951,13 +2094,14 @@ bool launch_newton_g64_init(const NewtonArgs &a, int nm, int np2, hipStream_t s)
     return false;
 }
 
-bool launch_newton_g64_rounds(const NewtonArgs &a, int nm, int np2, int &lin, int rounds, int blocks, hipStream_t s) {
+bool launch_newton_g64_rounds(const NewtonArgs &a, int nm, int np2, int &lin, int rounds, int num_cu, hipStream_t s) {
     if (!(nm == 45 && np2 == 45)) return false;
-    constexpr int KZ = 12, NGT = 3, NHT = 10;   // 48 moment rows, 46 sum columns, 153 order-16 moments
-    if (a.gnmm > 16 * NHT || a.gnmm != gp_nm(2 * order_of(45))) return false;   // logic_g64's LDS moments
+    // sixteen cells a sweep block, two blocks resident per CU; a cell a logic
+    // block, nine resident (LDS); cells beyond loop
+    const int sweep = std::min((a.ncells + 15) / 16, 2 * num_cu), logic = std::min(a.ncells, 9 * num_cu);
     for (int r = 0; r < rounds; ++r) {
-        hipLaunchKernelGGL((sweep_g64_kernel<45, 45, KZ, NGT, NHT>), dim3(blocks), dim3(256), 0, s, a, lin);
-        hipLaunchKernelGGL((logic_g64_kernel<45, 45>), dim3(4 * blocks), dim3(64), 0, s, a, lin);
+        hipLaunchKernelGGL(sweep_g64_kernel, dim3(sweep), dim3(256), 0, s, a, lin);
+        hipLaunchKernelGGL(logic_g64_kernel, dim3(logic), dim3(64), 0, s, a, lin);
         lin ^= 1;
     }
     return true;

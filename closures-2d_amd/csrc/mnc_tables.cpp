@@ -297,43 +297,60 @@ bool gaunt_pattern_values(int n, const std::vector<int> &gptr, const std::vector
 //   h[T][r][nt][l]  = w_q p2N[q][16nt + l%16]                            (B operand)
 // with q = 16T + R(r, l/16).
 int build_g64_tables(int moment_order, int quad_order, G64Tables &m) {
+    constexpr int N = 8, n = orbit_nm(N), n2 = orbit_nm(2 * N);
     Tables t;
     int st = build_tables(moment_order, quad_order, 1, t);
     if (st != MNC_OK) return st;
-    const int nm = t.nm, nq = t.nq, np2 = t.np2;
-    m.nt = (nq + 15) / 16;
-    m.kz = (nm + 3) / 4;
-    m.ngt = (nm + 1 + 15) / 16;
-    m.nht = (t.nmm + 15) / 16;
-    m.nmm = t.nmm;
-    auto P = [&](int q, int k) { return (q < nq && k < np2) ? t.p[size_t(q) * np2 + k] : 0.0; };
-    auto W = [&](int q) { return q < nq ? t.w[q] : 0.0; };
-    m.z.assign(size_t(m.nt) * m.kz * 64, 0.0);
-    m.g.assign(size_t(m.nt) * 4 * m.ngt * 64, 0.0);
-    m.h.assign(size_t(m.nt) * 4 * m.nht * 64, 0.0);
-    for (int T = 0; T < m.nt; ++T) {
-        for (int kk = 0; kk < m.kz; ++kk)
-            for (int l = 0; l < 64; ++l) {
-                const int k = 4 * kk + l / 16;
-                m.z[(size_t(T) * m.kz + kk) * 64 + l] = k < nm ? P(16 * T + l % 16, k) : 0.0;
-            }
-        for (int r = 0; r < 4; ++r)
-            for (int l = 0; l < 64; ++l) {
-                const int q = 16 * T + mfma_f64_row(r, l / 16);
-                for (int nt = 0; nt < m.ngt; ++nt) {
-                    const int j = 16 * nt + l % 16;
-                    m.g[((size_t(T) * 4 + r) * m.ngt + nt) * 64 + l] =
-                        j < nm ? W(q) * P(q, j) : (j == 16 * m.ngt - 1 ? W(q) : 0.0);
-                }
-                for (int nt = 0; nt < m.nht; ++nt) {
-                    const int col = 16 * nt + l % 16;
-                    m.h[((size_t(T) * 4 + r) * m.nht + nt) * 64 + l] = col < t.nmm ? W(q) * P(q, col) : 0.0;
-                }
-            }
+    if (t.N != N || t.nmm != n2) return MNC_ERR_ARG;
+    const int half = t.Q / 2, no = half * half;
+    m.nt = (no + 15) / 16;
+    m.idx.assign(4 * 48, -1);
+    int size[4] = {0, 0, 0, 0}, at[n2], cls[n2];
+    for (int k = 0; k < n2; ++k) {     // ascending: a class's order-N moments come first
+        cls[k] = orbit_class(k);
+        at[k] = size[cls[k]]++;
+        m.idx[cls[k] * 48 + at[k]] = k;
     }
-    m.gptr = t.gptr;
-    m.gk = t.gk;
-    m.gv = t.gv;
+    auto P = [&](int o, int k) { return t.p[size_t(2 * (o / half) * t.Q + o % half) * t.np2 + k]; };
+    auto W = [&](int o) { return t.w[size_t(2 * (o / half) * t.Q + o % half)]; };
+    for (int T = 0; T < m.nt; ++T) {
+        for (int c = 0; c < 4; ++c)
+            for (int kk = 0; 4 * kk < orbit_class_size(N, c); ++kk)
+                for (int l = 0; l < 64; ++l) {
+                    const int o = 16 * T + l % 16, e = 4 * kk + l / 16;
+                    m.z.push_back(o < no && e < orbit_class_size(N, c) ? P(o, m.idx[c * 48 + e]) : 0.0);
+                }
+        for (int r = 0; r < 4; ++r)
+            for (int c = 0; c < 4; ++c)
+                for (int col = 0; col < 48; col += 16)
+                    for (int l = 0; l < 64; ++l) {
+                        const int o = 16 * T + mfma_f64_row(r, l / 16), k = m.idx[c * 48 + col + l % 16];
+                        const bool w_itself = c == 0 && col + l % 16 == size[0];
+                        m.h.push_back(o >= no ? 0.0 : w_itself ? W(o) : k >= 0 ? W(o) * P(o, k) : 0.0);
+                    }
+    }
+    for (int c = 0; c < 4; ++c) {
+        std::vector<int> pairs;        // H_ij sums moments of the class of m_i m_j only
+        for (int i = 0; i < n; ++i)
+            for (int j = 0; j <= i; ++j)
+                if ((cls[i] ^ cls[j]) == c) pairs.push_back(256 * i + j);
+        m.pos.insert(m.pos.end(), pairs.begin(), pairs.end());
+        const int kz = (size[c] + 3) / 4;
+        for (size_t col = 0; col < pairs.size(); col += 16) {
+            std::vector<double> block(size_t(kz) * 64, 0.0);
+            for (size_t e = 0; e < 16 && col + e < pairs.size(); ++e) {
+                const int i = pairs[col + e] / 256, j = pairs[col + e] % 256;
+                for (int g = t.gptr[i * n + j]; g < t.gptr[i * n + j + 1]; ++g) {
+                    const int k = t.gk[g];
+                    // Other classes' moments are orthogonal to the product on any of
+                    // these quadratures.  From Q = 18 on the fit gives them nothing;
+                    // below, columns that vanish on the nodes get noise.
+                    if (cls[k] == c) block[size_t(at[k] / 4) * 64 + 16 * (at[k] % 4) + e] += t.gv[g];
+                }
+            }
+            m.map.insert(m.map.end(), block.begin(), block.end());
+        }
+    }
     return MNC_OK;
 }
 

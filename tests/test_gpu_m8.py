@@ -156,3 +156,34 @@ def test_orbit_flux_matches_fused(order, Q, nx, ny, ic):
     err = np.abs(res[0] - res[1]).max() / np.abs(res[1]).max()
     print("flux rel %.3e" % err)
     assert np.abs(res[1]).max() > 0.0 and err <= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Q,n", [(10, 1), (12, 15), (18, 17), (26, 1), (32, 33)])
+def test_m8_closures_over_tile_remainders(Q, n):
+    """Cells that do not fill a tile of 16 and orbit tiles that do not fill a
+    block's four waves (Q = 18: 81 orbits, six tiles).  tol 1e-8 bounds what two
+    converged solves' multipliers reproduce of u by: 4e-8 as above.  With fewer
+    nodes than order-16 moments there is no Gaunt map and the solve is refused."""
+    mnc = load_pkg("mnc")
+    print("case m8 remainders Q=%d n=%d" % (Q, n), flush=True)
+    tab = oracle().Tables(8, Q, False)
+    u, astar = _m8_inputs(tab, n, 100 + Q)
+    a0 = np.zeros_like(u)
+    a0[:, 0] = 2.0 * math.sqrt(math.pi) * (math.log(0.5 / math.sqrt(math.pi)) + np.log(u[:, 0]))
+    ctx = mnc.Context(8, Q)
+    if Q * Q < 153:
+        with pytest.raises(mnc.MncError) as e:
+            ctx.opt_batch_host(u, a0, mnc.options(tol=1e-8, line_search=mnc.LS_ROBUST))
+        assert e.value.code == mnc.ERR_ARG
+        ctx.close()
+        return
+    st, ug, ag, itg, rg, _ = ctx.opt_batch_host(u, a0, mnc.options(tol=1e-8, line_search=mnc.LS_ROBUST))
+    ctx.close()
+    sto, uo, ao, ito, ro, _ = tab.opt_batch(u, a0, max_iter=100, tol=1e-8, cond_h_max=1e10, line_search=1, nthreads=4)
+    assert st == 0 and sto == 0
+    rs = rg == ro
+    assert rs.mean() >= 0.97
+    un = np.linalg.norm(ug[rs] - uo[rs], axis=1) / np.linalg.norm(uo[rs], axis=1)
+    print("max ||du||/||u|| %.3e, same iterations %.2f" % (un.max(), (itg == ito).mean()))
+    assert un.max() <= 4e-8
