@@ -20,7 +20,11 @@
 //   direction L^-T (L^-1 g) and the condition bounds broadcast one lane's
 //   value to its row (DPP row_newbcast), so the four cells' dependent steps
 //   run side by side and nothing goes through LDS.
-// What bounds it: FP64 issue.  The measured times stand at the launch rule
+// What bounds it: FP64 issue and the dependent steps of the algebra.  At 256
+// registers and two waves per SIMD the M4 forms must not spill: with the cell's
+// state in registers, the factor's 105 broadcasts kept for the inverse and a branch
+// around each load of H, scratch traffic was three quarters of the time (150,001
+// closures 7.2 ms, now 3.1).  The measured times stand at the launch rule
 // (launch_rows).
 #include <cfloat>
 
@@ -200,11 +204,13 @@ __device__ __forceinline__ double rows_rcond(const double (&row)[NM], const doub
 constexpr int kRowWaves = 4;      // waves per block
 constexpr int kRowTiles = 4;      // orbit tiles whose class sums are kept in registers (four cells per wave)
 
-// Counts of one lane (lane 0 of each cell's row counts).
-struct RowStats {
-    int max_iter = 0, err = 0, sum = 0, n = 0, trials = 0, hist[5] = {0, 0, 0, 0, 0}, cells = 0, titer = 0, fallback = 0,
-        iso = 0, prev = 0;
-};
+// What a cell carries from one evaluation to the next, in LDS beside the wave's
+// sums: in registers it would stand beside the sums and the factor, and spill.
+enum : int { V_UL, V_AOLD, V_DL, kRowVectors };                  // an element per lane
+enum : int { S_U0, S_ASCALE, S_RTOL, S_FCUR, S_GD, S_FSCALE, S_MAXF, S_DELTA, kRowScalars };   // one per row
+// Counts of a row (its lane 0 counts).
+enum : int { R_MAX_ITER, R_ERR, R_SUM, R_N, R_TRIALS, R_HIST, R_CELLS = R_HIST + 5, R_TITER, R_FALLBACK, R_ISO, R_PREV,
+             kRowCounts };
 
 template <int N, bool GAUNT, bool PPN, bool WIDE>
 struct RowDims {
@@ -212,7 +218,8 @@ struct RowDims {
     static constexpr int NS = OrbitSums<N, GAUNT>::count;
     static constexpr int RAW = NS + 1 + (PPN ? NM : 0);           // sums per cell in LDS
     static constexpr int RAWP = RAW | 1;
-    static constexpr int LANE_WORDS = 4 * RAWP + 64;              // per wave: the sums, the iterates
+    // per wave: the sums, the iterates, the cells' state, the counts
+    static constexpr int LANE_WORDS = 4 * RAWP + 64 + 64 * kRowVectors + 4 * kRowScalars + 2 * kRowCounts;
     static constexpr int TB = WIDE ? 1 : kRowTiles;
 };
 
@@ -221,7 +228,7 @@ struct RowDims {
 // kernels without knowing the lists' counts; with at most one cell per wave
 // the WIDE one runs and the other leaves at once, else the other way round.
 template <int N, bool GAUNT, bool PPN, bool WIDE, bool TABLED>
-__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(WIDE ? 1 : 2)))
+__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
     using Dm = RowDims<N, GAUNT, PPN, WIDE>;
     constexpr int NM = Dm::NM, NP2 = Dm::NP2, NS = Dm::NS, RAWP = Dm::RAWP, TB = Dm::TB;
@@ -232,7 +239,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
     extern __shared__ double lds[];
     __shared__ int red[kRowWaves][16];
     int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // its LDS addresses in scalar registers
     const int count = fresh ? A.ncells : A.ctl[cw(lin)];
     const int total_cells = count + (fresh ? 0 : A.ctl[cw(lin2)]);
     const int waves = gridDim.x * kRowWaves;
@@ -244,15 +251,15 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
         for (int i = threadIdx.x; i < table; i += blockDim.x) lds[i] = A.ot[i];
     }
     double *raw = lds + table + wave * Dm::LANE_WORDS, *als = raw + 4 * RAWP;
+    double *vectors = als + 64, *scalars = vectors + 64 * kRowVectors;
+    int *counts = reinterpret_cast<int *>(scalars + 4 * kRowScalars);
+    for (int i = lane; i < 64 * kRowVectors + 4 * kRowScalars + 2 * kRowCounts; i += 64) vectors[i] = 0.0;
     __syncthreads();
     const double p0 = A.p[0];
     const int per_wave = WIDE ? 1 : min(4, max(1, (total_cells + waves - 1) / waves));
-    RowStats st;
-    // per-cell state: vectors one element per lane, scalars on every lane of the row
+    // per-cell state beside the one in LDS: the iterate one element per lane, scalars on every lane of the row
     int c = (!WIDE && (lane >> 4) >= per_wave) ? -2 : -1;              // -1 wants a cell, -2 has none left to take
-    double al = 0.0, ul = 0.0, aold = 0.0, dl = 0.0;
-    double u0 = 1.0, ascale = 0.0, t = 1.0, rtol = 0.0, fcur_s = 0.0, gd_s = 0.0, fscale_s = 0.0, maxf_s = 0.0;
-    double delta = 0.0;
+    double al = 0.0, t = 1.0;
     int mode = ST_NEWTON, iter = 0, total = 0, reg = 0, maxit = 0, warm = 2;
     for (;;) {
         // the lane's masks and offsets are formed anew each pass: kept across
@@ -264,6 +271,8 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
         const bool owner = WIDE ? rowc == 0 : true;             // WIDE: the four rows repeat one cell
         const bool in = r < NM;
         double *myraw = raw + (WIDE ? 0 : rowc * RAWP);
+        double *vl = vectors + lane, *sr = scalars + rowc;
+        int *st = counts + rowc * kRowCounts;
         // ---- cells for the rows without one ----
         const unsigned long long want = WIDE ? (__ballot(c == -1) & 1ull) : __ballot(c == -1 && r == 0);
         if (want) {
@@ -276,52 +285,56 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                     c = -2;
                 } else if (fresh) {                             // opt.cpp:87-101,170-205
                     c = s;
-                    u0 = A.u[size_t(c) * NM];
-                    ascale = log(u0) * 2.0 * kSqrtPi;
-                    ul = in ? A.u[size_t(c) * NM + r] / u0 : 0.0;
-                    delta = PPN ? A.delta / (u0 * u0) : 0.0;
+                    const double u0 = A.u[size_t(c) * NM], ascale = log(u0) * 2.0 * kSqrtPi;
+                    const double ul = in ? A.u[size_t(c) * NM + r] / u0 : 0.0;
+                    const double delta = PPN ? A.delta / (u0 * u0) : 0.0;
+                    sr[4 * S_U0] = u0;
+                    sr[4 * S_ASCALE] = ascale;
+                    vl[64 * V_UL] = ul;
+                    if constexpr (PPN) sr[4 * S_DELTA] = delta;
                     // isotropicAlpha (opt.cpp:27-46) if asked for, or (the learned
                     // start with its network off) if the alpha passed in is not finite
                     al = in ? A.alpha[size_t(c) * NM + r] : 0.0;
                     bool iso = A.warm == MNC_WARM_ISOTROPIC;
                     if (A.warm == MNC_WARM_LEARNED) {
                         iso = row_max(isfinite(al) ? 0.0 : 1.0) != 0.0;
-                        if (owner && r == 0) { st.iso += iso; st.prev += !iso; }
+                        if (owner && r == 0) { st[R_ISO] += iso; st[R_PREV] += !iso; }
                         warm = iso ? 1 : 2;
                     }
                     if (iso) al = r == 0 ? (PPN ? 1.0 - 4.0 * delta * kPi : 2.0 * kSqrtPi * log(0.5 / kSqrtPi)) : 0.0;
                     else if (PPN) al = al / u0;
                     else if (r == 0) al = al - ascale;
-                    rtol = sqrt(row_sum(ul * ul)) * A.tol;
+                    sr[4 * S_RTOL] = sqrt(row_sum(ul * ul)) * A.tol;
                     t = 1.0;
                     iter = total = reg = 0;
                     maxit = A.max_iter;
                     mode = ST_NEWTON;
                     if (!(u0 > 0.0)) {
                         if (owner && r == 0) {
-                            st.err |= 1 << MNC_ERR_U0;
+                            st[R_ERR] |= 1 << MNC_ERR_U0;
                             if (A.outs) { A.outs[c].iter = -1; A.outs[c].r = 0.0; A.outs[c].norm_g = 0.0; }
                         }
                         c = -1;
                     } else if (owner && r == 0) {
-                        ++st.cells;
+                        ++st[R_CELLS];
                     }
                 } else {
                     c = s < count ? A.lists[size_t(lin) * A.cap + s] : A.lists[size_t(lin2) * A.cap + (s - count)];
                     const St S{A.st_d, A.st_i, A.cap};
                     al = in ? S.d(St::F_AL + r, c) : 0.0;
-                    ul = in ? S.d(St::F_U + r, c) : 0.0;
-                    aold = in ? S.d(St::F_AOLD + r, c) : 0.0;
-                    dl = in ? S.d(St::F_D + r, c) : 0.0;
+                    const double aold = in ? S.d(St::F_AOLD + r, c) : 0.0;
+                    vl[64 * V_UL] = in ? S.d(St::F_U + r, c) : 0.0;
+                    vl[64 * V_AOLD] = aold;
+                    vl[64 * V_DL] = in ? S.d(St::F_D + r, c) : 0.0;
                     t = S.d(St::F_T, c);
-                    rtol = S.d(St::F_RTOL, c);
-                    u0 = S.d(St::F_U0, c);
-                    ascale = S.d(St::F_ASCALE, c);
-                    fcur_s = S.d(St::F_FCUR, c);
-                    gd_s = S.d(St::F_GD, c);
-                    fscale_s = S.d(St::F_FSCALE, c);
-                    maxf_s = S.d(St::F_MAXF, c);
-                    delta = PPN ? S.d(St::F_DELTA, c) : 0.0;
+                    sr[4 * S_RTOL] = S.d(St::F_RTOL, c);
+                    sr[4 * S_U0] = S.d(St::F_U0, c);
+                    sr[4 * S_ASCALE] = S.d(St::F_ASCALE, c);
+                    sr[4 * S_FCUR] = S.d(St::F_FCUR, c);
+                    sr[4 * S_GD] = S.d(St::F_GD, c);
+                    sr[4 * S_FSCALE] = S.d(St::F_FSCALE, c);
+                    sr[4 * S_MAXF] = S.d(St::F_MAXF, c);
+                    if constexpr (PPN) sr[4 * S_DELTA] = S.d(St::F_DELTA, c);
                     mode = S.i(St::I_MODE, c);
                     iter = S.i(St::I_ITER, c);
                     total = S.i(St::I_TOTAL, c);
@@ -329,8 +342,8 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                     maxit = S.i(St::I_MAXIT, c);
                     warm = S.i(St::I_WARM, c);
                     if (owner && r == 0) {
-                        ++st.cells;
-                        st.titer -= total;
+                        ++st[R_CELLS];
+                        st[R_TITER] -= total;
                     }
                     // The reference's Armijo test compares values of f down to
                     // their rounding, which differs between the kernels: a
@@ -351,7 +364,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
             continue;
         }
         // ---- the sweep ----
-        als[r * 4 + rowc] = r == 15 ? delta : al;
+        als[r * 4 + rowc] = PPN && r == 15 ? sr[4 * S_DELTA] : al;
         __builtin_amdgcn_wave_barrier();
         // after two failed trials only f is summed: the next trials mostly fail
         // too, and an accepted one is evaluated in full afterwards
@@ -468,25 +481,28 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
         // ---- one step of the per-cell logic ----
         bool done = false;
         if (c >= 0) {
+            const double ul = vl[64 * V_UL];
             constexpr int SFP = PPN ? NS + NM : L.first[1];
             const double sf = sum_at(SFP);
             bool newton = mode == ST_NEWTON, do_reg = false, converged = false;
             double err = 0.0, gv = 0.0;
             if (mode == ST_TRIAL) {                             // linesearch.cpp:45-98
-                if (owner && r == 0) ++st.trials;
+                if (owner && r == 0) ++st[R_TRIALS];
                 const double fnew = sf - row_sum(al * ul);
-                bool accept = fnew <= fcur_s + 1e-3 * t * gd_s;
+                const double gd_s = sr[4 * S_GD];
+                bool accept = fnew <= sr[4 * S_FCUR] + 1e-3 * t * gd_s;
                 // Robust mode: a full Newton step whose predicted decrease lies
                 // below the rounding resolution of f is taken.
-                if (!accept && A.ls_mode == MNC_LS_ROBUST && t == 1.0 && -gd_s <= 1e3 * DBL_EPSILON * fscale_s)
+                if (!accept && A.ls_mode == MNC_LS_ROBUST && t == 1.0 && -gd_s <= 1e3 * DBL_EPSILON * sr[4 * S_FSCALE])
                     accept = true;
                 if (accept) {
                     if (fonly) mode = ST_NEWTON;                // evaluated in full next
                     else newton = true;
                 } else {
                     t = 0.5 * t;
-                    if (t * maxf_s > DBL_EPSILON / 2) {
-                        al = fma(t, dl, aold);
+                    const double aold = vl[64 * V_AOLD];
+                    if (t * sr[4 * S_MAXF] > DBL_EPSILON / 2) {
+                        al = fma(t, vl[64 * V_DL], aold);
                     } else {                                    // exhausted
                         al = aold;
                         t = 0.0;
@@ -511,7 +527,14 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) at[q] = reinterpret_cast<const unsigned *>(A.opos)[r * 4 + q];
 #pragma unroll
-                    for (int k = 0; k < NM; ++k) h[k] = in ? sum_at((at[k >> 2] >> (8 * (k & 3))) & 255u) : 0.0;
+                    for (int k = 0; k < NM; ++k) h[k] = sum_at((at[k >> 2] >> (8 * (k & 3))) & 255u);
+                    // every lane loads (row 15 of the places is zeros) before any selects:
+                    // as conditional loads these were 15 branches, each with its wait
+#pragma unroll
+                    for (int k = 0; k < NM; ++k) {
+                        __asm__ volatile("" : "+v"(h[k]));
+                        h[k] = in ? h[k] : 0.0;
+                    }
                 }
                 const double h00 = row_bcast<0>(h[0]);
                 gv = in ? (PPN ? sum_at(NS + r) : h[0] / p0) - ul : 0.0;
@@ -549,6 +572,10 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                         h[k] = fma(-row_bcast<k>(l), l, h[k]);
                     });
                 });
+                // the factor as new values: else its 105 broadcasts are kept from the
+                // steps above for the ones below, in scratch
+#pragma unroll
+                for (int k = 0; k < NM; ++k) __asm__ volatile("" : "+v"(h[k]));
                 // Z = L^-1, column j on lane j, and L^-1 g on lane NM
                 double z[NM];
                 unroll<0, NM>([&](auto I) {
@@ -572,6 +599,14 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 });
                 double condest = 0.0;
                 bool ask = ok && !cond_proven_below(anorm, gersh, NM, A.cond_h_max);
+                if (ask) {
+                    // ||A^-1||_1 <= sqrt(n) trace(A^-1), the trace the sum of Z's squares:
+                    // a row's sum against the columns' products below
+                    double s = 0.0;
+#pragma unroll
+                    for (int k = 0; k < NM; ++k) s = fma(z[k], z[k], s);
+                    ask = !(2.0 * anorm * sqrt(double(NM)) * row_sum(in ? s : 0.0) <= A.cond_h_max);
+                }
                 if (ask) {
                     // ||A^-1||_1 from the columns of Z^T Z; the estimate never exceeds it
                     double s = 0.0;
@@ -606,7 +641,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 if (iter >= maxit || !ok || t == 0.0 || condest > A.cond_h_max) {
                     do_reg = true;                              // opt.cpp:244
                 } else {
-                    bool stop = err <= rtol;
+                    bool stop = err <= sr[4 * S_RTOL];
                     if (A.tol_gamma > 0.0) {
                         const double da1 = row_sum(in ? fabs(x) : 0.0);
                         stop = stop && gamma_ok(A, da1, PPN);
@@ -616,12 +651,12 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                     } else {                                    // linesearch.cpp:28-43
                         const double di = in ? -x : 0.0;
                         const double maxf = row_max(in ? fabs(di) / (fabs(al) + 1e-100) : 0.0);
-                        aold = al;
-                        dl = di;
-                        maxf_s = maxf;
-                        gd_s = row_sum(gv * di);
-                        fcur_s = fcur;
-                        fscale_s = fscale;
+                        vl[64 * V_AOLD] = al;
+                        vl[64 * V_DL] = di;
+                        sr[4 * S_MAXF] = maxf;
+                        sr[4 * S_GD] = row_sum(gv * di);
+                        sr[4 * S_FCUR] = fcur;
+                        sr[4 * S_FSCALE] = fscale;
                         t = 1.0;
                         if (t * maxf > DBL_EPSILON / 2) {
                             al = al + di;
@@ -638,7 +673,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 warm = kWarmFellBack;
                 if (owner && r == 0) {
                     St{A.st_d, A.st_i, A.cap}.i(St::I_WARM, c) = kWarmFellBack;
-                    ++st.fallback;
+                    ++st[R_FALLBACK];
                 }
                 al = r == 0 ? 2.0 * kSqrtPi * log(0.5 / kSqrtPi) : 0.0;
                 iter = 0;
@@ -648,21 +683,23 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 if (reg < 4) {
                     ++reg;
                     const double rr = kReg[reg];
-                    ul = r == 0 ? 1.0 : (in ? (A.u[size_t(c) * NM + r] / u0) * (1.0 - rr) : 0.0);
-                    rtol = sqrt(row_sum(ul * ul)) * A.tol;
-                    al = r == 0 ? (PPN ? 1.0 - 4.0 * delta * kPi : 2.0 * kSqrtPi * log(0.5 / kSqrtPi)) : 0.0;
+                    const double uk = r == 0 ? 1.0 : (in ? (A.u[size_t(c) * NM + r] / sr[4 * S_U0]) * (1.0 - rr) : 0.0);
+                    vl[64 * V_UL] = uk;
+                    sr[4 * S_RTOL] = sqrt(row_sum(uk * uk)) * A.tol;
+                    al = r == 0 ? (PPN ? 1.0 - 4.0 * sr[4 * S_DELTA] * kPi : 2.0 * kSqrtPi * log(0.5 / kSqrtPi)) : 0.0;
                     iter = 0;
                     t = 1.0;
                     if (reg == 4) maxit = 10 * maxit;
                     mode = ST_NEWTON;
                 } else {                                        // "Max regularization achieved."
                     if (owner && r == 0) {
-                        st.err |= 1 << MNC_ERR_MAXREG;
+                        st[R_ERR] |= 1 << MNC_ERR_MAXREG;
                         if (A.outs) { A.outs[c].iter = total; A.outs[c].r = -1.0; A.outs[c].norm_g = err; }
                     }
                     done = true;
                 }
             } else if (converged) {
+                const double u0 = sr[4 * S_U0];
                 double un, an;
                 if (PPN) {                                      // no reconstruction; opt.cpp:131-136
                     un = ul * u0;
@@ -670,7 +707,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 } else {                                        // :298-302, opt.cpp:107-109
                     const double u0p = row_bcast<0>(ul) + row_bcast<0>(gv);
                     un = ((ul + gv) / u0p) * u0;
-                    an = r == 0 ? (al - log(u0p) * 2.0 * kSqrtPi) + ascale : al;
+                    an = r == 0 ? (al - log(u0p) * 2.0 * kSqrtPi) + sr[4 * S_ASCALE] : al;
                 }
                 if (owner && in) {
                     A.u[size_t(c) * NM + r] = un;
@@ -678,11 +715,10 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
                 }
                 if (owner && r == 0) {
                     if (A.outs) { A.outs[c].iter = total; A.outs[c].r = kReg[reg]; A.outs[c].norm_g = err; }
-                    st.max_iter = total > st.max_iter ? total : st.max_iter;
-                    st.sum += total;
-                    ++st.n;
-#pragma unroll
-                    for (int i = 0; i < 5; ++i) st.hist[i] += reg == i;
+                    st[R_MAX_ITER] = max(total, st[R_MAX_ITER]);
+                    st[R_SUM] += total;
+                    ++st[R_N];
+                    ++st[R_HIST + reg];
                 }
                 done = true;
             }
@@ -691,17 +727,18 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
         __builtin_amdgcn_wave_barrier();
     }
     // statistics: the block's counts, one atomic each
+    static_assert(kRowCounts == 15, "one thread per count below");
     lane = threadIdx.x & 63;
-    int v[15] = {st.max_iter, st.err, st.sum, st.n, st.trials, st.hist[0], st.hist[1], st.hist[2], st.hist[3], st.hist[4],
-                 st.cells, st.titer + st.sum, st.fallback, st.iso, st.prev};
-#pragma unroll
-    for (int i = 0; i < 15; ++i) {
-#pragma unroll
-        for (int o = 16; o < 64; o <<= 1) {
-            const int x = __shfl_xor(v[i], o);
-            v[i] = i == 0 ? max(v[i], x) : (i == 1 ? v[i] | x : v[i] + x);
+    if (lane < kRowCounts) {
+        const int *n = counts + lane;
+        const int x[4] = {n[0], n[kRowCounts], n[2 * kRowCounts], n[3 * kRowCounts]};
+        int v = lane == R_MAX_ITER ? max(max(x[0], x[1]), max(x[2], x[3]))
+                                   : (lane == R_ERR ? x[0] | x[1] | x[2] | x[3] : x[0] + x[1] + x[2] + x[3]);
+        if (lane == R_TITER) {          // less what the listed cells brought with them
+            const int *m = counts + R_SUM;
+            v += m[0] + m[kRowCounts] + m[2 * kRowCounts] + m[3 * kRowCounts];
         }
-        if (lane == 0) red[wave][i] = v[i];
+        red[wave][lane] = v;
     }
     __syncthreads();
     if (threadIdx.x < 15) {
@@ -721,7 +758,7 @@ void rows_kernel(NewtonArgs A, int lin, int lin2, int fresh, int few) {
     }
 }
 
-constexpr int kRowTableBytes = 40 * 1024;    // the orbit table in LDS up to here (with the sums under 64 KB), else read from L2
+constexpr int kRowLdsBytes = 64 * 1024;      // the orbit table in LDS while it and the waves' words fit, else read from L2
 
 template <int N, bool GAUNT, bool PPN, bool WIDE>
 void launch_rows_w(const NewtonArgs &a, int blocks, int lin, int lin2, bool fresh, bool few, hipStream_t s) {
@@ -729,7 +766,7 @@ void launch_rows_w(const NewtonArgs &a, int blocks, int lin, int lin2, bool fres
     const size_t table = size_t(Dm::NP2 + 1) * a.nop * sizeof(double);
     const size_t own = size_t(kRowWaves) * Dm::LANE_WORDS * sizeof(double);
     const dim3 g(blocks), b(64 * kRowWaves);
-    if (table <= size_t(kRowTableBytes))
+    if (table + own <= size_t(kRowLdsBytes) - 512)
         hipLaunchKernelGGL((rows_kernel<N, GAUNT, PPN, WIDE, true>), g, b, table + own, s, a, lin, lin2, int(fresh), int(few));
     else
         hipLaunchKernelGGL((rows_kernel<N, GAUNT, PPN, WIDE, false>), g, b, own, s, a, lin, lin2, int(fresh), int(few));
@@ -741,8 +778,8 @@ void launch_rows_n(const NewtonArgs &a, int lin, int lin2, bool fresh, int num_c
     // not four); four cells per wave share the algebra's issue slots.  Up to
     // two waves per SIMD the first wins, above it the chip is full either way.
     // Against the lockstep kernels and a tail of one wave per cell (M4, Q = 16):
-    // 2,049 closures from near starts 1.01 -> 0.149 ms, 150,001 cold ones with
-    // a fifth near the realizability boundary 12.3 -> 6.98 ms; 60 of M2 320 -> 73 us.
+    // 2,049 closures from near starts 1.01 -> 0.09 ms, 150,001 cold ones with
+    // a fifth near the realizability boundary 12.3 -> 3.1 ms; 60 of M2 320 -> 71 us.
     if (fresh) {
         const int waves = 4 * num_cu;                         // one per SIMD
         if (a.ncells <= 2 * waves) {
