@@ -577,6 +577,7 @@ mnc::GridArgs grid_args(mnc_ctx *ctx) {
     g.nm = t.nm;
     g.np2 = t.np2;
     g.nq = t.nq;
+    g.half = t.Q / 2;
     g.dx = ctx->grid.dx;
     g.dy = ctx->grid.dy;
     g.theta = ctx->grid.theta;

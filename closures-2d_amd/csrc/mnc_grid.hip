@@ -307,26 +307,66 @@ __global__ void ghost_y_kernel(GridArgs g) {
     g.moments[(size_t(i) * NY + y3 + jj) * nm + k] = g.moments[(size_t(i) * NY + y1 + jj) * nm + k];
 }
 
-// The fused ansatz + flux with the directions split into gridDim.z groups of
-// consecutive q: block (tile, z) sums the flux of its TX x TY cells over group
-// z's directions into fpart[z] (interior cells, [cell][k]), and
-// flux_sum_kernel adds the groups in order and applies the Euler stage.  With
-// 80,656 cells a launch of one group per tile is about one wave per SIMD and
-// waits on latency; the groups multiply the waves in flight.  alpha of the
-// halo cells a thread evaluates stays in its registers, so LDS holds only E.
-// Per cell and direction the arithmetic is flux_fused_kernel's except that
-// (f1 + f2) / dx + (f3 + f4) / dy multiplies by reciprocals, and the q sum is
-// split into the groups: the result moves at rounding level.
-template <int NM, int TX, int TY, int QC>
+// minmod(theta (r - c), (r - l) / 2, theta (c - l)): 0 unless all three share
+// their sign, else the smallest magnitude with it (slopefit's values).
+__device__ __forceinline__ double slope3(double l, double c, double r, double theta) {
+    const double a = theta * (r - c), b = theta * (c - l), m = 0.5 * (r - l);
+    const double v = fmin(fmin(fabs(a), fabs(b)), fabs(m));
+    const int s = __double2hiint(m);
+    return ((__double2hiint(a) ^ s) | (__double2hiint(b) ^ s)) < 0 ? 0.0 : copysign(v, m);
+}
+
+// Difference of the face values around c for the upwind side `up` (+1: the wind
+// comes from below).
+template <int UP>
+__device__ __forceinline__ double face_diff(double m2, double m1, double c, double p1, double p2, double theta) {
+    if constexpr (UP > 0) return c + 0.5 * slope3(m1, c, p1, theta) - m1 - 0.5 * slope3(m2, m1, c, theta);
+    else return p1 - 0.5 * slope3(c, p1, p2, theta) - c + 0.5 * slope3(m1, c, p1, theta);
+}
+
+template <class T>
+__device__ __forceinline__ void each_class(T &&f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+    f(std::integral_constant<int, 3>{});
+}
+
+template <int NM> constexpr int order_of_nm() {
+    int N = 0;
+    while (orbit_nm(N) < NM) ++N;
+    return N;
+}
+template <int NM> struct Classes {
+    unsigned char of[NM];
+    constexpr Classes() : of{} {
+        for (int k = 0; k < NM; ++k) of[k] = (unsigned char)orbit_class(k);
+    }
+};
+
+// The fused ansatz + flux with the quadrature's orbits (mnc_orbit.h) split into
+// gridDim.z groups: block (tile, z) sums the flux of its TX x TY cells over group
+// z's orbits into fpart[z] (interior cells, [cell][k]), and flux_sum_kernel adds
+// the groups in order and applies the Euler stage.  Per chunk of OC orbits the
+// ansatz at their four images goes to LDS for the tile and its halo of two cells
+// (evaluated by both neighbouring tiles; alpha of a thread's halo cells stays in
+// registers), then each thread takes its cell's stencil.  Bound by FP64 issue, some
+// 500 instructions per orbit and cell: the four images share one pass over the
+// moments before the ansatz and one after the stencil, their upwind sides are
+// known when compiled, and a slope is thirteen instructions.  Direction by
+// direction (two passes of n FMAs, branches on the signs, slopes of selects) M4,
+// Q = 16 took 190 us a stage at 280^2 and 63 at 133 x 101; now 133 and 45.
+template <int NM, int TX, int TY, int OC>
 __global__ __launch_bounds__(TX * TY) void flux_split_kernel(GridArgs g) {
     static_assert(TX == kSplitTile && TY == kSplitTile, "the tile flags' geometry");
     if (g.tile_mode != 0) {   // this launch's share of the tiles (uniform over the block)
         const bool flagged = g.tile_flag[blockIdx.x * gridDim.y + blockIdx.y] != 0;
         if (flagged != (g.tile_mode == 2)) return;
     }
+    constexpr Classes<NM> cls{};
     constexpr int HX = TX + 4, HY = TY + 4, NH = HX * HY, NT = TX * TY;
     constexpr int HPT = (NH + NT - 1) / NT;                  // halo cells evaluated per thread
-    __shared__ double E_s[QC][NH];
+    __shared__ double E_s[4 * OC][NH];
     const int tid = threadIdx.x;
     const int tx0 = blockIdx.x * TX, ty0 = blockIdx.y * TY;
     const int NX = g.NX, NY = g.NY;
@@ -344,58 +384,51 @@ __global__ __launch_bounds__(TX * TY) void flux_split_kernel(GridArgs g) {
     const bool active = (tx0 + li < g.nx) && (ty0 + lj < g.ny);
     const int hc = (li + 2) * HY + (lj + 2);
     const double theta = g.theta, rdx = 1.0 / g.dx, rdy = 1.0 / g.dy;
-    const int per = (g.nq + gridDim.z - 1) / gridDim.z;
-    const int qa = blockIdx.z * per, qb = min(g.nq, qa + per);
+    const int half = g.half, no = half * half;
+    const int per = (no + gridDim.z - 1) / gridDim.z;
+    const int oa = blockIdx.z * per, ob = min(no, oa + per);
+    auto node = [&](int o) { return 4 * half * (o / half) + o % half; };   // the orbit's node with xi, eta > 0
     double F[NM];
 #pragma unroll
     for (int k = 0; k < NM; ++k) F[k] = 0.0;
-    for (int q0 = qa; q0 < qb; q0 += QC) {
-        const int nqc = min(QC, qb - q0);
+    for (int o0 = oa; o0 < ob; o0 += OC) {
+        const int noc = min(OC, ob - o0);
         __syncthreads();
-        for (int qq = 0; qq < nqc; ++qq) {
-            const double *row = g.p + size_t(q0 + qq) * g.np2;
+        for (int oo = 0; oo < noc; ++oo) {
+            const double *row = g.p + size_t(node(o0 + oo)) * g.np2;
 #pragma unroll
             for (int hh = 0; hh < HPT; ++hh) {
                 const int h = tid + hh * NT;
                 if (h < NH) {
-                    double sa = 0.0;
+                    double z[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                    for (int k = 0; k < NM; ++k) sa = fma(al[hh][k], row[k], sa);
-                    E_s[qq][h] = ansatz_value(g, sa);
+                    for (int k = 0; k < NM; ++k) z[cls.of[k]] = fma(al[hh][k], row[k], z[cls.of[k]]);
+                    const double ep = z[0] + z[1], em = z[0] - z[1], op = z[2] + z[3], om = z[2] - z[3];
+                    E_s[4 * oo][h] = ansatz_value(g, ep + op);
+                    E_s[4 * oo + 1][h] = ansatz_value(g, em + om);         // -xi: classes 1 and 3 change sign
+                    E_s[4 * oo + 2][h] = ansatz_value(g, ep - op);         // -eta: classes 2 and 3
+                    E_s[4 * oo + 3][h] = ansatz_value(g, em - om);         // both: classes 1 and 2
                 }
             }
         }
         __syncthreads();
         if (!active) continue;
-        for (int qq = 0; qq < nqc; ++qq) {
-            const int q = q0 + qq;
-            const double *E = E_s[qq];
-            const double xi = g.xi[q], eta = g.eta[q], w = g.w[q];
-            double f1 = 0.0, f2 = 0.0, f3 = 0.0, f4 = 0.0;
-            if (xi > 0) {
-                const double k1 = E[hc - 2 * HY], k2 = E[hc - HY], k3 = E[hc], k4 = E[hc + HY];
-                f1 = k3 + 0.5 * slopefit(k2, k3, k4, theta) - k2 - 0.5 * slopefit(k1, k2, k3, theta);
-                f1 = f1 * xi * w;
-            }
-            if (xi < 0) {
-                const double k1 = E[hc - HY], k2 = E[hc], k3 = E[hc + HY], k4 = E[hc + 2 * HY];
-                f2 = k3 - 0.5 * slopefit(k2, k3, k4, theta) - k2 + 0.5 * slopefit(k1, k2, k3, theta);
-                f2 = f2 * xi * w;
-            }
-            if (eta > 0) {
-                const double k1 = E[hc - 2], k2 = E[hc - 1], k3 = E[hc], k4 = E[hc + 1];
-                f3 = k3 + 0.5 * slopefit(k2, k3, k4, theta) - k2 - 0.5 * slopefit(k1, k2, k3, theta);
-                f3 = f3 * eta * w;
-            }
-            if (eta < 0) {
-                const double k1 = E[hc - 1], k2 = E[hc], k3 = E[hc + 1], k4 = E[hc + 2];
-                f4 = k3 - 0.5 * slopefit(k2, k3, k4, theta) - k2 + 0.5 * slopefit(k1, k2, k3, theta);
-                f4 = f4 * eta * w;
-            }
-            const double comb = (f1 + f2) * rdx + (f3 + f4) * rdy;
+        for (int oo = 0; oo < noc; ++oo) {
+            const int q = node(o0 + oo);
+            const double fx = g.xi[q] * g.w[q] * rdx, fy = g.eta[q] * g.w[q] * rdy;
+            double comb[4];
+            each_class([&](auto img) {
+                constexpr int I = decltype(img)::value, UX = I & 1 ? -1 : 1, UY = I & 2 ? -1 : 1;
+                const double *e = &E_s[4 * oo + I][hc];
+                const double c = e[0], xm1 = *(e - HY), xp1 = e[HY], ym1 = *(e - 1), yp1 = e[1];
+                const double xo = UX > 0 ? *(e - 2 * HY) : e[2 * HY], yo = UY > 0 ? *(e - 2) : e[2];
+                comb[I] = UX * fx * face_diff<UX>(xo, xm1, c, xp1, xo, theta) + UY * fy * face_diff<UY>(yo, ym1, c, yp1, yo, theta);
+            });
+            const double ep = comb[0] + comb[1], em = comb[0] - comb[1], op = comb[2] + comb[3], om = comb[2] - comb[3];
+            const double C[4] = {ep + op, em + om, ep - op, em - om};
             const double *row = g.p + size_t(q) * g.np2;
 #pragma unroll
-            for (int k = 0; k < NM; ++k) F[k] = fma(row[k], comb, F[k]);
+            for (int k = 0; k < NM; ++k) F[k] = fma(row[k], C[cls.of[k]], F[k]);
         }
     }
     if (!active) return;
@@ -431,7 +464,7 @@ void launch_fused_t(const GridArgs &g, int tile, int stage, double dt, hipStream
     if constexpr (NM <= 15) {   // alpha of two halo cells per thread in registers
         if (tile == 3) {
             const dim3 grid((g.nx + 15) / 16, (g.ny + 15) / 16, g.groups);
-            hipLaunchKernelGGL((flux_split_kernel<NM, 16, 16, 8>), grid, dim3(256), 0, s, g);
+            hipLaunchKernelGGL((flux_split_kernel<NM, 16, 16, 2>), grid, dim3(256), 0, s, g);
             hipLaunchKernelGGL((flux_sum_kernel<NM>), dim3((g.nx * g.ny + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
                                g, g.groups, stage, dt);
             return;
@@ -469,14 +502,6 @@ struct FluxShape {
     static constexpr int k0(int c) { return c == 0 ? 0 : k0(c - 1) + kz(c - 1); }
     static constexpr int KZ = k0(4);
 };
-template <class T>
-__device__ __forceinline__ void each_class(T &&f) {
-    f(std::integral_constant<int, 0>{});
-    f(std::integral_constant<int, 1>{});
-    f(std::integral_constant<int, 2>{});
-    f(std::integral_constant<int, 3>{});
-}
-
 // E[4 orbit + image][cell] of the orbit tiles T0 .. T0 + ntc - 1.  A wave takes 16
 // cells and every gridDim.y-th tile.  Bound by the exponentials and the store (82 MB at 96^2).
 template <int N>
@@ -517,23 +542,6 @@ __global__ __launch_bounds__(256) void ansatz_orbit_kernel(GridArgs g, int T0, i
             E[3 * size_t(ncell)] = ansatz_value(g, em - om);         // both: classes 1 and 2
         }
     }
-}
-
-// minmod(theta (r - c), (r - l) / 2, theta (c - l)): 0 unless all three share
-// their sign, else the smallest magnitude with it (slopefit's values).
-__device__ __forceinline__ double slope3(double l, double c, double r, double theta) {
-    const double a = theta * (r - c), b = theta * (c - l), m = 0.5 * (r - l);
-    const double v = fmin(fmin(fabs(a), fabs(b)), fabs(m));
-    const int s = __double2hiint(m);
-    return ((__double2hiint(a) ^ s) | (__double2hiint(b) ^ s)) < 0 ? 0.0 : copysign(v, m);
-}
-
-// Difference of the face values around c for the upwind side `up` (+1: the wind
-// comes from below).
-template <int UP>
-__device__ __forceinline__ double face_diff(double m2, double m1, double c, double p1, double p2, double theta) {
-    if constexpr (UP > 0) return c + 0.5 * slope3(m1, c, p1, theta) - m1 - 0.5 * slope3(m2, m1, c, theta);
-    else return p1 - 0.5 * slope3(c, p1, p2, theta) - c + 0.5 * slope3(m1, c, p1, theta);
 }
 
 constexpr int kFluxWaves = 8;
@@ -626,12 +634,6 @@ __global__ __launch_bounds__(64 * kFluxWaves) void flux_orbit_kernel(GridArgs g,
         if (stage == 2) v = 0.5 * (v + g.moments_old[o]);
         g.moments[o] = v;
     }
-}
-
-template <int NM> constexpr int order_of_nm() {
-    int N = 0;
-    while (orbit_nm(N) < NM) ++N;
-    return N;
 }
 
 template <int NM>

@@ -261,6 +261,7 @@ void mlp_predict_listed(const MlpBuffers &b, const double *u, const int *list, c
 // Arguments of the grid kernels (mnc_grid.hip).
 struct GridArgs {
     int nx, ny, NX, NY, nm, np2, nq;
+    int half;             // Q / 2: half x half orbits of four mirrored nodes
     double dx, dy, theta, init_x, init_y;
     int init_cond;
     const double *w, *p, *xi, *eta;
