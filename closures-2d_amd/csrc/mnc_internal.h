@@ -267,7 +267,7 @@ struct GridArgs {
     const double *w, *p, *xi, *eta;
     double *moments, *alpha, *moments_old, *sigma_t, *sigma_s, *flux, *ansatz;
     double *fpart;        // [groups][nx*ny][nm]: per-group partial fluxes (flux_tile 3)
-    int groups;           // direction groups of flux_tile 3 (1..kMaxFluxGroups)
+    int groups;           // direction groups of flux_tile 3
     int ppn;              // the PPn ansatz (computeAnsatz, momopt_update.cpp:54-57)
     double delta;         // its delta
     // flux_tile 3 on part of the grid: 0 every tile; 1 the tiles whose flag is
@@ -278,7 +278,8 @@ struct GridArgs {
     const int *tile_flag; // [tiles_x][tiles_y] of kSplitTile x kSplitTile cells
     int tile_mode;
 };
-constexpr int kMaxFluxGroups = 8;
+constexpr int kMaxFluxGroups = 8;      // what a caller may set
+constexpr int kMostFluxGroups = 16;    // what a small grid takes by itself
 constexpr int kSplitTile = 16;   // flux_tile 3's cells per tile side
 // flags[tx][ty] = 1 for the flux_tile 3 tiles whose stencil region (the tile
 // and two cells around it) holds a cell on list0 (count *cnt0) or list1 (*cnt1);

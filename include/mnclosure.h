@@ -324,7 +324,7 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *                  as 1): 16x16 tiles with the directions split
  *                  into "flux_groups" groups summed in order and reciprocals
  *                  of dx, dy (rounding-level differences from 0-2)
- *   "flux_groups"  direction groups of flux_tile 3 (1-8, default 6)
+ *   "flux_groups"  direction groups of flux_tile 3 (1-8; by default 6, more on small grids)
  *   "flux_overlap" flux_tile 3 in mnc_update: 1 (default): after a stage's
  *                  lockstep rounds, the flux of the tiles whose stencil region
  *                  holds no cell left for the Newton tail runs on a second
