@@ -376,12 +376,19 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     lp.r0 = 0;
     // FP64 cells go straight to the tail kernel unless rounds are asked for.
     // Not with the reference's line search below TOL 1e-6: there its Armijo
-    // test compares values of f that differ by f's rounding, so the path
-    // depends on the order of the sums, and the lockstep kernels sum in the
-    // reference's; twelve rounds end all but the slow cells there.
+    // test compares values of f that differ by f's rounding, so a cell's last
+    // steps depend on the order of the sums, and the lockstep kernels sum in the
+    // reference's.  Seven rounds are the fewest after which no more than one per
+    // cent of the cells that take the reference's iterations end elsewhere than it
+    // does (3,000 M3 closures, Q = 30, four draws: 1.27% without rounds, 1.05 after
+    // six, 0.84 after seven, 0.84 after twelve; 0.88 with six and the former tail
+    // of a wave per cell).  Against that form (ms, M4, Q = 16, means over draws):
+    // 2,049 closures from near starts 2.4 -> 1.6 (its best draws 1.5), cold 3.4 ->
+    // 1.8, 200,003 cold 16.3 -> 9.7, 150,001 with beams 19.5 -> 9.3, a 133 x 101
+    // lattice's step 7.9 -> 3.5; with twelve rounds 2.5, 2.8, 8.4, 9.6 and 5.4.
     const bool by_rounding = o->line_search == MNC_LS_REFERENCE && o->tol_rel < 1e-6;
     const bool network = learned && ctx->learned_gate_log10 < kGateOff;
-    const int rounds = ctx->rounds >= 0 ? ctx->rounds : (mixed || network ? 6 : (by_rounding ? 12 : 0));
+    const int rounds = ctx->rounds >= 0 ? ctx->rounds : (mixed || network ? 6 : (by_rounding ? 7 : 0));
     lp.r1 = rounds;
     lp.num_cu = ctx->num_cu;
     lp.fresh = rounds == 0 && !mixed && !network && (ctx->tail_mode == 0 || ctx->tail_mode == 3 || ctx->ppn);

@@ -790,8 +790,9 @@ void launch_rows_n(const NewtonArgs &a, int lin, int lin2, bool fresh, int num_c
         }
         return;
     }
-    launch_rows_w<N, GAUNT, PPN, true>(a, tail_blocks, lin, lin2, false, true, s);
-    launch_rows_w<N, GAUNT, PPN, false>(a, tail_blocks, lin, lin2, false, true, s);
+    const bool few = a.ncells > tail_blocks * kRowWaves;       // else every list fits one cell per wave
+    launch_rows_w<N, GAUNT, PPN, true>(a, tail_blocks, lin, lin2, false, few, s);
+    if (few) launch_rows_w<N, GAUNT, PPN, false>(a, tail_blocks, lin, lin2, false, true, s);
 }
 
 }  // namespace

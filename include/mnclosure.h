@@ -280,7 +280,7 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *   "rounds"       lockstep sweep/logic rounds before the persistent tail (0-512);
  *                  until it is set: 6 in mixed precision or where the network
  *                  is consulted, 0 in FP64 (the tail's kernel takes every cell;
- *                  12 with the reference's line search below TOL 1e-6, whose
+ *                  7 with the reference's line search below TOL 1e-6, whose
  *                  decisions depend on the order of the sums); reads 6 then
  *   "tail_blocks"  workgroups of the persistent tail kernel (1-65536)
  *   "tail_mode"    0: a 16-lane row per remaining cell, four cells per wave (one

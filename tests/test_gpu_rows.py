@@ -98,3 +98,35 @@ def test_rows_bad_cells_and_lists():
         assert np.array_equal(itl, itg)
         assert np.abs(al - ag).max() <= 1e-10 * (1.0 + np.abs(ag).max())
     ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,Q,n,ppn", [(2, 12, 60, False), (4, 16, 2048, False), (4, 16, 2500, False), (2, 12, 70, True)])
+def test_reference_line_search_takes_seven_rounds(order, Q, n, ppn):
+    """Below TOL 1e-6 the reference's line search goes by the rounding of f, so an
+    untouched context runs seven lockstep rounds, no more (each costs a small batch a
+    lane's walk over the quadrature), before this kernel takes what is left: the same
+    bits and counts as with the rounds set, for batches that one cell per wave
+    covers and that it does not."""
+    mnc, o = load_pkg("mnc"), oracle()
+    print("case reference rounds N=%d n=%d ppn=%d" % (order, n, ppn), flush=True)
+    tab, u, _ = _mn_batch(o, order, Q, False, n, 40 + n)
+    a0 = isotropic_start(u)
+    if ppn:
+        a0[:, 0] = u[:, 0] - 4.0 * np.pi * 1e-10 / u[:, 0]
+    res = []
+    for rounds in (None, 7):
+        ctx = mnc.Context(order, Q, moment_type=mnc.MOMENT_PPN if ppn else mnc.MOMENT_MN)
+        if rounds is not None:
+            ctx.tune("rounds", rounds)
+        opt = mnc.options(tol=1e-8, line_search=mnc.LS_REFERENCE, delta_ppn=1e-10 if ppn else 0.0)
+        out = ctx.opt_batch_host(u, a0, opt, allow_status=(mnc.OK, mnc.ERR_MAXREG))
+        s = ctx.stats()
+        res.append((out, (s.iter_sum, s.trial_sum, s.tail_cells, s.tail_iter_sum)))
+        ctx.close()
+    assert res[0][0][0] == res[1][0][0] and res[0][1] == res[1][1]
+    for a, b in zip(res[0][0][1:], res[1][0][1:]):
+        assert np.array_equal(a, b)
+    if not ppn:
+        _, _, _, ito, ro, _ = tab.opt_batch(u, a0, tol=1e-8, nthreads=8)
+        assert ((res[0][0][3] == ito) & (res[0][0][4] == ro)).mean() >= 0.95
