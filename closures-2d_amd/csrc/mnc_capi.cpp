@@ -63,7 +63,7 @@ struct mnc_ctx {
     int mix_blocks = 0;              // 0: one per CU
     int flux_tile = 3;               // 0: ansatz to HBM + flux; 1: fused, 8x8 tiles; 2: fused, 16x16;
                                      // 3: fused, 16x16, directions split into flux_groups
-    int flux_groups = 0;             // direction groups of flux_tile 3; 0: by the grid (flux_groups_of)
+    int flux_groups = 0;             // direction groups of flux_tile 3; 0: by the grid (auto_flux_groups)
     int flux_overlap = 1;            // flux_tile 3: the flux of tiles clear of the Newton tail runs beside it
     int learned_fused = 1;           // 1: network and judge in one kernel; 0: the GEMM kernels, then the judge
     int learned_fallback_iters = 10;   // a network-started cell failing at level 0 within this many
@@ -578,8 +578,7 @@ int run_optcb_grid(mnc_ctx *ctx, int nc, const mnc_options *o, bool check) {
 // as give three blocks per CU, up to 16 (each group's sums are one more pass
 // through flux_sum_kernel).  Of 63 tiles (133 x 101 M4 cells) 45 + 7.5 and 40 + 9.8 us, of 16 (50 x 50
 // M2) 22.3 + 5.3 and 12.6 + 6.6 us a stage, with six and by this rule.
-int flux_groups_of(const mnc_ctx *ctx) {
-    if (ctx->flux_groups > 0) return ctx->flux_groups;
+int auto_flux_groups(const mnc_ctx *ctx) {
     const int T = mnc::kSplitTile;
     const int tiles = std::max(1, ((ctx->grid.num_cells_x + T - 1) / T) * ((ctx->grid.num_cells_y + T - 1) / T));
     const int half = ctx->tab.Q / 2, orbits = half * half;
@@ -587,6 +586,7 @@ int flux_groups_of(const mnc_ctx *ctx) {
     const int per = (orbits + want - 1) / want;          // no group without orbits
     return std::max(1, (orbits + per - 1) / per);
 }
+int flux_groups_of(const mnc_ctx *ctx) { return ctx->flux_groups > 0 ? ctx->flux_groups : auto_flux_groups(ctx); }
 
 mnc::GridArgs grid_args(mnc_ctx *ctx) {
     mnc::GridArgs g{};
@@ -999,7 +999,7 @@ int mnc_grid_create(mnc_ctx *ctx, const mnc_grid_desc *grid, const double *momen
     if ((st = dalloc(ctx, &ctx->d_mom, n)) || (st = dalloc(ctx, &ctx->d_alpha, n)) ||
         (st = dalloc(ctx, &ctx->d_old, n)) || (st = dalloc(ctx, &ctx->d_flux, n)) ||
         (st = dalloc(ctx, &ctx->d_st, nc)) || (st = dalloc(ctx, &ctx->d_ss, nc)) ||
-        (st = dalloc(ctx, &ctx->d_fpart, size_t(std::max(mnc::kMaxFluxGroups, flux_groups_of(ctx))) * grid->num_cells_x *
+        (st = dalloc(ctx, &ctx->d_fpart, size_t(std::max(mnc::kMaxFluxGroups, auto_flux_groups(ctx))) * grid->num_cells_x *
                                              grid->num_cells_y * ctx->tab.nm)) ||
         (st = dalloc(ctx, &ctx->d_tflag, size_t((grid->num_cells_x + mnc::kSplitTile - 1) / mnc::kSplitTile) *
                                              ((grid->num_cells_y + mnc::kSplitTile - 1) / mnc::kSplitTile))))
@@ -1324,7 +1324,7 @@ int mnc_tune(mnc_ctx *ctx, const char *key, int value) {
         return MNC_OK;
     }
     if (std::strcmp(key, "rounds") == 0) {
-        if (value < 0 || value > 512) return ctx_fail(ctx, MNC_ERR_ARG, "rounds out of range");
+        if (value < -1 || value > 512) return ctx_fail(ctx, MNC_ERR_ARG, "rounds out of range");
         ctx->rounds = value;
         return MNC_OK;
     }
@@ -1364,7 +1364,7 @@ int mnc_tune(mnc_ctx *ctx, const char *key, int value) {
         return MNC_OK;
     }
     if (std::strcmp(key, "flux_groups") == 0) {
-        if (value < 1 || value > mnc::kMaxFluxGroups) return ctx_fail(ctx, MNC_ERR_ARG, "flux_groups must be 1 to 8");
+        if (value < 0 || value > mnc::kMaxFluxGroups) return ctx_fail(ctx, MNC_ERR_ARG, "flux_groups must be 0 to 8");
         ctx->flux_groups = value;
         return MNC_OK;
     }
@@ -1396,7 +1396,7 @@ int mnc_tune(mnc_ctx *ctx, const char *key, int value) {
 
 int mnc_get_tune(const mnc_ctx *ctx, const char *key, int *value) {
     if (!ctx || !key || !value) return MNC_ERR_ARG;
-    if (std::strcmp(key, "rounds") == 0) { *value = ctx->rounds >= 0 ? ctx->rounds : 6; return MNC_OK; }
+    if (std::strcmp(key, "rounds") == 0) { *value = ctx->rounds; return MNC_OK; }
     if (std::strcmp(key, "tail_mode") == 0) { *value = ctx->tail_mode; return MNC_OK; }
     if (std::strcmp(key, "mix_cond_log10") == 0) { *value = ctx->mix_cond_log10; return MNC_OK; }
     if (std::strcmp(key, "mix_defer") == 0) { *value = ctx->mix_defer; return MNC_OK; }
@@ -1408,7 +1408,7 @@ int mnc_get_tune(const mnc_ctx *ctx, const char *key, int *value) {
     if (std::strcmp(key, "has_mixed") == 0) { *value = ctx->has_mix ? 1 : 0; return MNC_OK; }
     if (std::strcmp(key, "graph") == 0) { *value = ctx->use_graph; return MNC_OK; }
     if (std::strcmp(key, "flux_tile") == 0) { *value = ctx->flux_tile; return MNC_OK; }
-    if (std::strcmp(key, "flux_groups") == 0) { *value = ctx->flux_groups > 0 || ctx->has_grid ? flux_groups_of(ctx) : 6; return MNC_OK; }
+    if (std::strcmp(key, "flux_groups") == 0) { *value = ctx->flux_groups; return MNC_OK; }
     if (std::strcmp(key, "learned_gate_log10") == 0) { *value = ctx->learned_gate_log10; return MNC_OK; }
     if (std::strcmp(key, "learned_fallback_iters") == 0) { *value = ctx->learned_fallback_iters; return MNC_OK; }
     if (std::strcmp(key, "learned_fused") == 0) { *value = ctx->learned_fused; return MNC_OK; }

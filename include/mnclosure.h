@@ -278,10 +278,10 @@ int mnc_reset_stats(mnc_ctx *ctx);
 
 /* Tuning knobs of the batched solve (set by the autotuner or by hand):
  *   "rounds"       lockstep sweep/logic rounds before the persistent tail (0-512);
- *                  until it is set: 6 in mixed precision or where the network
- *                  is consulted, 0 in FP64 (the tail's kernel takes every cell;
- *                  7 with the reference's line search below TOL 1e-6, whose
- *                  decisions depend on the order of the sums); reads 6 then
+ *                  -1 (default): by the solve: 6 in mixed precision or where the
+ *                  network is consulted, 0 in FP64 (the tail's kernel takes every
+ *                  cell; 7 with the reference's line search below TOL 1e-6, whose
+ *                  decisions depend on the order of the sums)
  *   "tail_blocks"  workgroups of the persistent tail kernel (1-65536)
  *   "tail_mode"    0: a 16-lane row per remaining cell, four cells per wave (one
  *                  wave per cell when there are few);
@@ -324,7 +324,8 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *                  as 1): 16x16 tiles with the directions split
  *                  into "flux_groups" groups summed in order and reciprocals
  *                  of dx, dy (rounding-level differences from 0-2)
- *   "flux_groups"  direction groups of flux_tile 3 (1-8; by default 6, more on small grids)
+ *   "flux_groups"  direction groups of flux_tile 3 (1-8); 0 (default): 6, more on
+ *                  small grids
  *   "flux_overlap" flux_tile 3 in mnc_update: 1 (default): after a stage's
  *                  lockstep rounds, the flux of the tiles whose stencil region
  *                  holds no cell left for the Newton tail runs on a second

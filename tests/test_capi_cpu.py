@@ -62,3 +62,23 @@ def test_driver_reports_missing_deck_key(tmp_path):
                        timeout=60)
     assert r.returncode != 0
     assert "main.cpp:input error at line 83" in r.stdout
+
+
+def test_tuning_knobs_read_back_and_restore():
+    """What mnc_get_tune reads is what mnc_tune takes back, also for a knob nobody has
+    set, and restores it."""
+    mnc = load_pkg("mnc")
+    ctx = mnc.Context(4, 16, device=-1)
+    for key, other in (("rounds", 3), ("flux_groups", 2), ("tail_mode", 2), ("tail_blocks", 7), ("mix_blocks", 9),
+                       ("mix_defer", 1), ("mix_split", 2), ("mix_cond_log10", 5), ("flux_tile", 1), ("flux_overlap", 0),
+                       ("graph", 1), ("learned_gate_log10", 2), ("learned_fallback_iters", 4), ("learned_fused", 0)):
+        was = ctx.get_tune(key)
+        ctx.tune(key, other)
+        assert ctx.get_tune(key) == other
+        ctx.tune(key, was)
+        assert ctx.get_tune(key) == was
+    assert ctx.get_tune("rounds") == -1 and ctx.get_tune("flux_groups") == 0      # by the solve, by the grid
+    for key, value in (("rounds", -2), ("rounds", 513), ("flux_groups", -1), ("flux_groups", 9)):
+        with pytest.raises(mnc.MncError):
+            ctx.tune(key, value)
+    ctx.close()

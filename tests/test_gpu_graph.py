@@ -146,3 +146,37 @@ def test_flux_overlap_equals_serial(precision):
         assert st_s.iter_sum == st_o.iter_sum and st_s.tail_cells == st_o.tail_cells
     print("tail cells over 8 steps: %d" % st_s.tail_cells)
     assert st_s.tail_cells > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(20, 18), (70, 50)])
+def test_restored_knobs_leave_the_route(nx, ny):
+    """Reading a knob, trying another value and writing the first back leaves a step as
+    it was, on grids whose direction groups the grid chooses (2 x 2 and 5 x 4 tiles)
+    and with the buffer of a grid created under fewer groups: the same bits."""
+    mnc, gi = load_pkg("mnc"), load_pkg("grid_init")
+    print("case restored knobs %dx%d" % (nx, ny), flush=True)
+    d = dict(num_cells_x=nx, num_cells_y=ny, a_x=-3.5, b_x=3.5, a_y=-3.5, b_y=3.5, gaussian_sigma=0.0,
+             floor_value=1e-6, sigma=1.0, init_cond=1, moment_order=4, quad_order=16, cfl_factor=0.9,
+             tol=1e-8, cond_h_max=1e10, max_iter=100, use_gaunt=0, theta=2.0, line_search=1)
+    opt = mn_options(mnc, d)
+    keys = ("rounds", "flux_groups", "tail_mode", "tail_blocks", "flux_overlap", "flux_tile", "graph")
+    res = []
+    for change in (False, True):
+        ctx, g = gpu_grid_from_deck(mnc, gi, d)
+        if change:
+            was = {k: ctx.get_tune(k) for k in keys}
+            for k, v in zip(keys, (2, 1, 2, 5, 0, 1, 1)):
+                ctx.tune(k, v)
+            ctx.update(g.max_dt, opt)
+            h = gi.initial_state(nx, ny, -3.5, 3.5, -3.5, 3.5, 1, 0.0, 1e-6, 1.0, 15, 0.9, 2.0)
+            ctx.grid_create(nx, ny, h.dx, h.dy, h.init_x, h.init_y, 1, 2.0, h.moments, h.alpha, h.sigma_t, h.sigma_s)
+            for k in keys:
+                ctx.tune(k, was[k])
+        ctx.reset_stats()
+        for _ in range(3):
+            ctx.update(g.max_dt, opt)
+        s = ctx.stats()
+        res.append(ctx.grid_get() + ((s.iter_sum, s.tail_cells),))
+        ctx.close()
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1]) and res[0][2] == res[1][2]
