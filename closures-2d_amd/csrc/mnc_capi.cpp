@@ -286,6 +286,25 @@ int mlp_check(mnc_ctx *ctx, bool need_ready) {
 // learned_gate_log10 at this value switches the network off
 constexpr int kGateOff = 5;
 
+// A solve whose path depends on the rounding of f: the reference's Armijo test below
+// TOL 1e-6 compares values of f that differ by that rounding.
+bool by_rounding(const mnc_options *o) { return o->line_search == MNC_LS_REFERENCE && o->tol_rel < 1e-6; }
+
+// Lockstep rounds of a solve for which none are set.  FP64 cells go straight to the
+// tail's kernel.  Not if the path depends on the rounding of f, and with it on the
+// order of the sums: the lockstep kernels sum in the reference's.  Seven rounds are
+// the fewest after which no more than one per cent of the cells that take the
+// reference's iterations end elsewhere than it does (3,000 M3 closures, Q = 30, four
+// draws: 1.27% without rounds, 1.05 after six, 0.84 after seven and after twelve; 0.88
+// with six and the former tail of a wave per cell).  Against that form (ms, M4, Q = 16,
+// means over draws): 2,049 closures from near starts 2.4 -> 1.6 (its best draws 1.5),
+// cold 3.4 -> 1.8, 200,003 cold 16.3 -> 9.7, 150,001 with beams 19.5 -> 9.3, a step of a
+// 133 x 101 lattice 7.9 -> 3.5; with twelve rounds 2.5, 2.8, 8.4, 9.6 and 5.4.
+int auto_rounds(const mnc_ctx *ctx, const mnc_options *o) {
+    const bool network = o->warm_start == MNC_WARM_LEARNED && ctx->learned_gate_log10 < kGateOff;
+    return o->precision == MNC_PREC_MIXED || network ? 6 : (by_rounding(o) ? 7 : 0);
+}
+
 // na: the no-allocation entry point's state regions (the library's fixed
 // scratch array) in place of the context's buffers; then nothing is allocated
 // and no timing events are recorded.
@@ -374,21 +393,8 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     a.gnt = ctx->g64.nt;
     mnc::LaunchPlan lp;
     lp.r0 = 0;
-    // FP64 cells go straight to the tail kernel unless rounds are asked for.
-    // Not with the reference's line search below TOL 1e-6: there its Armijo
-    // test compares values of f that differ by f's rounding, so a cell's last
-    // steps depend on the order of the sums, and the lockstep kernels sum in the
-    // reference's.  Seven rounds are the fewest after which no more than one per
-    // cent of the cells that take the reference's iterations end elsewhere than it
-    // does (3,000 M3 closures, Q = 30, four draws: 1.27% without rounds, 1.05 after
-    // six, 0.84 after seven, 0.84 after twelve; 0.88 with six and the former tail
-    // of a wave per cell).  Against that form (ms, M4, Q = 16, means over draws):
-    // 2,049 closures from near starts 2.4 -> 1.6 (its best draws 1.5), cold 3.4 ->
-    // 1.8, 200,003 cold 16.3 -> 9.7, 150,001 with beams 19.5 -> 9.3, a 133 x 101
-    // lattice's step 7.9 -> 3.5; with twelve rounds 2.5, 2.8, 8.4, 9.6 and 5.4.
-    const bool by_rounding = o->line_search == MNC_LS_REFERENCE && o->tol_rel < 1e-6;
     const bool network = learned && ctx->learned_gate_log10 < kGateOff;
-    const int rounds = ctx->rounds >= 0 ? ctx->rounds : (mixed || network ? 6 : (by_rounding ? 7 : 0));
+    const int rounds = ctx->rounds >= 0 ? ctx->rounds : auto_rounds(ctx, o);
     lp.r1 = rounds;
     lp.num_cu = ctx->num_cu;
     lp.fresh = rounds == 0 && !mixed && !network && (ctx->tail_mode == 0 || ctx->tail_mode == 3 || ctx->ppn);
@@ -1477,9 +1483,16 @@ int mnc_autotune(mnc_ctx *ctx, double dt, const mnc_options *opt, int steps, cha
     }
     knobs.push_back({"graph", {0, 1}, &ctx->use_graph});
     knobs.push_back({"flux_tile", {0, 1, 2, 3}, &ctx->flux_tile});
-    knobs.push_back({"flux_groups", {2, 3, 4, 6, 8}, &ctx->flux_groups});
+    knobs.push_back({"flux_groups", {0, 2, 3, 4, 6, 8}, &ctx->flux_groups});
     knobs.push_back({"flux_overlap", {0, 1}, &ctx->flux_overlap});
-    knobs.push_back({"rounds", {0, 2, 4, 6, 8, 12}, &ctx->rounds});
+    // -1 stands for each solve's own rule, which sends plain FP64 solves straight to the
+    // tail's kernel.  A path that depends on rounding gets no fewer than that rule
+    // gives; mixed and learned solves may also do without rounds (all FP64 then).
+    const bool floor = by_rounding(opt);
+    std::vector<int> rounds = floor && opt->precision != MNC_PREC_MIXED ? std::vector<int>{-1, 8, 12}
+                                                                        : std::vector<int>{-1, 2, 4, 6, 8, 12};
+    if (!floor && auto_rounds(ctx, opt) != 0) rounds.push_back(0);
+    knobs.push_back({"rounds", rounds, &ctx->rounds});
     knobs.push_back({"tail_mode", {0, 1, 2}, &ctx->tail_mode});
     knobs.push_back({"tail_blocks", {cu, 2 * cu, 4 * cu}, &ctx->tail_blocks});
     if (opt->precision == MNC_PREC_MIXED) knobs.push_back({"mix_blocks", {cu / 2, cu, 2 * cu}, &ctx->mix_blocks});

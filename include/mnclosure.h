@@ -281,7 +281,8 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *                  -1 (default): by the solve: 6 in mixed precision or where the
  *                  network is consulted, 0 in FP64 (the tail's kernel takes every
  *                  cell; 7 with the reference's line search below TOL 1e-6, whose
- *                  decisions depend on the order of the sums)
+ *                  decisions depend on the order of the sums).  A mixed-precision
+ *                  solve with 0 is the FP64 one
  *   "tail_blocks"  workgroups of the persistent tail kernel (1-65536)
  *   "tail_mode"    0: a 16-lane row per remaining cell, four cells per wave (one
  *                  wave per cell when there are few);
@@ -352,7 +353,11 @@ int mnc_get_tune(const mnc_ctx *ctx, const char *key, int *value);
  * precision) "mix_blocks", and keeps the fastest (a gate that consults the
  * network only when it beats the network off by more than 1%).  Every candidate converges
  * to the same tolerance; "mix_cond_log10" trades mixed-precision steps
- * against FP64 ones.  The grid state
+ * against FP64 ones, and "rounds" 0, if it is the fastest, takes them all in FP64.  With
+ * the reference's line search below TOL 1e-6 no fewer rounds are tried than that solve
+ * takes by itself.  The settings kept hold for every later solve of the context, whatever
+ * its options, until they are set again ("rounds" -1, "flux_groups" 0: by the solve, by
+ * the grid).  The grid state
  * and the statistics are restored after every trial, so the call leaves the
  * solution where it was.  report (may be NULL) receives one "key=value ms/step"
  * line per trial.  The tail kernels sum in different orders, so the choice can

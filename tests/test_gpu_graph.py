@@ -180,3 +180,26 @@ def test_restored_knobs_leave_the_route(nx, ny):
         res.append(ctx.grid_get() + ((s.iter_sum, s.tail_cells),))
         ctx.close()
     assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1]) and res[0][2] == res[1][2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ls,precision,least", [(0, "fp64", 7), (1, "fp64", 1), (1, "mixed", 0)])
+def test_autotune_keeps_to_the_round_rule(ls, precision, least):
+    """The autotuner tries no fewer lockstep rounds than a solve whose path depends on
+    rounding takes by itself, and none at all only where that is the solve's FP64
+    route; what it keeps can be undone."""
+    mnc, gi = load_pkg("mnc"), load_pkg("grid_init")
+    print("case autotune rounds ls=%d %s" % (ls, precision), flush=True)
+    d = dict(num_cells_x=24, num_cells_y=24, a_x=-3.5, b_x=3.5, a_y=-3.5, b_y=3.5, gaussian_sigma=0.0,
+             floor_value=1e-4, sigma=1.0, init_cond=1, moment_order=2, quad_order=12, cfl_factor=0.9,
+             tol=1e-8, cond_h_max=1e10, max_iter=100, use_gaunt=0, theta=2.0, line_search=ls)
+    opt = mn_options(mnc, d, precision=mnc.PREC_MIXED if precision == "mixed" else mnc.PREC_FP64)
+    ctx, g = gpu_grid_from_deck(mnc, gi, d)
+    report = ctx.autotune(g.max_dt, opt, steps=1)
+    tried = [int(l.split()[0].split("=")[1]) for l in report if l.startswith("rounds=")]
+    assert len(tried) >= 2 and all(r == -1 or r >= least for r in tried)
+    assert ctx.get_tune("rounds") in [-1] + tried
+    ctx.tune("rounds", -1)
+    ctx.tune("flux_groups", 0)
+    assert ctx.get_tune("rounds") == -1 and ctx.get_tune("flux_groups") == 0
+    ctx.close()
