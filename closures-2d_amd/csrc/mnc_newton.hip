@@ -1738,9 +1738,11 @@ __device__ __forceinline__ void chol_column(double (&a)[NM], double &rd, double 
 // cell.  Lane i holds row i of H in registers, lane n the gradient, and the factor
 // goes column by column: the pivot by a lane read, the column to LDS, and every
 // lane updates its row from LDS broadcasts, so that the gradient's lane ends with
-// L^-1 g.  Bound by the 45 dependent columns and 990 broadcast FMAs; with the
-// rows in LDS, H formed there term by term from the Gaunt map in HBM and
-// dot products in a chain this took 438 us at 10,000 cells, now 193.  The
+// L^-1 g.  Bound by the 45 dependent columns and 990 broadcast FMAs, at two waves
+// per SIMD (256 registers, 28 more spilled); with the rows in LDS, H formed there
+// term by term from the Gaunt map in HBM and dot products in a chain this took
+// 438 us a round (mean over the solves of 10,000 cells), now 165 (193 with nine
+// blocks launched per CU, whose last eighth started when the others ended).  The
 // steps are those of cell_logic (opt.cpp:209-318, linesearch.cpp:38-98);
 // cells needing another sweep go onto list lin^1.
 __global__ __launch_bounds__(64, 2) void logic_g64_kernel(NewtonArgs A, int lin) {
@@ -2097,8 +2099,8 @@ bool launch_newton_g64_init(const NewtonArgs &a, int nm, int np2, hipStream_t s)
 bool launch_newton_g64_rounds(const NewtonArgs &a, int nm, int np2, int &lin, int rounds, int num_cu, hipStream_t s) {
     if (!(nm == 45 && np2 == 45)) return false;
     // sixteen cells a sweep block, two blocks resident per CU; a cell a logic
-    // block, nine resident (LDS); cells beyond loop
-    const int sweep = std::min((a.ncells + 15) / 16, 2 * num_cu), logic = std::min(a.ncells, 9 * num_cu);
+    // block, eight resident (two waves per SIMD by its registers); cells beyond loop
+    const int sweep = std::min((a.ncells + 15) / 16, 2 * num_cu), logic = std::min(a.ncells, 8 * num_cu);
     for (int r = 0; r < rounds; ++r) {
         hipLaunchKernelGGL(sweep_g64_kernel, dim3(sweep), dim3(256), 0, s, a, lin);
         hipLaunchKernelGGL(logic_g64_kernel, dim3(logic), dim3(64), 0, s, a, lin);
