@@ -542,6 +542,35 @@ int cb_state_alloc(mnc_ctx *ctx, int nc) {
     return MNC_OK;
 }
 
+// The host-array change-of-basis entry's buffers.  The context keeps them from call to
+// call (126 MB of workspace at M4, Q = 16, whose allocation and release took longer than
+// the solve of 5,000 cells) up to a bound; beyond it (66,000 M4 cells) the solve outlasts
+// the allocation, and they are given back with the call.  No captured step holds
+// their addresses, so they do not end the captures.
+constexpr size_t kCbKeepBytes = size_t(256) << 20;
+
+void cb_batch_release(mnc_ctx *ctx) {
+    (void)hipFree(ctx->d_cb_batch);
+    (void)hipFree(ctx->d_cb_outs);
+    ctx->d_cb_batch = nullptr;
+    ctx->d_cb_outs = nullptr;
+    ctx->cb_batch_cap = ctx->cb_outs_cap = 0;
+}
+
+int cb_batch_buffers(mnc_ctx *ctx, size_t doubles, size_t cells) {
+    if (doubles <= ctx->cb_batch_cap && cells <= ctx->cb_outs_cap) return MNC_OK;
+    cb_batch_release(ctx);
+    if (hipMalloc((void **)&ctx->d_cb_batch, doubles * sizeof(double)) != hipSuccess ||
+        hipMalloc((void **)&ctx->d_cb_outs, cells * sizeof(mnc_outs)) != hipSuccess) {
+        (void)hipGetLastError();
+        cb_batch_release(ctx);
+        return ctx_fail(ctx, MNC_ERR_HIP, "hipMalloc failed");
+    }
+    ctx->cb_batch_cap = doubles;
+    ctx->cb_outs_cap = cells;
+    return MNC_OK;
+}
+
 int run_optcb_grid(mnc_ctx *ctx, int nc, const mnc_options *o, bool check) {
     const int nm = ctx->tab.nm, nq = ctx->tab.nq;
     int st;
@@ -881,19 +910,8 @@ int mnc_optcb_batch_host(mnc_ctx *ctx, int ncells, double *u, double *P2M, doubl
     const int nm = ctx->tab.nm, nq = ctx->tab.nq;
     const int blocks = std::min(ncells, 16 * ctx->num_cu);
     const size_t nv = size_t(ncells) * nm, nb = size_t(ncells) * nm * nm, nws = size_t(blocks) * nq * nm;
-    // the context keeps the largest batch's buffers: 126 MB of workspace at M4,
-    // whose allocation and release took longer than the solve of 5,000 cells
     const size_t nd = 3 * nv + nb + nws;
-    if (nd > ctx->cb_batch_cap) {
-        ctx->cb_batch_cap = 0;
-        if ((st = dalloc(ctx, &ctx->d_cb_batch, nd))) return st;
-        ctx->cb_batch_cap = nd;
-    }
-    if (size_t(ncells) > ctx->cb_outs_cap) {
-        ctx->cb_outs_cap = 0;
-        if ((st = dalloc(ctx, &ctx->d_cb_outs, size_t(ncells)))) return st;
-        ctx->cb_outs_cap = size_t(ncells);
-    }
+    if ((st = cb_batch_buffers(ctx, nd, size_t(ncells)))) return st;
     double *d = ctx->d_cb_batch;
     mnc_outs *d_outs = ctx->d_cb_outs;
     double *d_u = d, *d_aP = d + nv, *d_aM = d + 2 * nv, *d_B = d + 3 * nv, *d_ws = d_B + nb;
@@ -943,7 +961,9 @@ int mnc_optcb_batch_host(mnc_ctx *ctx, int ncells, double *u, double *P2M, doubl
         MNC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         return s2;
     };
-    return run();
+    st = run();
+    if (nd * sizeof(double) > kCbKeepBytes) cb_batch_release(ctx);
+    return st;
 }
 
 int mnc_batch_set(mnc_ctx *ctx, int ncells, const double *u, const double *alpha) {

@@ -313,3 +313,32 @@ def test_driver_change_of_basis_time_stepping(tmp_path):
     err = rel_l2(density(res[2]), density(res[0]))
     print("optbfgs vs Newton time stepping: density rel-L2 %.3e" % err)
     assert err < 1e-7
+
+
+def _free_bytes(mnc):
+    import ctypes
+    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert ctypes.CDLL(mnc.LIB_PATH).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.gpu
+def test_optcb_batch_gives_large_buffers_back():
+    """The context keeps a batch's buffers only up to a bound: after 80,000 M4 cells
+    (298 MB) the card's free memory is what it was, and batches before and after
+    give the same bits."""
+    mnc, o = load_pkg("mnc"), oracle()
+    print("case optcb buffers", flush=True)
+    tab = o.Tables(4, 16, False)
+    u, _, _ = config2_batch(tab.w, tab.p, tab.xi, tab.eta, tab.nm, 80000, np.random.default_rng(3), near_boundary_frac=0.0)
+    P2M, aP = _identity_start(o, tab.nm, len(u))
+    ctx = mnc.Context(4, 16, use_gaunt=False)
+    opt = mnc.options(tol=1e-8, line_search=mnc.LS_ROBUST)
+    first = ctx.optcb_batch_host(u[:64], P2M[:64], aP[:64], opt)
+    free = _free_bytes(mnc)
+    all_ = ctx.optcb_batch_host(u, P2M, aP, opt)
+    assert abs(_free_bytes(mnc) - free) <= 32 << 20
+    again = ctx.optcb_batch_host(u[:64], P2M[:64], aP[:64], opt)
+    ctx.close()
+    for a, b, c in zip(first[1:], all_[1:], again[1:]):
+        assert np.array_equal(a, np.asarray(b)[:64].reshape(a.shape)) and np.array_equal(a, c)
