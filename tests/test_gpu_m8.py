@@ -187,3 +187,52 @@ def test_m8_closures_over_tile_remainders(Q, n):
     un = np.linalg.norm(ug[rs] - uo[rs], axis=1) / np.linalg.norm(uo[rs], axis=1)
     print("max ||du||/||u|| %.3e, same iterations %.2f" % (un.max(), (itg == ito).mean()))
     assert un.max() <= 4e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Q", [14, 16])
+def test_m8_closures_on_rank_deficient_quadratures(Q):
+    """Fewer nodes than resolve all order-16 moments: the Gaunt fit's coefficients for
+    columns that vanish on the nodes are large and arbitrary, and the map keeps only
+    those of the product's own class.  The direct Hessian of the oracle at the same
+    tolerance, 4e-8 as above, and its iterations."""
+    mnc = load_pkg("mnc")
+    print("case m8 rank deficient Q=%d" % Q, flush=True)
+    tab = oracle().Tables(8, Q, False)
+    u, astar = _m8_inputs(tab, 100, 100 + Q)
+    a0 = np.zeros_like(u)
+    a0[:, 0] = 2.0 * math.sqrt(math.pi) * (math.log(0.5 / math.sqrt(math.pi)) + np.log(u[:, 0]))
+    ctx = mnc.Context(8, Q)
+    st, ug, ag, itg, rg, _ = ctx.opt_batch_host(u, a0, mnc.options(tol=1e-8, line_search=mnc.LS_ROBUST))
+    ctx.close()
+    sto, uo, ao, ito, ro, _ = tab.opt_batch(u, a0, max_iter=100, tol=1e-8, cond_h_max=1e10, line_search=1, nthreads=8)
+    assert st == 0 and sto == 0
+    rs = rg == ro
+    un = np.linalg.norm(ug[rs] - uo[rs], axis=1) / np.linalg.norm(uo[rs], axis=1)
+    print("same level %.3f, same iterations %.3f, max ||du||/||u|| %.3e" % (rs.mean(), (itg == ito).mean(), un.max()))
+    assert rs.mean() >= 0.97 and (rs & (itg == ito)).mean() >= 0.9
+    assert un.max() <= 4e-8
+
+
+@pytest.mark.gpu
+def test_orbit_flux_in_chunks_matches_fused():
+    """500 x 490 cells at order 5, Q = 66: the ansatz of 69 tiles of orbits exceeds 8 GiB
+    and goes in chunks of 35 and 34 tiles.  Against the fused kernel, 1e-12 of the
+    largest flux as above (17,000 roundings of either sign add up to some 130)."""
+    mnc = load_pkg("mnc")
+    print("case orbit flux chunks", flush=True)
+    nx, ny, order, Q, nm = 500, 490, 5, 66, 21
+    rng = np.random.default_rng(11)
+    shape = (nx + 4, ny + 4)
+    a = rng.normal(0.0, 0.3, shape + (nm,)) / (1.0 + np.arange(nm))
+    m = rng.random(shape + (nm,))
+    ctx = mnc.Context(order, Q)
+    ctx.grid_create(nx, ny, 2.0 / nx, 2.0 / ny, -1.0, -1.0, 2, 1.7, m, a, np.ones(shape), np.ones(shape))
+    res = {}
+    for tile in (1, 0):
+        ctx.tune("flux_tile", tile)
+        res[tile] = ctx.flux()
+    ctx.close()
+    err = np.abs(res[0] - res[1]).max() / np.abs(res[1]).max()
+    print("flux rel %.3e" % err)
+    assert err <= 1e-12

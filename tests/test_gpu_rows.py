@@ -130,3 +130,66 @@ def test_reference_line_search_takes_seven_rounds(order, Q, n, ppn):
     if not ppn:
         _, _, _, ito, ro, _ = tab.opt_batch(u, a0, tol=1e-8, nthreads=8)
         assert ((res[0][0][3] == ito) & (res[0][0][4] == ro)).mean() >= 0.95
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,Q,gaunt", [(1, 82, False), (4, 34, False), (4, 36, True)])
+@pytest.mark.parametrize("n", [3, 2053])
+def test_rows_with_the_table_in_l2(order, Q, gaunt, n):
+    """Quadratures whose orbit table does not fit in LDS beside the waves' words (the
+    smallest such at M1 and M4): the oracle's iterations and, with the bound of
+    test_rows_match_oracle, its answers."""
+    mnc, o = load_pkg("mnc"), oracle()
+    print("case rows L2 N=%d Q=%d gaunt=%d n=%d" % (order, Q, gaunt, n), flush=True)
+    tab, u, _ = _mn_batch(o, order, Q, gaunt, n, Q + n)
+    a0 = isotropic_start(u)
+    tol = 1e-6 if gaunt else 1e-8
+    ctx = mnc.Context(order, Q, use_gaunt=gaunt)
+    st, ug, ag, itg, rg, _ = ctx.opt_batch_host(u, a0, mnc.options(tol=tol, line_search=mnc.LS_ROBUST))
+    ctx.close()
+    m = min(n, 200)
+    sto, uo, ao, ito, _, _ = tab.opt_batch(u[-m:], a0[-m:], tol=tol, nthreads=8, line_search=1)
+    assert st == sto == 0 and np.all(rg == 0.0)
+    same = itg[-m:] == ito
+    assert same.mean() >= 0.99
+    assert np.abs(ug[-m:][same] - uo[same]).max() <= 1e-10 * np.abs(uo).max()
+    assert np.abs(ag[-m:][same] - ao[same]).max() <= 1e-10 * (1.0 + np.abs(ao).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,Q,gaunt,ppn", [(2, 12, False, False), (4, 16, False, False), (4, 16, True, False),
+                                               (3, 12, False, True)])
+@pytest.mark.parametrize("n", [5, 2100])
+def test_rows_supplementary_stop(order, Q, gaunt, ppn, n):
+    """tol_gamma holds cells back that pass the gradient test: the oracle's iterations
+    (Mn: more of them than without it) and its answers (a further quadratic step
+    leaves them at rounding, 1e-10 as above)."""
+    mnc, o = load_pkg("mnc"), oracle()
+    print("case rows tol_gamma N=%d gaunt=%d ppn=%d n=%d" % (order, gaunt, ppn, n), flush=True)
+    tab = o.Tables(order, Q, gaunt)
+    rng = np.random.default_rng(7 * order + n)
+    nm, delta = tab.nm, 1e-10 if ppn else 0.0
+    if ppn:
+        alpha = 0.3 * rng.normal(size=(n, nm)) / (1.0 + np.arange(nm))
+        alpha[:, 0] = rng.uniform(4.0, 8.0, n)
+        z = alpha @ tab.p[:, :nm].T
+        u = (0.5 * z + np.sqrt(0.25 * z * z + delta)) @ (tab.w[:, None] * tab.p[:, :nm])
+        a0 = np.zeros_like(u)
+        a0[:, 0] = u[:, 0] - 4.0 * np.pi * delta / u[:, 0]
+    else:
+        tab, u, _ = _mn_batch(o, order, Q, gaunt, n, 7 * order + n)
+        a0 = isotropic_start(u)
+    ctx = mnc.Context(order, Q, use_gaunt=gaunt, moment_type=mnc.MOMENT_PPN if ppn else mnc.MOMENT_MN)
+    kw = dict(tol=1e-2, line_search=mnc.LS_ROBUST, delta_ppn=delta)
+    it0 = ctx.opt_batch_host(u, a0, mnc.options(**kw))[3]
+    st, ug, ag, itg, rg, _ = ctx.opt_batch_host(u, a0, mnc.options(tol_gamma=1.1, **kw))
+    ctx.close()
+    m = min(n, 600)
+    sto, uo, ao, ito, _, _ = tab.opt_batch(u[-m:], a0[-m:], tol=1e-2, nthreads=8, line_search=1, delta_ppn=delta,
+                                           moment_type=o.MOMENT_PPN if ppn else o.MOMENT_MN, tol_gamma=1.1)
+    assert st == sto == 0 and np.all(rg == 0.0)
+    same = itg[-m:] == ito
+    assert same.mean() >= 0.99
+    assert np.all(itg >= it0) and (ppn or itg.sum() > it0.sum())   # PPn's quadratic steps need none
+    assert np.abs(ug[-m:][same] - uo[same]).max() <= 1e-10 * np.abs(uo).max()
+    assert np.abs(ag[-m:][same] - ao[same]).max() <= 1e-10 * (1.0 + np.abs(ao).max())
