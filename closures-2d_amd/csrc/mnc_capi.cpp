@@ -19,7 +19,7 @@ struct mnc_ctx {
     mnc::Tables tab;
     int num_cu = 256;
     // tables on device
-    double *d_w = nullptr, *d_p = nullptr, *d_pT = nullptr, *d_xi = nullptr, *d_eta = nullptr, *d_gv = nullptr;
+    double *d_w = nullptr, *d_p = nullptr, *d_xi = nullptr, *d_eta = nullptr, *d_gv = nullptr;
     int *d_gptr = nullptr, *d_gk = nullptr;
     // solver state / stats
     int *d_ctl = nullptr;            // [0],[1] list counts, [2] tail queue, [3] error bits, [4] deferred
@@ -103,7 +103,7 @@ struct mnc_ctx {
     size_t cb_batch_cap = 0, cb_outs_cap = 0;
     double *d_mlp_io = nullptr;      // host-call staging (inputs, targets/outputs)
     size_t mlp_io_cap = 0;
-    double *d_us = nullptr, *d_guess = nullptr;   // Newton prologue: u/u0 and the MLP guesses
+    double *d_guess = nullptr;       // the unfused learned start's guesses
     size_t guess_cap = 0;
     // timing
     bool timing = false;
@@ -345,7 +345,6 @@ int run_newton(mnc_ctx *ctx, int ncells, double *u, double *alpha, const mnc_opt
     a.outs = outs;
     a.w = ctx->d_w;
     a.p = ctx->d_p;
-    a.pT = ctx->d_pT;
     a.nq = t.nq;
     a.gptr = ctx->d_gptr;
     a.gk = ctx->d_gk;
@@ -617,7 +616,7 @@ int auto_flux_groups(const mnc_ctx *ctx) {
     const int T = mnc::kSplitTile;
     const int tiles = std::max(1, ((ctx->grid.num_cells_x + T - 1) / T) * ((ctx->grid.num_cells_y + T - 1) / T));
     const int half = ctx->tab.Q / 2, orbits = half * half;
-    const int want = std::max(6, std::min(mnc::kMostFluxGroups, 3 * ctx->num_cu / tiles));
+    const int want = std::max(6, std::min(mnc::kMaxFluxGroups, 3 * ctx->num_cu / tiles));
     const int per = (orbits + want - 1) / want;          // no group without orbits
     return std::max(1, (orbits + per - 1) / per);
 }
@@ -661,7 +660,6 @@ mnc::GridArgs grid_args(mnc_ctx *ctx) {
     g.op = ctx->d_fop;
     g.odir = ctx->d_fodir;
     g.oidx = ctx->d_foidx;
-    g.ont = ctx->ftab.nt;
     return g;
 }
 
@@ -739,10 +737,7 @@ int mnc_create(const mnc_setup *setup, mnc_ctx **out) {
             return MNC_ERR_HIP;
         return MNC_OK;
     };
-    std::vector<double> pT(t.p.size());
-    for (int q = 0; q < t.nq; ++q)
-        for (int k = 0; k < t.np2; ++k) pT[size_t(k) * t.nq + q] = t.p[size_t(q) * t.np2 + k];
-    if (up(&ctx->d_w, t.w) || up(&ctx->d_p, t.p) || up(&ctx->d_pT, pT) || up(&ctx->d_xi, t.xi) || up(&ctx->d_eta, t.eta) ||
+    if (up(&ctx->d_w, t.w) || up(&ctx->d_p, t.p) || up(&ctx->d_xi, t.xi) || up(&ctx->d_eta, t.eta) ||
         up(&ctx->d_gptr, t.gptr) || up(&ctx->d_gk, t.gk) || up(&ctx->d_gv, t.gv) ||
         hipMalloc((void **)&ctx->d_ctl, mnc::kCtlWords * sizeof(int)) != hipSuccess ||
         hipMemset(ctx->d_ctl, 0, mnc::kCtlWords * sizeof(int)) != hipSuccess ||
@@ -798,10 +793,10 @@ void mnc_destroy(mnc_ctx *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (auto &g : ctx->graphs) drop_graph(g);
     for (auto &ev : ctx->events) { (void)hipEventDestroy(ev.a); (void)hipEventDestroy(ev.b); }
-    void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_pT, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
+    void *ptrs[] = {ctx->d_w, ctx->d_p, ctx->d_xi, ctx->d_eta, ctx->d_gv, ctx->d_gptr, ctx->d_gk,
                     ctx->d_mz, ctx->d_mg, ctx->d_mh, ctx->d_mgptr, ctx->d_mgk, ctx->d_mgv, ctx->d_mpv, ctx->d_gz, ctx->d_gh, ctx->d_gmap, ctx->d_gidx, ctx->d_gpos,
                     ctx->d_ot, ctx->d_opos, ctx->d_ogoff, ctx->d_ogk, ctx->d_ogv,
-                    ctx->d_foz, ctx->d_fop, ctx->d_fodir, ctx->d_foidx, ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_us, ctx->d_guess,
+                    ctx->d_foz, ctx->d_fop, ctx->d_fodir, ctx->d_foidx, ctx->d_cb_batch, ctx->d_cb_outs, ctx->d_mlp, ctx->d_mlp_scratch, ctx->d_mlp_loss, ctx->d_mlp_io, ctx->d_guess,
                     ctx->d_ctl, ctx->d_stats, ctx->d_std, ctx->d_sti, ctx->d_lists, ctx->d_mom, ctx->d_alpha, ctx->d_old,
                     ctx->d_st, ctx->d_ss, ctx->d_flux, ctx->d_ansatz, ctx->d_fpart, ctx->d_bu, ctx->d_ba, ctx->d_bo,
                     ctx->d_cbB, ctx->d_cbaP, ctx->d_cbws, ctx->d_tflag};
@@ -1025,7 +1020,7 @@ int mnc_grid_create(mnc_ctx *ctx, const mnc_grid_desc *grid, const double *momen
     if ((st = dalloc(ctx, &ctx->d_mom, n)) || (st = dalloc(ctx, &ctx->d_alpha, n)) ||
         (st = dalloc(ctx, &ctx->d_old, n)) || (st = dalloc(ctx, &ctx->d_flux, n)) ||
         (st = dalloc(ctx, &ctx->d_st, nc)) || (st = dalloc(ctx, &ctx->d_ss, nc)) ||
-        (st = dalloc(ctx, &ctx->d_fpart, size_t(std::max(mnc::kMaxFluxGroups, auto_flux_groups(ctx))) * grid->num_cells_x *
+        (st = dalloc(ctx, &ctx->d_fpart, size_t(std::max(mnc::kTuneFluxGroups, auto_flux_groups(ctx))) * grid->num_cells_x *
                                              grid->num_cells_y * ctx->tab.nm)) ||
         (st = dalloc(ctx, &ctx->d_tflag, size_t((grid->num_cells_x + mnc::kSplitTile - 1) / mnc::kSplitTile) *
                                              ((grid->num_cells_y + mnc::kSplitTile - 1) / mnc::kSplitTile))))
@@ -1390,7 +1385,7 @@ int mnc_tune(mnc_ctx *ctx, const char *key, int value) {
         return MNC_OK;
     }
     if (std::strcmp(key, "flux_groups") == 0) {
-        if (value < 0 || value > mnc::kMaxFluxGroups) return ctx_fail(ctx, MNC_ERR_ARG, "flux_groups must be 0 to 8");
+        if (value < 0 || value > mnc::kTuneFluxGroups) return ctx_fail(ctx, MNC_ERR_ARG, "flux_groups must be 0 to 8");
         ctx->flux_groups = value;
         return MNC_OK;
     }

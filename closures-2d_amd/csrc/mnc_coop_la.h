@@ -186,8 +186,8 @@ __device__ __forceinline__ bool reg_cholesky(double (&row)[NM], int lane) {
 }
 
 // x <- (L L^T)^{-1} x, x_i on lane i, with the reciprocals of the diagonal
-// (wave-uniform rd[j]) in place of divisions: the tail's Newton direction and
-// the condition estimate's repeated solves.
+// (wave-uniform rd[j]) in place of divisions, for the condition estimate's
+// repeated solves.
 template <int NM>
 __device__ __forceinline__ void reg_apply_inv_rcp(const double (&row)[NM], const double (&col)[NM],
                                                   const double (&rd)[NM], double &x, int lane) {
@@ -287,56 +287,6 @@ __device__ __forceinline__ double reg_inv_norm1(const double (&row)[NM], const d
 #pragma unroll
         for (int i = k + 1; i < NM; ++i) z[i] = fma(-readlane_d(row[k], i), z[k], z[i]);
     }
-    double c = 0.0;
-#pragma unroll
-    for (int i = 0; i < NM; ++i) {
-        double d = 0.0;
-#pragma unroll
-        for (int k = i; k < NM; ++k) d = fma(readlane_d(z[k], i), z[k], d);
-        c += fabs(d);
-    }
-    if constexpr (NM <= 16) return row16_max(lane < NM ? c : 0.0);
-    else return wave_max(lane < NM ? c : 0.0);
-}
-
-// reg_inv_norm1 that also solves x <- (L L^T)^{-1} x (x_i on lane i) for the
-// cost of one more lane: lane NM carries x through the forward substitution
-// that forms Z, and the back substitution then runs beside the Z^T Z
-// products.  Lane NM's updates fma(-L[i][k], z_k, z_i) are
-// reg_apply_inv_rcp's fma(-x_k, L[i][k], x_i) (the same exact product), in
-// the same order, and the back substitution is its second loop, so x comes
-// out bit for bit as reg_apply_inv_rcp leaves it.
-template <int NM>
-__device__ __forceinline__ double reg_inv_norm1_solve(const double (&row)[NM], const double (&col)[NM],
-                                                      const double (&rd)[NM], double &x, int lane) {
-    static_assert(NM < 64, "lane NM carries the right-hand side");
-    double z[NM];
-#pragma unroll
-    for (int i = 0; i < NM; ++i) {
-        const double xi = readlane_d(x, i);
-        z[i] = lane == NM ? xi : ((i == lane) ? 1.0 : 0.0);
-    }
-#pragma unroll
-    for (int k = 0; k < NM; ++k) {
-        z[k] = z[k] * rd[k];
-#pragma unroll
-        for (int i = k + 1; i < NM; ++i) z[i] = fma(-readlane_d(row[k], i), z[k], z[i]);
-    }
-    // y = L^{-1} x from lane NM, y_j on lane j (where reg_apply_inv_rcp's
-    // forward loop leaves it), then its back substitution
-    double y = 0.0;
-#pragma unroll
-    for (int j = 0; j < NM; ++j) {
-        const double v = readlane_d(z[j], NM);
-        y = lane == j ? v : y;
-    }
-#pragma unroll
-    for (int j = NM - 1; j >= 0; --j) {
-        const double xj = readlane_d(y, j) * rd[j];
-        if (lane == j) y = xj;
-        else if (lane < j) y = fma(-col[j], xj, y);
-    }
-    x = lane < NM ? y : x;
     double c = 0.0;
 #pragma unroll
     for (int i = 0; i < NM; ++i) {

@@ -34,7 +34,6 @@ struct NewtonArgs {
     mnc_outs *outs;       // [ncells] or nullptr
     const double *w;      // [nq]
     const double *p;      // [nq][np2]
-    const double *pT;     // [np2][nq], the same table transposed
     int nq;
     const int *gptr;      // Gaunt CSR (nm*nm+1)
     const int *gk;
@@ -129,7 +128,7 @@ int build_mix_tables(int moment_order, int quad_order, MixTables &m);
 // not fit a lane), by quadrature orbits and moment classes (mnc_orbit.h).
 struct G64Tables {
     int nt = 0;                    // tiles of 16 orbits, padded with zero weight
-    std::vector<double> z;         // [nt][kG64Z][64]: moments of 16 orbits, four of a class at a time
+    std::vector<double> z;         // [nt][sum of ceil(n_c / 4)][64]: moments of 16 orbits, four of a class at a time
     std::vector<double> h;         // [nt][4][12][64]: w m of four orbits, the order-2N moments of a class in
                                    // three columns of 16 (after class 0's, w itself)
     std::vector<double> map;       // class by class [column of 16 Hessian entries][four moments][64]: the Gaunt map
@@ -213,7 +212,6 @@ struct NoAllocState {
     int *st_i = nullptr, *lists = nullptr, *ctl = nullptr;
     size_t cap = 0;
 };
-size_t noalloc_scratch_bytes();
 // The array's address on `device`, which must be current: resolved with
 // hipGetSymbolAddress on the first call for that device and kept per device
 // (each GPU holds its own copy of the array at its own address).
@@ -224,7 +222,6 @@ bool noalloc_layout(int nm, int np2, void *base, NoAllocState &out);
 constexpr int kMixMaxTiles = 16;   // quadrature tiles of 16 points held in LDS (nq <= 256)
 constexpr int kMixParts = 3;       // bf16 parts per table value in the mixed sweep's Hessian table
 int mix_tiles(int nm);             // 16-column tiles of the order-2N moments the mixed kernel expects
-int newton_block();
 // Zeroes the solve-control words (a kernel, so the step can be captured).
 void launch_ctl_reset(int *ctl, hipStream_t s);
 void newton_store_fields(int nm, int np2, int *dfields, int *ifields);
@@ -270,16 +267,15 @@ struct GridArgs {
     int groups;           // direction groups of flux_tile 3
     int ppn;              // the PPn ansatz (computeAnsatz, momopt_update.cpp:54-57)
     double delta;         // its delta
-    // flux_tile 3 on part of the grid: 0 every tile; 1 the tiles whose flag is
-    // 0 (no unfinished closure in their stencil region); 2 the flagged ones
     const double *oz, *op, *odir;   // FluxTables (orders 5 to 8)
     const int *oidx;
-    int ont;
+    // flux_tile 3 on part of the grid: 0 every tile; 1 the tiles whose flag is
+    // 0 (no unfinished closure in their stencil region); 2 the flagged ones
     const int *tile_flag; // [tiles_x][tiles_y] of kSplitTile x kSplitTile cells
     int tile_mode;
 };
-constexpr int kMaxFluxGroups = 8;      // what a caller may set
-constexpr int kMostFluxGroups = 16;    // what a small grid takes by itself
+constexpr int kTuneFluxGroups = 8;     // the most a caller may set
+constexpr int kMaxFluxGroups = 16;     // the most a small grid takes by itself
 constexpr int kSplitTile = 16;   // flux_tile 3's cells per tile side
 // flags[tx][ty] = 1 for the flux_tile 3 tiles whose stencil region (the tile
 // and two cells around it) holds a cell on list0 (count *cnt0) or list1 (*cnt1);
@@ -309,7 +305,7 @@ struct CbArgs {
 int launch_optcb(const CbArgs &a, int max_blocks, int num_cu, hipStream_t s);
 
 void launch_ghost_fill(const GridArgs &g, hipStream_t s);
-// Orders 5 to 8 count nodes in whole tiles of 16 orbits (64 of the ont tiles' 64 ont nodes).
+// Orders 5 to 8 count nodes in whole tiles of 16 orbits, 64 a tile.
 void launch_ansatz(const GridArgs &g, int q0, int nqc, hipStream_t s);
 // stage: 0 = flux only (writes g.flux), 1 = Euler stage, 2 = Euler + Heun average
 bool launch_flux_euler(const GridArgs &g, int q0, int nqc, int stage, double dt, bool first_chunk,

@@ -211,14 +211,6 @@ __device__ __forceinline__ double rcond(const T (&l)[Tri<N>::size], double anorm
     return (1.0 / double(est)) / anorm;
 }
 
-template <int N>
-__device__ __forceinline__ double nrm2(const double (&x)[N]) {
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) s = fma(x[i], x[i], s);
-    return sqrt(s);
-}
-
 __device__ __forceinline__ unsigned long long lane_mask_lt() {
     const int lane = threadIdx.x & 63;
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -2028,7 +2020,6 @@ void launch_mixed_all(const NewtonArgs &a, const LaunchPlan &lp, hipStream_t s) 
 
 }  // namespace
 
-int newton_block() { return kBlock; }
 int newton_list_word(int l) { return l < 2 ? l : l + 2; }   // cw() on the host
 
 __global__ void ctl_reset_kernel(int *ctl) {
@@ -2131,7 +2122,6 @@ constexpr size_t kNoAllocBytes = noalloc_bytes(Store<15, 45>::dfields, Store<15,
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
-size_t noalloc_scratch_bytes() { return kNoAllocBytes; }
 
 bool noalloc_layout(int nm, int np2, void *base, NoAllocState &out) {
     int df = 0, ifl = 0;

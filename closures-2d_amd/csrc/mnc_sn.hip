@@ -44,32 +44,21 @@ __device__ __forceinline__ double sn_slope(double l, double c, double r) {
     return (__double2hiint(d1) ^ __double2hiint(d2)) < 0 ? 0.0 : copysign(v, d1);
 }
 
-// ghosts of f (and of f2 when not null) <- the opposite interior layers of f
-// (x: interior rows; y: interior columns)
-__global__ void sn_ghost_kernel(double *f, double *f2, int nx, int ny, int nq) {
+// ghosts of f <- the opposite interior layers of from (x: interior rows; y: interior columns)
+__global__ void sn_ghost_kernel(const double *from, double *f, int nx, int ny, int nq) {
     const int NY = ny + 4;
     const long long nxw = 2LL * ny * nq, nyw = 2LL * nx * nq;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < nxw + nyw;
          t += (long long)gridDim.x * blockDim.x) {
         if (t < nxw) {
             const int q = int(t % nq), j = 2 + int((t / nq) % ny), g = int(t / (nq * (long long)ny));
-            const double lo = f[(size_t(nx + g) * NY + j) * nq + q], hi = f[(size_t(2 + g) * NY + j) * nq + q];
-            f[(size_t(g) * NY + j) * nq + q] = lo;
-            f[(size_t(nx + 2 + g) * NY + j) * nq + q] = hi;
-            if (f2) {
-                f2[(size_t(g) * NY + j) * nq + q] = lo;
-                f2[(size_t(nx + 2 + g) * NY + j) * nq + q] = hi;
-            }
+            f[(size_t(g) * NY + j) * nq + q] = from[(size_t(nx + g) * NY + j) * nq + q];
+            f[(size_t(nx + 2 + g) * NY + j) * nq + q] = from[(size_t(2 + g) * NY + j) * nq + q];
         } else {
             const long long u = t - nxw;
             const int q = int(u % nq), i = 2 + int((u / nq) % nx), g = int(u / (nq * (long long)nx));
-            const double lo = f[(size_t(i) * NY + ny + g) * nq + q], hi = f[(size_t(i) * NY + 2 + g) * nq + q];
-            f[(size_t(i) * NY + g) * nq + q] = lo;
-            f[(size_t(i) * NY + ny + 2 + g) * nq + q] = hi;
-            if (f2) {
-                f2[(size_t(i) * NY + g) * nq + q] = lo;
-                f2[(size_t(i) * NY + ny + 2 + g) * nq + q] = hi;
-            }
+            f[(size_t(i) * NY + g) * nq + q] = from[(size_t(i) * NY + ny + g) * nq + q];
+            f[(size_t(i) * NY + ny + 2 + g) * nq + q] = from[(size_t(i) * NY + 2 + g) * nq + q];
         }
     }
 }

@@ -289,13 +289,14 @@ bool gaunt_pattern_values(int n, const std::vector<int> &gptr, const std::vector
     return true;
 }
 
-// Operand tables of the FP64 matrix-core sweep (v_mfma_f64_16x16x4f64 layouts
-// as for the mixed sweep; the exponent of point 16T + R(r, l/16) sits in
-// element r of lane l after the first product):
-//   z[T][kk][l]     = p[16T + l%16][4kk + l/16]                         (A operand)
-//   g[T][r][nt][l]  = w_q p[q][16nt + l%16], column 16 ngt - 1 = w_q      (B operand)
-//   h[T][r][nt][l]  = w_q p2N[q][16nt + l%16]                            (B operand)
-// with q = 16T + R(r, l/16).
+// Operand tables of the FP64 matrix-core sweep (v_mfma_f64_16x16x4f64: lane l gives
+// row or column l % 16, term l / 16 of four; element r of lane l receives row
+// mfma_f64_row(r, l / 16), column l % 16), by orbits and classes (mnc_orbit.h).
+// P(o, k) is moment k at orbit o's node with xi, eta > 0, m_c(e) the e-th of class c:
+//   z    exponents: P(16 T + l % 16, m_c(4 kk + l / 16)), the classes one after the other
+//   h    sums over four orbits o = 16 T + mfma_f64_row(r, l / 16): w P(o, m_c(16 m + l % 16))
+//        in column m = 0, 1, 2 of class c; after class 0's moments w itself
+//   map  the Hessian entry 16 col + l % 16 of class c from its moment 4 kk + l / 16
 int build_g64_tables(int moment_order, int quad_order, G64Tables &m) {
     constexpr int N = 8, n = orbit_nm(N), n2 = orbit_nm(2 * N);
     Tables t;
