@@ -79,6 +79,23 @@ def flops_per_iter(n, nq):
     return f_iter, f_trial
 
 
+def flops_done_rows(n, nq):
+    """FP64 flops that the row kernel does for one Newton iteration and one Armijo trial,
+    by the quadrature's nq / 4 orbits: per orbit the class sums of alpha.m (2n), the
+    exponents and class sums of four nodes (about 24), the Hessian sums (n(n+1)); the
+    factor, its inverse (n^3/3 each) and the direction (4n^2)."""
+    no = nq / 4.0
+    return no * (2 * n + 24 + n * (n + 1)) + 2 * n ** 3 / 3.0 + 4 * n * n, no * (2 * n + 24)
+
+
+def flops_done_m8(solves, iters, trials):
+    """FP64 flops of the M8 kernels (n = 45, Q = 32): a sweep for each solve's start and
+    each trial, of 16 cells 1,624 matrix products of 2,048 flops (16 orbit tiles of 13
+    for the exponents and 48 for the order-16 moments, 648 for the Gaunt map); the
+    factor and its two solves for each iteration."""
+    return (solves + trials) * 1624 * 2048 / 16.0 + iters * (45 ** 3 / 3.0 + 2 * 45 * 45)
+
+
 def make_grid(mnc, gi, d):
     mt = d.get("moment_type", 0)
     ctx = mnc.Context(d["moment_order"], d["quad_order"], use_gaunt=d["use_gaunt"], moment_type=mt)
@@ -165,7 +182,8 @@ T0 = time.perf_counter()
 
 
 FORCE_TUNE = {}
-ISOLATED_ROUNDS = (6, 12, 48, 96, 192)   # lockstep rounds tried on the isolated batch
+# lockstep rounds tried on the isolated batch: each solve's own rule, none, and from 6 up
+ISOLATED_ROUNDS = (-1, 0, 6, 12, 48, 96)
 TUNE_STEPS = 10           # steps per autotuning trial
 
 
@@ -318,12 +336,10 @@ def bench_isolated(mnc, n, seed, oracle_sample, train_steps):
                 ctx.batch_solve(opt)
                 return time.perf_counter() - t1
 
-            # the lockstep rounds before the persistent tail: a cold-started batch
-            # needs ~20 sweeps per cell, so more rounds move work from the tail
-            # (one wave per cell) to the lane-parallel rounds; keep the fastest
-            # (and, mixed precision, whether steps redone in FP64 wait for the
-            # tail or join FP64 lockstep rounds)
-            ctx.tune("tail_mode", 0)                  # the context is shared by the forms
+            # the lockstep rounds before the tail's kernel (a row of lanes per cell),
+            # which takes every cell if there are none; keep the fastest (and, mixed
+            # precision, whether steps redone in FP64 wait for the tail or join FP64
+            # lockstep rounds)
             timed_solve()                              # first run allocates
             tries = {}
             for defer in ((0, 1) if "precision" in kw else (0,)):
@@ -336,20 +352,12 @@ def bench_isolated(mnc, n, seed, oracle_sample, train_steps):
             ctx.tune("rounds", best_rounds)
             if "precision" in kw:
                 ctx.tune("mix_defer", best_defer)
-            # the tail at one or at two waves per SIMD (latency against cells in flight)
-            tail_tries = {0: tries[(best_rounds, best_defer)]}
-            ctx.tune("tail_mode", 3)
-            tail_tries[3] = min(timed_solve(), timed_solve())
-            best_tail = min(tail_tries, key=tail_tries.get)
-            ctx.tune("tail_mode", best_tail)
             best = min(timed_solve() for _ in range(3))
             st = ctx.stats()
             ug, _, itg, rg = ctx.batch_get()
             progress("isolated %s (line search %d): %.3f s" % (name, ls, best))
             res[name] = {"closures_per_s": n / best, "s": best, "rounds": best_rounds, "mix_defer": best_defer,
-                         "tail_mode": best_tail,
-                         "tried_s": dict({"rounds=%d defer=%d" % k: v for k, v in tries.items()},
-                                         **{"tail_mode=%d" % k: v for k, v in tail_tries.items()}),
+                         "tried_s": {"rounds=%d defer=%d" % k: v for k, v in tries.items()},
                          "newton_iters_per_closure": st.iter_sum / st.num_dual_solves,
                          "trials_per_closure": st.trial_sum / st.num_dual_solves,
                          "reg_hist": list(st.hist_reg), "warm_pick_mlp_iso_prev": list(st.warm_pick),
@@ -534,8 +542,7 @@ def bench_m8(mnc, gi, steps, n=512, sample=1000):
     kst = ctx.stats()
     kn, kms = ctx.timing_get(mnc.KCLASS_NEWTON)
     ctx.timing_enable(False)
-    f_iter, f_trial = flops_per_iter(45, 32 * 32)
-    m8_flops = kst.iter_sum * f_iter + kst.trial_sum * f_trial
+    m8_flops = flops_done_m8(kst.num_dual_solves, kst.iter_sum, kst.trial_sum)
     m8_achieved = m8_flops / (kms * 1e-3) / 1e12 if kms > 0 else 0.0
     # closures of `sample` cells of the final state, GPU vs oracle, from the stored alpha
     rng = np.random.default_rng(5)
@@ -560,16 +567,15 @@ def bench_m8(mnc, gi, steps, n=512, sample=1000):
             "roofline": {"bound": "mfma", "achieved": m8_achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": m8_achieved / FP64_PEAK_TFLOPS, "traffic": None,
                          "kernel": "Newton solve per stage (sweep_g64_kernel + logic_g64_kernel rounds), HIP events "
-                                   "over the %d steps run again; flops: iterations x %.3f Mflop + trials x %.1f kflop "
-                                   "(the reference's direct-Hessian FP64 count at n = 45, nq = 1024)"
-                                   % (steps, f_iter / 1e6, f_trial / 1e3),
+                                   "over the %d steps run again; flops: the matrix products of the sweeps, by "
+                                   "quadrature orbits, and the factorisations that the kernels do" % steps,
                          "algorithmic_flops_per_launch": m8_flops / max(2 * steps, 1),
                          "avg_launch_ms": kms / max(2 * steps, 1)}}
 
 
 def bench_ppn(mnc, gi, d, steps, warmup, cpu_seconds):
     """The PPn form of the same lattice workload (MOMOPT_MOMENT_TYPE 1,
-    MOMOPT_DELTA_PPN 1e-10; FP64 lane kernels and cooperative tail, robust line
+    MOMOPT_DELTA_PPN 1e-10; FP64, a row of lanes per cell, robust line
     search): converged closures/s and s/step over K steps from t = 0, the
     Newton roofline as for the Mn forms, and the CPU oracle on the first steps
     of the same run (cpu_seconds of wall clock, 0 skips it)."""
@@ -772,10 +778,11 @@ def main():
     value = best["closures"] / best["wall"]
     kst = best["kstats"]
     stages = 2 * best["kernel_steps"]                 # two closure solves per Heun step
-    # the dominant kernel: the persistent tail (FP64, one wave per cell), its
-    # Newton iterations and Armijo trials counted on the device
+    # the tail's kernel (FP64, a row of lanes per cell; every cell of a solve without
+    # lockstep rounds), its Newton iterations and Armijo trials counted on the device
     tn, tms = best["tail"]
-    tail_flops = kst.tail_iter_sum * f_iter + kst.tail_trial_sum * f_trial
+    r_iter, r_trial = flops_done_rows(n, nq)
+    tail_flops = kst.tail_iter_sum * r_iter + kst.tail_trial_sum * r_trial
     tail_achieved = tail_flops / (tms * 1e-3) / 1e12 if tms > 0 else 0.0
     # the whole Newton stage (prologue, lockstep rounds and tail)
     sms = best["newton"][1] + tms
@@ -795,6 +802,10 @@ def main():
         else:
             net = " (network gate 10^%d: %.2f%% of the closures start from its guess)" % (
                 gate, 100.0 * picks[0] / max(sum(picks), 1))
+    all_fp64 = form == "plain-fp64" or (best["tuned"]["rounds"] == 0 and
+                                        not (form == "learned+mixed" and best["tuned"]["learned_gate_log10"] < 5))
+    if all_fp64 and form != "plain-fp64":
+        net += " (no mixed rounds: the autotuner's choice, every solve in FP64)"
     out = {
         "metric": "converged Mn closures/s, M4 lattice 280^2, steps 1-%d of 569 (t = 0 to %.4f), TOL 1e-8, "
                   "%s%s vs plain FP64" % (args.steps, t_end, form, net),
@@ -807,7 +818,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f64" if form == "plain-fp64" else "f64+bf16",
+        "dtype": "f64" if all_fp64 else "f64+bf16",
         "data": "synthetic (the reference's lattice initial condition, generated in-process)",
         "config": {"workload": "M4 lattice 280x280, Q=16 (nq=256), 7x7 checkerboard on [-3.5,3.5]^2, "
                                "floor 1e-10, TOL 1e-8, direct Hessian, robust line search, Heun dt=%.6g; timed "
@@ -827,19 +838,20 @@ def main():
                        "bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                        "frac": achieved / FP64_PEAK_TFLOPS, "traffic": stage_traffic(form),
                        "kernel": "Newton solve per stage (init + lockstep rounds + tail), %s form; flops are the "
-                                 "reference algorithm's FP64 count (iterations x %.1f kflop + trials x %.1f kflop); "
+                                 "reference algorithm's FP64 count (iterations x %.1f kflop + trials x %.1f kflop), "
+                                 "of which the row kernel does about a quarter; "
                                  "traffic: HBM bytes per stage from calibrated FETCH_SIZE + WRITE_SIZE "
                                  "(profiles/newton_stage_traffic.md)" % (form, f_iter / 1e3, f_trial / 1e3),
                        "algorithmic_flops_per_launch": alg_flops / max(stages, 1),
                        "avg_launch_ms": sms / max(stages, 1)}},
         "roofline": {"bound": "mfma", "achieved": tail_achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": tail_achieved / FP64_PEAK_TFLOPS, "traffic": stage_traffic("tail-" + form),
-                     "kernel": "tail_coop_kernel (the persistent FP64 tail, one wave per cell still iterating "
-                               "after the lockstep rounds), %s form, HIP events on the context's stream over the %d "
+                     "kernel": "rows_kernel (FP64, a row of lanes per cell: the cells left by the lockstep rounds, "
+                               "or all without them), %s form, HIP events on the context's stream over the %d "
                                "timed steps run again eagerly; flops: the Newton iterations (x %.1f kflop) and "
-                               "Armijo trials (x %.1f kflop) done in the tail, counted on the device: %.1f cells, "
-                               "%.0f iterations and %.0f trials per launch"
-                               % (form, best["kernel_steps"], f_iter / 1e3, f_trial / 1e3,
+                               "Armijo trials (x %.1f kflop) done in it, by quadrature orbits, counted on the "
+                               "device: %.1f cells, %.0f iterations and %.0f trials per launch"
+                               % (form, best["kernel_steps"], r_iter / 1e3, r_trial / 1e3,
                                   kst.tail_cells / max(stages, 1), kst.tail_iter_sum / max(stages, 1),
                                   kst.tail_trial_sum / max(stages, 1)),
                      "algorithmic_flops_per_launch": tail_flops / max(tn, 1),
