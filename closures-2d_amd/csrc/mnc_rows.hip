@@ -20,12 +20,13 @@
 //   direction L^-T (L^-1 g) and the condition bounds broadcast one lane's
 //   value to its row (DPP row_newbcast), so the four cells' dependent steps
 //   run side by side and nothing goes through LDS.
-// What bounds it: FP64 issue and the dependent steps of the algebra.  At 256
-// registers and two waves per SIMD the M4 forms must not spill: with the cell's
-// state in registers, the factor's 105 broadcasts kept for the inverse and a branch
-// around each load of H, scratch traffic was three quarters of the time (150,001
-// closures 7.2 ms, now 3.1).  The measured times stand at the launch rule
-// (launch_rows).
+// What bounds it: FP64 issue and the dependent steps of the algebra.  Two waves per
+// SIMD leave 256 registers, which the M4 forms of Mn exceed by 20 (four cells per
+// wave) and 16; PPn and the lower orders fit.  With the cell's state in registers,
+// the factor's 105 broadcasts kept for the inverse and a branch around each load of H
+// they exceeded them by 316, and scratch traffic was three quarters of the time
+// (150,001 closures 7.0 ms a call, now 2.85).  Further times stand at the launch rule
+// (launch_rows_n).
 #include <cfloat>
 
 #include "mnc_newton_state.h"
@@ -774,15 +775,22 @@ void launch_rows_w(const NewtonArgs &a, int blocks, int lin, int lin2, bool fres
 
 template <int N, bool GAUNT, bool PPN>
 void launch_rows_n(const NewtonArgs &a, int lin, int lin2, bool fresh, int num_cu, int tail_blocks, hipStream_t s) {
-    // A cell per wave shortens one evaluation (one orbit per lane at Q = 16,
-    // not four); four cells per wave share the algebra's issue slots.  Up to
-    // two waves per SIMD the first wins, above it the chip is full either way.
-    // Against the lockstep kernels and a tail of one wave per cell (M4, Q = 16):
-    // 2,049 closures from near starts 1.01 -> 0.09 ms, 150,001 cold ones with
-    // a fifth near the realizability boundary 12.3 -> 3.1 ms; 60 of M2 320 -> 71 us.
+    // A cell per wave shortens one evaluation (one orbit per lane at Q = 16, not
+    // four); four cells per wave share the algebra's issue slots and take a quarter
+    // of the waves.  The first wins while every cell has a SIMD to itself.  Kernel us,
+    // one cell per wave and four, Q = 16 (M2: 12):
+    //   closures          256      1,024     2,048     4,096     8,192
+    //   M4 cold          70  91    86 100   119 103   192 116   305 163
+    //   M4 near starts   40  47    52  51    76  55   112  66   177  94
+    //   M2 near starts   23  28    36  29    59  34    83  44   130  69
+    // The four-cell form fills the chip, at two waves per SIMD, from 8,192 cells on; below,
+    // some of it idles, and the time is the evaluations' latency.
+    // Against the lockstep kernels and a tail of one wave per cell (the whole call,
+    // M4, Q = 16): 2,049 closures from near starts 1.01 -> 0.09 ms, 150,001 cold ones
+    // with a fifth near the realizability boundary 12.3 -> 2.85; 60 of M2 320 -> 71 us.
     if (fresh) {
         const int waves = 4 * num_cu;                         // one per SIMD
-        if (a.ncells <= 2 * waves) {
+        if (a.ncells <= waves) {
             launch_rows_w<N, GAUNT, PPN, true>(a, (a.ncells + kRowWaves - 1) / kRowWaves, lin, lin2, true, false, s);
         } else {
             const int want = (a.ncells + 4 * kRowWaves - 1) / (4 * kRowWaves);
