@@ -65,7 +65,7 @@ struct mnc_ctx {
                                      // 3: fused, 16x16, directions split into flux_groups
     int flux_groups = 0;             // direction groups of flux_tile 3; 0: by the grid (auto_flux_groups)
     int flux_overlap = 1;            // flux_tile 3: the flux of tiles clear of the Newton tail runs beside it
-    int learned_fused = 1;           // 1: network and judge in one kernel; 0: the GEMM kernels, then the judge
+    int learned_fused = 1;           // 1: network and judge in one kernel; 0: the network's kernel, then the FP64 judge
     int learned_fallback_iters = 10;   // a network-started cell failing at level 0 within this many
                                      // iterations restarts from isotropicAlpha at level 0
     int learned_gate_log10 = -2;     // the network is consulted when ||g(best start)|| > 10^this ||u||;

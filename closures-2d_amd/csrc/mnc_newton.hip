@@ -980,7 +980,7 @@ __global__ __launch_bounds__(kBlock) void judge_kernel(NewtonArgs A) {
 // For the cells the first round parked on list kMlpList: the MLP
 // 15 -> 128 -> 128 -> 128 -> 15 (GELU) on the matrix cores, sixteen cells per
 // wave (v_mfma_f32_16x16x32_bf16: bf16 operands, FP32 sums, bias and GELU in
-// FP32, the arithmetic of the unfused GEMM kernels in mnc_mlp.hip, so the
+// FP32, the arithmetic of net_kernel in mnc_mlp.hip, so the
 // guesses are the same), then the judge: the gradient norm of the scaled
 // problem at the guess, also on the matrix cores (v_mfma_f32_16x16x4_f32), which
 // replaces the parked start when it is smaller; the cells join list 1.

@@ -146,8 +146,8 @@ typedef struct {
     long long warm_pick[3];      /* MNC_WARM_LEARNED starts taken from: [0] the
                                     MLP, [1] isotropicAlpha, [2] the alpha passed in */
     long long mixed_deferred;    /* MNC_PREC_MIXED Newton steps redone in FP64       */
-    long long tail_cells;        /* cells the persistent tail took (those still
-                                    iterating after the lockstep rounds)            */
+    long long tail_cells;        /* cells the tail's kernel took: those still iterating
+                                    after the lockstep rounds, or all without them  */
     long long tail_iter_sum;     /* Newton iterations done in the tail              */
     long long tail_trial_sum;    /* Armijo trials done in the tail                  */
     long long warm_fallback;     /* MNC_WARM_LEARNED cells started from the MLP's
@@ -176,7 +176,8 @@ int mnc_get_gaunt(const mnc_ctx *ctx, int *ptr, int *k, double *v);
 
 /* Batched closure on DEVICE arrays u[ncells][n], alpha[ncells][n] (in/out,
  * exactly opt()'s in/out meaning: u becomes the reconstructed ansatz moments,
- * alpha the multipliers); outs is a device array of ncells or NULL.
+ * alpha the multipliers); outs is a device array of ncells or NULL.  The order of
+ * the sums depends on ncells: a batch solved in parts agrees to rounding.
  * Replaces the per-cell opt() loop of solveOptimization
  * (momopt_update.cpp:214-238 -> opt.cpp:82-148). */
 int mnc_opt_batch(mnc_ctx *ctx, int ncells, double *u, double *alpha,
@@ -283,7 +284,8 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *                  cell; 7 with the reference's line search below TOL 1e-6, whose
  *                  decisions depend on the order of the sums).  A mixed-precision
  *                  solve with 0 is the FP64 one
- *   "tail_blocks"  workgroups of the persistent tail kernel (1-65536)
+ *   "tail_blocks"  workgroups of the tail's kernel (1-65536) for the cells that
+ *                  lockstep rounds leave; without rounds it goes by the cells
  *   "tail_mode"    0: a 16-lane row per remaining cell, four cells per wave (one
  *                  wave per cell when there are few);
  *                  1: one lane per cell; 2: one wave per cell, algebra per lane;
@@ -311,8 +313,8 @@ int mnc_reset_stats(mnc_ctx *ctx);
  *                  kernel (weights and quadrature in LDS, activations never
  *                  leave the chip, the guess's gradient norm from FP32
  *                  matrix-core sums; quadratures up to 512 points, larger ones
- *                  take the 0 path); 0: the separate GEMM kernels of
- *                  mnc_mlp_predict, then the FP64 comparison kernel
+ *                  take the 0 path); 0: the network's own kernel, as
+ *                  in mnc_mlp_predict, then the FP64 comparison kernel
  *   "learned_fallback_iters"  MNC_WARM_LEARNED: a cell started from the
  *                  network's guess that meets a regularization criterion at
  *                  level 0 within this many Newton iterations restarts once
