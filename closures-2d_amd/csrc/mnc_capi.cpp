@@ -549,8 +549,8 @@ int cb_state_alloc(mnc_ctx *ctx, int nc) {
 constexpr size_t kCbKeepBytes = size_t(256) << 20;
 
 void cb_batch_release(mnc_ctx *ctx) {
-    (void)hipFree(ctx->d_cb_batch);
-    (void)hipFree(ctx->d_cb_outs);
+    if (ctx->d_cb_batch) (void)hipFree(ctx->d_cb_batch);
+    if (ctx->d_cb_outs) (void)hipFree(ctx->d_cb_outs);
     ctx->d_cb_batch = nullptr;
     ctx->d_cb_outs = nullptr;
     ctx->cb_batch_cap = ctx->cb_outs_cap = 0;

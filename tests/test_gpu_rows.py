@@ -193,3 +193,27 @@ def test_rows_supplementary_stop(order, Q, gaunt, ppn, n):
     assert np.all(itg >= it0) and (ppn or itg.sum() > it0.sum())   # PPn's quadratic steps need none
     assert np.abs(ug[-m:][same] - uo[same]).max() <= 1e-10 * np.abs(uo).max()
     assert np.abs(ag[-m:][same] - ao[same]).max() <= 1e-10 * (1.0 + np.abs(ao).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,Q,gaunt", [(2, 12, False), (4, 16, False), (4, 16, True)])
+def test_rows_agree_across_the_launch_rule(order, Q, gaunt):
+    """One cell per wave up to four per CU, four cells per wave above: on both sides of
+    the line (on a card of 256 CUs) the same cells take the same iterations and end
+    at the same answers to rounding (1e-10 as above), and a repeated call at the
+    same bits."""
+    mnc, o = load_pkg("mnc"), oracle()
+    print("case rows launch rule N=%d gaunt=%d" % (order, gaunt), flush=True)
+    tab, u, _ = _mn_batch(o, order, Q, gaunt, 1025, 300 + order)
+    a0 = isotropic_start(u)
+    opt = mnc.options(tol=1e-6 if gaunt else 1e-8, line_search=mnc.LS_ROBUST)
+    ctx = mnc.Context(order, Q, use_gaunt=gaunt)
+    wide, four = ctx.opt_batch_host(u[:1024], a0[:1024], opt), ctx.opt_batch_host(u, a0, opt)
+    again = ctx.opt_batch_host(u, a0, opt)
+    ctx.close()
+    assert wide[0] == four[0] == 0
+    same = wide[3] == four[3][:1024]
+    assert same.mean() >= 0.99
+    for k in (1, 2):
+        assert np.abs(wide[k][same] - four[k][:1024][same]).max() <= 1e-10 * (1.0 + np.abs(four[k]).max())
+        assert np.array_equal(four[k], again[k])
